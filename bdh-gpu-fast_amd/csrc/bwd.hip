@@ -5,7 +5,8 @@
 //   distinct Q, K:   dQ = lower(G) K,  dK = upper(G) Q
 //   dV = sum_h M_h^T dO_h,  M = tril(Q K^T, -1)  (heads summed when V broadcasts)
 //
-// Kernels:
+// fp32 operands run on f32.hip; bf16 ones on syrk.hip where its constraints
+// hold and on these kernels otherwise:
 //  1. k_scores (TRANS) recomputes M as split-K partial tiles stored transposed,
 //     so rows of M^T are contiguous for the dV product.
 //  2. k_bwd_g forms G tile by tile: below the diagonal dO_i V_j^T, above it
@@ -22,11 +23,10 @@ struct GArgs {
   View dO, v;
   int64_t H, Hv, T, Dv;
   bool vec_do, vec_v;
-  void* g;       // [slab][tpad][tpad] in the compute dtype
+  void* g;       // [slab][tpad][tpad] bf16
   int64_t tpad;
 };
 
-template <bool BF>
 __device__ __forceinline__ void zero_acc(f32x16 (&acc)[2][2]) {
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -36,32 +36,32 @@ __device__ __forceinline__ void zero_acc(f32x16 (&acc)[2][2]) {
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 }
 
-template <bool BF, typename TA, typename TB>
-__device__ __forceinline__ void g_product(Smem<BF>& sm, const TA* a, int64_t ars, bool avec, int ar0,
+template <typename TA, typename TB>
+__device__ __forceinline__ void g_product(Smem& sm, const TA* a, int64_t ars, bool avec, int ar0,
                                           const TB* b, int64_t brs, bool bvec, int br0, int T, int Dv,
                                           f32x16 (&acc)[2][2]) {
-  KRows<TA, BF, false, 0> la;
+  KRows<TA, false, 0> la;
   la.base = a;
   la.rs = ars;
   la.r0 = ar0;
   la.nrows = T;
   la.K = Dv;
   la.vec = avec;
-  KRows<TB, BF, false, 0> lb;
+  KRows<TB, false, 0> lb;
   lb.base = b;
   lb.rs = brs;
   lb.r0 = br0;
   lb.nrows = T;
   lb.K = Dv;
   lb.vec = bvec;
-  zero_acc<BF>(acc);
-  mainloop<BF, false>(sm, la, lb, false, 0, Dv, acc, true);
+  zero_acc(acc);
+  mainloop<false>(sm, la, lb, false, 0, Dv, acc, true);
 }
 
-template <bool BF, typename TDO, typename TV>
+template <typename TDO, typename TV>
 __global__ __launch_bounds__(kNT) void k_bwd_g(GArgs a) {
-  typedef typename Mode<BF>::lds_t TG;
-  __shared__ Smem<BF> sm;
+  typedef bf16_t TG;
+  __shared__ Smem sm;
   const int ti = blockIdx.x, tj = blockIdx.y, slab = blockIdx.z;
   const int b = slab / a.H, h = slab % a.H;
   const int hv = a.Hv == 1 ? 0 : h;
@@ -77,10 +77,10 @@ __global__ __launch_bounds__(kNT) void k_bwd_g(GArgs a) {
     if (pass == 0 && ti < tj) continue;
     if (pass == 1 && ti > tj) continue;
     if (pass == 0)
-      g_product<BF, TDO, TV>(sm, dO, a.dO.s2, a.vec_do, ti * kTile, v, a.v.s2, a.vec_v, tj * kTile, T, Dv,
+      g_product<TDO, TV>(sm, dO, a.dO.s2, a.vec_do, ti * kTile, v, a.v.s2, a.vec_v, tj * kTile, T, Dv,
                              acc);
     else
-      g_product<BF, TV, TDO>(sm, v, a.v.s2, a.vec_v, ti * kTile, dO, a.dO.s2, a.vec_do, tj * kTile, T, Dv,
+      g_product<TV, TDO>(sm, v, a.v.s2, a.vec_v, ti * kTile, dO, a.dO.s2, a.vec_do, tj * kTile, T, Dv,
                              acc);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -112,22 +112,23 @@ struct DqArgs {
 };
 
 // MASK: 0 full G (self attention), 1 keep j < i (dQ = dS K), 2 keep j > i (dK = dS^T Q).
-template <bool BF, typename TX, typename TO, int MASK, bool ROPE>
+template <typename TO, int MASK, bool ROPE>
 __global__ __launch_bounds__(kNT) void k_bwd_dq(DqArgs a) {
-  typedef typename Mode<BF>::lds_t TG;
-  __shared__ Smem<BF> sm;
+  typedef bf16_t TG;
+  typedef bf16_t TX;
+  __shared__ Smem sm;
   const int ti = blockIdx.x, tn = blockIdx.y, slab = blockIdx.z;
   const int b = slab / a.H, h = slab % a.H;
   const int T = int(a.T), N = int(a.N);
 
-  KRows<TG, BF, false, MASK> la;
+  KRows<TG, false, MASK> la;
   la.base = static_cast<const TG*>(a.g) + int64_t(slab) * a.tpad * a.tpad;
   la.rs = a.tpad;
   la.r0 = ti * kTile;
   la.nrows = T;
   la.K = T;
   la.vec = true;
-  NRows<TX, BF, ROPE> lb;
+  NRows<TX, ROPE> lb;
   lb.base = static_cast<const TX*>(a.x.p) + b * a.x.s0 + h * a.x.s1;
   lb.rs = a.x.s2;
   lb.n0 = tn * kTile;
@@ -141,8 +142,8 @@ __global__ __launch_bounds__(kNT) void k_bwd_dq(DqArgs a) {
   if (MASK == 1) ke = min(T, (ti + 1) * kTile);
   if (MASK == 2) kb = ti * kTile;
   f32x16 acc[2][2];
-  zero_acc<BF>(acc);
-  mainloop<BF, false>(sm, la, lb, false, kb, ke, acc, true);
+  zero_acc(acc);
+  mainloop<false>(sm, la, lb, false, kb, ke, acc, true);
 
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = wave >> 1, wn = wave & 1;
@@ -182,31 +183,31 @@ struct DvArgs {
   View o;
 };
 
-template <bool BF, typename TDO, typename TO>
+template <typename TDO, typename TO>
 __global__ __launch_bounds__(kNT) void k_bwd_dv(DvArgs a) {
-  __shared__ Smem<BF> sm;
+  __shared__ Smem sm;
   const int R = blockIdx.x, Dt = blockIdx.y, bv = blockIdx.z;
   const int b = bv / int(a.Hv), hv = bv % int(a.Hv);
   const int h_lo = a.Hv == 1 ? 0 : hv;
   const int h_hi = a.Hv == 1 ? int(a.H) : hv + 1;
   const int T = int(a.T);
   f32x16 acc[2][2];
-  zero_acc<BF>(acc);
+  zero_acc(acc);
   for (int h = h_lo; h < h_hi; ++h) {
     const int slab = b * int(a.H) + h;
-    SplitRows<BF, true> la;
+    SplitRows<true> la;
     la.slab = a.spT + int64_t(slab) * a.ntl * kTileElems;
     la.split_stride = a.split_stride;
     la.nsplit = a.nsplit;
     la.R = R;
-    NRows<TDO, BF, false> lb;
+    NRows<TDO, false> lb;
     lb.base = static_cast<const TDO*>(a.dO.p) + b * a.dO.s0 + h * a.dO.s1;
     lb.rs = a.dO.s2;
     lb.n0 = Dt * kTile;
     lb.ncols = int(a.Dv);
     lb.krows = T;
     lb.vec4 = a.vec4_do;
-    mainloop<BF, false>(sm, la, lb, false, R * kTile, T, acc, true);
+    mainloop<false>(sm, la, lb, false, R * kTile, T, acc, true);
   }
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = wave >> 1, wn = wave & 1;
@@ -236,16 +237,16 @@ struct BwdPlan {
 };
 
 // saved: the score tiles come from the forward's workspace, so the first
-// region is not needed.  rope (bf16): room for the MFMA route as well.
-BwdPlan plan_bwd(int64_t B, int64_t H, int64_t T, int64_t K, bool bf, bool saved = false, bool rope = false) {
+// region is not needed.  rope: room for the MFMA route as well.
+BwdPlan plan_bwd(int64_t B, int64_t H, int64_t T, int64_t K, bool saved = false, bool rope = false) {
   BwdPlan p;
-  p.f = plan_fwd(B, H, T, K, bf);
+  p.f = plan_fwd(B, H, T, K);
   p.tpad = p.f.nt * kTile;
   // the first region holds the generic M^T partials or the bf16 score tiles
   // of the MFMA path, whichever is larger
-  p.g_off = saved ? 0 : align_up(std::max(p.f.ws_bytes, bf ? sy_bwd_workspace(B, H, T, K) : size_t(0)), 256);
-  p.ws_bytes = p.g_off + size_t(B * H) * size_t(p.tpad) * size_t(p.tpad) * (bf ? 2 : 4);
-  if (rope && bf) {
+  p.g_off = saved ? 0 : align_up(std::max(p.f.ws_bytes, sy_bwd_workspace(B, H, T, K)), 256);
+  p.ws_bytes = p.g_off + size_t(B * H) * size_t(p.tpad) * size_t(p.tpad) * 2;
+  if (rope) {
     p.r_sy = sy_rope_scores_workspace(B, H, T, K);
     if (p.r_sy > 0) {
       const size_t x_elems = size_t(B * H) * size_t(T) * size_t(K);
@@ -256,6 +257,25 @@ BwdPlan plan_bwd(int64_t B, int64_t H, int64_t T, int64_t K, bool bf, bool saved
     }
   }
   return p;
+}
+
+// fp32: [score tiles | dV pieces | G].
+struct F32BwdPlan {
+  F32Plan f;
+  int64_t tpad;
+  size_t dv_off, g_off, ws_bytes;
+};
+F32BwdPlan plan_f32_bwd(int64_t B, int64_t H, int64_t Hv, int64_t T, int64_t K, int64_t Dv, bool self) {
+  F32BwdPlan p;
+  p.f = plan_f32(B, H, T, K, self);
+  p.tpad = (T + kTile - 1) / kTile * kTile;
+  p.dv_off = align_up(p.f.m_bytes, 256);
+  p.g_off = align_up(p.dv_off + f32_dv_bytes(B, H, Hv, T, Dv), 256);
+  p.ws_bytes = p.g_off + size_t(B * H) * size_t(p.tpad) * size_t(p.tpad) * 4;
+  return p;
+}
+size_t f32_bwd_bytes(int64_t B, int64_t H, int64_t Hv, int64_t T, int64_t K, int64_t Dv) {
+  return std::max(plan_f32_bwd(B, H, Hv, T, K, Dv, true).ws_bytes, plan_f32_bwd(B, H, Hv, T, K, Dv, false).ws_bytes);
 }
 
 bool rows16b(const bdh_tensor4* t) {
@@ -312,7 +332,7 @@ int rope_fast_bwd(const bdh_tensor4* x, const bdh_tensor4* v, const bdh_tensor4*
 // rotating x at absolute positions as it stages it, so R(x) is never
 // written.  Workspace: G bf16.
 size_t rope_saved_bwd_bytes(int64_t B, int64_t H, int64_t T, int64_t N, size_t* g_off, int64_t* tpad) {
-  const BwdPlan p = plan_bwd(B, H, T, N, true, true, false);
+  const BwdPlan p = plan_bwd(B, H, T, N, true, false);
   if (g_off) *g_off = 0;
   if (tpad) *tpad = p.tpad;
   return size_t(B * H) * size_t(p.tpad) * size_t(p.tpad) * 2;
@@ -356,47 +376,43 @@ bool vec4_rows(const bdh_tensor4* t) {
   return t->size[3] % 4 == 0;
 }
 
-template <bool BF, typename TDO, typename TV>
+template <typename TDO, typename TV>
 int launch_g(const GArgs& a, int64_t nt, int64_t BH, hipStream_t s) {
   dim3 grid((unsigned)(nt), unsigned(nt), unsigned(BH));
-  BDH_LAUNCH("k_bwd_g", (k_bwd_g<BF, TDO, TV>), grid, dim3(kNT), 0, s, a);
+  BDH_LAUNCH("k_bwd_g", (k_bwd_g<TDO, TV>), grid, dim3(kNT), 0, s, a);
   return BDH_OK;
 }
 
-template <bool BF>
 int run_g(const GArgs& a, int64_t nt, int64_t BH, int32_t do_dt, int32_t v_dt, hipStream_t s) {
   const bool db = do_dt == BDH_BF16, vb = v_dt == BDH_BF16;
-  if (db) return vb ? launch_g<BF, bf16_t, bf16_t>(a, nt, BH, s) : launch_g<BF, bf16_t, float>(a, nt, BH, s);
-  return vb ? launch_g<BF, float, bf16_t>(a, nt, BH, s) : launch_g<BF, float, float>(a, nt, BH, s);
+  if (db) return vb ? launch_g<bf16_t, bf16_t>(a, nt, BH, s) : launch_g<bf16_t, float>(a, nt, BH, s);
+  return vb ? launch_g<float, bf16_t>(a, nt, BH, s) : launch_g<float, float>(a, nt, BH, s);
 }
 
-template <bool BF, typename TX, typename TO, int MASK, bool ROPE>
+template <typename TO, int MASK, bool ROPE>
 int launch_dq(const DqArgs& a, int64_t nt, int64_t BH, hipStream_t s) {
   dim3 grid((unsigned)(nt), unsigned((a.N + kTile - 1) / kTile), unsigned(BH));
-  BDH_LAUNCH("k_bwd_dq", (k_bwd_dq<BF, TX, TO, MASK, ROPE>), grid, dim3(kNT), 0, s, a);
+  BDH_LAUNCH("k_bwd_dq", (k_bwd_dq<TO, MASK, ROPE>), grid, dim3(kNT), 0, s, a);
   return BDH_OK;
 }
 
-// X has the compute dtype (it is q or k); only the output dtype varies.
-template <bool BF, int MASK, bool ROPE>
+// X (q or k) is bf16; only the output dtype varies.
+template <int MASK, bool ROPE>
 int run_dq(const DqArgs& a, int64_t nt, int64_t BH, int32_t o_dt, hipStream_t s) {
-  typedef typename std::conditional<BF, bf16_t, float>::type TX;
-  return o_dt == BDH_BF16 ? launch_dq<BF, TX, bf16_t, MASK, ROPE>(a, nt, BH, s)
-                          : launch_dq<BF, TX, float, MASK, ROPE>(a, nt, BH, s);
+  return o_dt == BDH_BF16 ? launch_dq<bf16_t, MASK, ROPE>(a, nt, BH, s) : launch_dq<float, MASK, ROPE>(a, nt, BH, s);
 }
 
-template <bool BF, typename TDO, typename TO>
+template <typename TDO, typename TO>
 int launch_dv(const DvArgs& a, int64_t nt, int64_t BHv, hipStream_t s) {
   dim3 grid((unsigned)(nt), unsigned((a.Dv + kTile - 1) / kTile), unsigned(BHv));
-  BDH_LAUNCH("k_bwd_dv", (k_bwd_dv<BF, TDO, TO>), grid, dim3(kNT), 0, s, a);
+  BDH_LAUNCH("k_bwd_dv", (k_bwd_dv<TDO, TO>), grid, dim3(kNT), 0, s, a);
   return BDH_OK;
 }
 
-template <bool BF>
 int run_dv(const DvArgs& a, int64_t nt, int64_t BHv, int32_t do_dt, int32_t o_dt, hipStream_t s) {
   const bool db = do_dt == BDH_BF16, ob = o_dt == BDH_BF16;
-  if (db) return ob ? launch_dv<BF, bf16_t, bf16_t>(a, nt, BHv, s) : launch_dv<BF, bf16_t, float>(a, nt, BHv, s);
-  return ob ? launch_dv<BF, float, bf16_t>(a, nt, BHv, s) : launch_dv<BF, float, float>(a, nt, BHv, s);
+  if (db) return ob ? launch_dv<bf16_t, bf16_t>(a, nt, BHv, s) : launch_dv<bf16_t, float>(a, nt, BHv, s);
+  return ob ? launch_dv<float, bf16_t>(a, nt, BHv, s) : launch_dv<float, float>(a, nt, BHv, s);
 }
 
 bool same4(const bdh_tensor4* a, const bdh_tensor4* b) {
@@ -436,6 +452,43 @@ int check_bwd(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v, 
   return BDH_OK;
 }
 
+// fp32 operands (f32.hip).
+int run_f32_bwd(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v, const bdh_tensor4* dout,
+                const bdh_tensor4* dq, const bdh_tensor4* dk, const bdh_tensor4* dv, const float* freqs,
+                int64_t rope_start, void* ws, size_t ws_bytes, hipStream_t s) {
+  const int64_t B = q->size[0], H = q->size[1], T = q->size[2], N = q->size[3];
+  const bool self = k == nullptr;
+  const F32BwdPlan p = plan_f32_bwd(B, H, v->size[1], T, N, v->size[3], self);
+  if (ws == nullptr || ws_bytes < p.ws_bytes) return BDH_ERR_WORKSPACE;
+  char* w = static_cast<char*>(ws);
+  float* g = reinterpret_cast<float*>(w + p.g_off);
+  if (numel4(dv) > 0) {
+    ScoresArgs sa;
+    sa.q = view_of(q);
+    sa.q.s1 = q->stride[1];
+    sa.k = self ? sa.q : view_of(k);
+    if (!self) sa.k.s1 = k->stride[1];
+    sa.H = H;
+    sa.T = T;
+    sa.K = N;
+    sa.q_is_k = self ? 1 : 0;
+    sa.vec_q = vec16_ok(q);
+    sa.vec_k = self ? sa.vec_q : vec16_ok(k);
+    sa.freqs = freqs;
+    sa.rope_start = rope_start;
+    sa.sp = reinterpret_cast<float*>(w);
+    sa.qr.p = nullptr;
+    sa.qr_bf = false;
+    BDH_TRY(f32_scores(sa, p.f, B * H, s));
+    BDH_TRY(f32_dv(sa.sp, p.f, dout, dv, reinterpret_cast<float*>(w + p.dv_off), s));
+  }
+  if (numel4(dq) == 0) return BDH_OK;
+  BDH_TRY(f32_g(dout, v, g, p.tpad, s));
+  if (self) return f32_dq(g, p.tpad, q, dq, 0, freqs, rope_start, s);
+  BDH_TRY(f32_dq(g, p.tpad, k, dq, 1, nullptr, 0, s));
+  return f32_dq(g, p.tpad, q, dk, 2, nullptr, 0, s);
+}
+
 int run_bwd(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v, const bdh_tensor4* dout,
             const bdh_tensor4* dq, const bdh_tensor4* dk, const bdh_tensor4* dv, const float* freqs,
             int64_t rope_start, void* ws, size_t ws_bytes, hipStream_t s, const void* saved = nullptr) {
@@ -446,20 +499,21 @@ int run_bwd(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v, co
   const bool rope = freqs != nullptr;
   if (numel4(dq) == 0 && numel4(dv) == 0) return BDH_OK;
   if (saved != nullptr && !(self && bf && !rope)) return BDH_ERR_ARG;
-  const BwdPlan p = plan_bwd(B, H, T, N, bf, saved != nullptr, rope && self);
+  if (!bf) return run_f32_bwd(q, k, v, dout, dq, dk, dv, freqs, rope_start, ws, ws_bytes, s);
+  const BwdPlan p = plan_bwd(B, H, T, N, saved != nullptr, rope && self);
   if (ws == nullptr || ws_bytes < p.ws_bytes) return BDH_ERR_WORKSPACE;
   const int64_t BH = B * H;
 
-  if (self && bf && rope) {
+  if (self && rope) {
     const int rc = rope_fast_bwd(q, v, dout, dq, dv, freqs, rope_start, ws, ws_bytes, p, s);
     if (rc != kNotEligible) return rc;
   }
 
-  // bf16 self attention without RoPE: score tiles by the forward score kernel
+  // self attention without RoPE: score tiles by the forward score kernel
   // (or saved by the forward) and dV from them (syrk.hip), in place of steps
   // 1 and 4 below
   int fast_dv = kNotEligible;
-  if (self && bf && !rope) fast_dv = sy_bwd_dv(q, v, dout, dv, ws, p.g_off, s, saved);
+  if (self && !rope) fast_dv = sy_bwd_dv(q, v, dout, dv, ws, p.g_off, s, saved);
   if (saved != nullptr && fast_dv == kNotEligible) return BDH_ERR_ARG;  // the saved tiles are unusable here
   if (fast_dv != kNotEligible && fast_dv != BDH_OK) return fast_dv;
 
@@ -482,7 +536,7 @@ int run_bwd(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v, co
   sa.ntl = int(p.f.ntl);
   sa.qr.p = nullptr;
   sa.qr_bf = false;
-  if (fast_dv == kNotEligible) BDH_TRY(run_scores(sa, p.f, BH, bf, rope, true, s));
+  if (fast_dv == kNotEligible) BDH_TRY(run_scores(sa, p.f, BH, rope, true, s));
 
   // 2. G = dS + dS^T.
   GArgs ga;
@@ -499,12 +553,11 @@ int run_bwd(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v, co
   ga.tpad = p.tpad;
   // bf16 G from bf16 dO and V: the MFMA score kernel with the G epilogue
   // (syrk.hip); otherwise the generic tile kernel
-  const int gfast = bf ? sy_bwd_g(dout, v, ga.g, p.tpad, s) : kNotEligible;
+  const int gfast = sy_bwd_g(dout, v, ga.g, p.tpad, s);
   if (gfast != kNotEligible)
     BDH_TRY(gfast);
   else
-    BDH_TRY(bf ? run_g<true>(ga, p.f.nt, BH, dout->dtype, v->dtype, s)
-               : run_g<false>(ga, p.f.nt, BH, dout->dtype, v->dtype, s));
+    BDH_TRY(run_g(ga, p.f.nt, BH, dout->dtype, v->dtype, s));
 
   // 3. dQ (merged for self attention), dK.
   DqArgs da;
@@ -519,7 +572,7 @@ int run_bwd(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v, co
     // bf16 self attention without RoPE: the MFMA kernel with transposing LDS
     // reads (syrk.hip); otherwise the generic tile kernel below
     int fast = kNotEligible;
-    if (self && bf && !rope) fast = sy_dq(ga.g, p.tpad, gfast != kNotEligible, q, dq, s);
+    if (self && !rope) fast = sy_dq(ga.g, p.tpad, gfast != kNotEligible, q, dq, s);
     if (fast != kNotEligible) {
       BDH_TRY(fast);
     } else if (self) {
@@ -529,26 +582,22 @@ int run_bwd(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v, co
       da.o = view_of(dq);
       da.o.s1 = dq->stride[1];
       if (rope)
-        BDH_TRY(bf ? run_dq<true, 0, true>(da, p.f.nt, BH, dq->dtype, s)
-                   : run_dq<false, 0, true>(da, p.f.nt, BH, dq->dtype, s));
+        BDH_TRY(run_dq<0, true>(da, p.f.nt, BH, dq->dtype, s));
       else
-        BDH_TRY(bf ? run_dq<true, 0, false>(da, p.f.nt, BH, dq->dtype, s)
-                   : run_dq<false, 0, false>(da, p.f.nt, BH, dq->dtype, s));
+        BDH_TRY(run_dq<0, false>(da, p.f.nt, BH, dq->dtype, s));
     } else {
       da.x = view_of(k);
       da.x.s1 = k->stride[1];
       da.vec4_x = vec4_rows(k);
       da.o = view_of(dq);
       da.o.s1 = dq->stride[1];
-      BDH_TRY(bf ? run_dq<true, 1, false>(da, p.f.nt, BH, dq->dtype, s)
-                 : run_dq<false, 1, false>(da, p.f.nt, BH, dq->dtype, s));
+      BDH_TRY(run_dq<1, false>(da, p.f.nt, BH, dq->dtype, s));
       da.x = view_of(q);
       da.x.s1 = q->stride[1];
       da.vec4_x = vec4_rows(q);
       da.o = view_of(dk);
       da.o.s1 = dk->stride[1];
-      BDH_TRY(bf ? run_dq<true, 2, false>(da, p.f.nt, BH, dk->dtype, s)
-                 : run_dq<false, 2, false>(da, p.f.nt, BH, dk->dtype, s));
+      BDH_TRY(run_dq<2, false>(da, p.f.nt, BH, dk->dtype, s));
     }
   }
 
@@ -567,8 +616,7 @@ int run_bwd(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v, co
     va.vec4_do = vec4_rows(dout);
     va.o = view_of(dv);
     va.o.s1 = dv->stride[1];
-    BDH_TRY(bf ? run_dv<true>(va, p.f.nt, B * Hv, dout->dtype, dv->dtype, s)
-               : run_dv<false>(va, p.f.nt, B * Hv, dout->dtype, dv->dtype, s));
+    BDH_TRY(run_dv(va, p.f.nt, B * Hv, dout->dtype, dv->dtype, s));
   }
   return BDH_OK;
 }
@@ -580,9 +628,7 @@ using namespace bdh;
 
 extern "C" size_t bdh_tril_score_v_bwd_workspace(int64_t B, int64_t H, int64_t Hv, int64_t T, int64_t Dk,
                                                  int64_t Dv, int32_t qk_dtype) {
-  (void)Hv;
-  (void)Dv;
-  return plan_bwd(B, H, T, Dk, qk_dtype == BDH_BF16).ws_bytes;
+  return qk_dtype == BDH_BF16 ? plan_bwd(B, H, T, Dk).ws_bytes : f32_bwd_bytes(B, H, Hv, T, Dk, Dv);
 }
 
 extern "C" int bdh_tril_score_v_bwd(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v,
@@ -605,9 +651,8 @@ extern "C" int bdh_tril_score_v_keeps_scores(const bdh_tensor4* q, const bdh_ten
 
 extern "C" size_t bdh_tril_score_v_bwd_saved_workspace(int64_t B, int64_t H, int64_t Hv, int64_t T, int64_t N,
                                                        int64_t Dv, int32_t x_dtype) {
-  (void)Hv;
-  (void)Dv;
-  return plan_bwd(B, H, T, N, x_dtype == BDH_BF16, true).ws_bytes;
+  // fp32 forwards keep no tiles
+  return x_dtype == BDH_BF16 ? plan_bwd(B, H, T, N, true).ws_bytes : f32_bwd_bytes(B, H, Hv, T, N, Dv);
 }
 
 extern "C" int bdh_tril_score_v_bwd_saved(const bdh_tensor4* x, const bdh_tensor4* v, const bdh_tensor4* dout,
@@ -624,9 +669,7 @@ extern "C" int bdh_tril_score_v_bwd_saved(const bdh_tensor4* x, const bdh_tensor
 
 extern "C" size_t bdh_tril_rope_score_v_bwd_workspace(int64_t B, int64_t H, int64_t Hv, int64_t T,
                                                       int64_t N, int64_t Dv, int32_t x_dtype) {
-  (void)Hv;
-  (void)Dv;
-  return plan_bwd(B, H, T, N, x_dtype == BDH_BF16, false, true).ws_bytes;
+  return x_dtype == BDH_BF16 ? plan_bwd(B, H, T, N, false, true).ws_bytes : f32_bwd_bytes(B, H, Hv, T, N, Dv);
 }
 
 extern "C" int bdh_tril_rope_score_v_keeps_scores(const bdh_tensor4* x, const bdh_tensor4* v, size_t* scores_bytes) {

@@ -1,4 +1,4 @@
-// Forward-kernel arguments and launch helpers shared by fwd.hip and bwd.hip.
+// Forward-kernel arguments and launch helpers shared by fwd.hip, bwd.hip and f32.hip.
 #pragma once
 
 #include "tile_gemm.h"
@@ -30,6 +30,7 @@ struct ScoresArgs {
   int ntl;
   View qr;    // optional RoPE(x) output (diagonal tiles write it)
   bool qr_bf;
+  bool qr_vec = false;  // its rows start at multiples of four values (fp32 kernels)
   // Queries at an offset (chunked prefill): query row i is global row
   // past + i over keys [0, T); the launch covers the packed lower tiles from
   // t0 on (row tiles >= past / 128).  0 for the ordinary op.
@@ -99,8 +100,28 @@ size_t sy_rope_scores_workspace(int64_t B, int64_t H, int64_t T, int64_t N);
 int sy_rope_scores(const bdh_tensor4* x, const bdh_tensor4* v, const float* freqs, int64_t rope_start,
                    const bdh_tensor4* qr, void* ws, size_t ws_bytes, hipStream_t s, const void** tiles);
 
-FwdPlan plan_fwd(int64_t B, int64_t H, int64_t T, int64_t K, bool bf, int64_t past = 0);
-int run_scores(const ScoresArgs& a, const FwdPlan& p, int64_t BH, bool bf, bool rope, bool trans,
-               hipStream_t s);
+// fp32 operands (f32.hip): score tiles on the bf16 matrix cores.
+struct F32Plan {
+  int te_log = 8;       // tile edge 1 << te_log
+  int64_t nt = 0, s0 = 0, t0 = 0, ntl = 0;  // as in FwdPlan
+  int64_t nfull = 0, per = 0;               // full tiles and work items of one split of a slab
+  int64_t splits = 1, kc = 0;
+  size_t tile_bytes = 0, m_bytes = 0;       // one split's tiles; all of them
+};
+F32Plan plan_f32(int64_t B, int64_t H, int64_t T, int64_t K, bool self, int64_t past = 0);
+// M = tril(Q K^T, -1) into a.sp (packed tiles; the splits summed).
+int f32_scores(const ScoresArgs& a, const F32Plan& p, int64_t BH, hipStream_t s);
+int f32_score_v(const float* m, const F32Plan& p, const bdh_tensor4* v, const bdh_tensor4* out, int64_t T,
+                int64_t past, hipStream_t s);
+size_t f32_dv_bytes(int64_t B, int64_t H, int64_t Hv, int64_t T, int64_t Dv);
+int f32_dv(const float* m, const F32Plan& p, const bdh_tensor4* dout, const bdh_tensor4* dv, float* part,
+           hipStream_t s);
+int f32_g(const bdh_tensor4* dout, const bdh_tensor4* v, float* g, int64_t tpad, hipStream_t s);
+// mask: 0 full G (with freqs: X rotated, the result rotated back), 1 lower(G) X, 2 upper(G) X.
+int f32_dq(const float* g, int64_t tpad, const bdh_tensor4* x, const bdh_tensor4* out, int mask, const float* freqs,
+           int64_t rope_start, hipStream_t s);
+
+FwdPlan plan_fwd(int64_t B, int64_t H, int64_t T, int64_t K, int64_t past = 0);
+int run_scores(const ScoresArgs& a, const FwdPlan& p, int64_t BH, bool rope, bool trans, hipStream_t s);
 
 }  // namespace bdh

@@ -1,6 +1,8 @@
 // Cold strict-tril attention forward for gfx950:
 //   out[b,h,i,:] = sum_{j<i} <Q_i, K_j> V_j,   optionally Q = K = RoPE(x).
 //
+// bf16 operands take the kernels of syrk.hip where their constraints hold and
+// fp32 operands those of f32.hip; what follows serves every other bf16 call.
 // Two kernels per call:
 //  1. k_scores: split-K partial score tiles S = Q K^T over the packed lower
 //     tiles (ti >= tj) of every (b,h) slab.  With Q = K a diagonal tile loads
@@ -9,14 +11,16 @@
 //     tile from HBM into LDS (phase frac(pos*freq), v_sin/v_cos).
 //  2. k_score_v: out = tril(sum_splits S, -1) V, reading the partial tiles of
 //     the lower triangle only (fully masked tiles are never touched).
+#include <algorithm>
+
 #include "fwd.h"
 
 namespace bdh {
 
-template <typename TIn, bool ROPE, bool TRANS>
+template <bool ROPE, bool TRANS>
 __global__ __launch_bounds__(kNT) void k_scores(ScoresArgs a) {
-  constexpr bool BF = std::is_same<TIn, bf16_t>::value;
-  __shared__ Smem<BF> sm;
+  typedef bf16_t TIn;
+  __shared__ Smem sm;
   int ti, tj;
   lower_tile_coords(int(blockIdx.x) + a.t0, ti, tj);
   const int slab = blockIdx.y;
@@ -25,7 +29,7 @@ __global__ __launch_bounds__(kNT) void k_scores(ScoresArgs a) {
   const int kb = int(split * a.kc);
   const int ke = int(min(a.K, int64_t(kb) + a.kc));
 
-  KRows<TIn, BF, ROPE, 0> la, lb;
+  KRows<TIn, ROPE, 0> la, lb;
   la.base = static_cast<const TIn*>(a.q.p) + b * a.q.s0 + h * a.q.s1;
   la.rs = a.q.s2;
   la.r0 = ti * kTile;
@@ -63,7 +67,7 @@ __global__ __launch_bounds__(kNT) void k_scores(ScoresArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-  mainloop<BF, TRANS>(sm, la, lb, b_is_a, kb, ke, acc, active);
+  mainloop<TRANS>(sm, la, lb, b_is_a, kb, ke, acc, active);
 
   if (!active) return;
   float* dst = a.sp + (int64_t(split) * gridDim.y + slab) * a.ntl * kTileElems +
@@ -84,20 +88,20 @@ __global__ __launch_bounds__(kNT) void k_scores(ScoresArgs a) {
       }
 }
 
-template <bool BF, typename TV, typename TO>
+template <typename TV, typename TO>
 __global__ __launch_bounds__(kNT) void k_score_v(ScoreVArgs a) {
-  __shared__ Smem<BF> sm;
+  __shared__ Smem sm;
   const int R = int(blockIdx.x) + a.s0, Dt = blockIdx.y, slab = blockIdx.z;
   const int b = slab / a.H, h = slab % a.H;
   const int hv = a.Hv == 1 ? 0 : h;
 
-  SplitRows<BF, false> la;
+  SplitRows<false> la;
   la.slab = a.sp + int64_t(slab) * a.ntl * kTileElems;
   la.split_stride = a.split_stride;
   la.nsplit = a.nsplit;
   la.R = R;
   la.t0 = a.t0;
-  NRows<TV, BF, false> lb;
+  NRows<TV, false> lb;
   lb.base = static_cast<const TV*>(a.v.p) + b * a.v.s0 + hv * a.v.s1;
   lb.rs = a.v.s2;
   lb.n0 = Dt * kTile;
@@ -114,7 +118,7 @@ __global__ __launch_bounds__(kNT) void k_score_v(ScoreVArgs a) {
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
   const int ke = int(min(a.T, int64_t(R + 1) * kTile));
-  mainloop<BF, false>(sm, la, lb, false, 0, ke, acc, true);
+  mainloop<false>(sm, la, lb, false, 0, ke, acc, true);
 
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = wave >> 1, wn = wave & 1;
@@ -135,9 +139,9 @@ __global__ __launch_bounds__(kNT) void k_score_v(ScoreVArgs a) {
 // ---------------------------------------------------------------- host side
 // past > 0: only the row tiles from past / 128 on (their packed lower tiles
 // are the suffix from t0 = s0 (s0 + 1) / 2); ntl counts the tiles launched.
-FwdPlan plan_fwd(int64_t B, int64_t H, int64_t T, int64_t K, bool bf, int64_t past) {
+FwdPlan plan_fwd(int64_t B, int64_t H, int64_t T, int64_t K, int64_t past) {
   FwdPlan p;
-  const int64_t BK = bf ? Mode<true>::BK : Mode<false>::BK;
+  const int64_t BK = kBK;
   p.nt = (T + kTile - 1) / kTile;
   p.s0 = past / kTile;
   p.t0 = p.s0 * (p.s0 + 1) / 2;
@@ -156,49 +160,31 @@ FwdPlan plan_fwd(int64_t B, int64_t H, int64_t T, int64_t K, bool bf, int64_t pa
   return p;
 }
 
-template <typename TIn, bool ROPE, bool TRANS>
+template <bool ROPE, bool TRANS>
 int launch_scores(const ScoresArgs& a, const FwdPlan& p, int64_t BH, hipStream_t s) {
   if (p.ntl == 0) return BDH_OK;
   dim3 grid((unsigned)(p.ntl), unsigned(BH), unsigned(p.splits));
-  BDH_LAUNCH("k_scores", (k_scores<TIn, ROPE, TRANS>), grid, dim3(kNT), 0, s, a);
+  BDH_LAUNCH("k_scores", (k_scores<ROPE, TRANS>), grid, dim3(kNT), 0, s, a);
   return BDH_OK;
 }
 
-int run_scores(const ScoresArgs& a, const FwdPlan& p, int64_t BH, bool bf, bool rope, bool trans,
-               hipStream_t s) {
-  if (bf) {
-    if (rope) return trans ? launch_scores<bf16_t, true, true>(a, p, BH, s)
-                           : launch_scores<bf16_t, true, false>(a, p, BH, s);
-    return trans ? launch_scores<bf16_t, false, true>(a, p, BH, s)
-                 : launch_scores<bf16_t, false, false>(a, p, BH, s);
-  }
-  if (rope) return trans ? launch_scores<float, true, true>(a, p, BH, s)
-                         : launch_scores<float, true, false>(a, p, BH, s);
-  return trans ? launch_scores<float, false, true>(a, p, BH, s)
-               : launch_scores<float, false, false>(a, p, BH, s);
+int run_scores(const ScoresArgs& a, const FwdPlan& p, int64_t BH, bool rope, bool trans, hipStream_t s) {
+  if (rope) return trans ? launch_scores<true, true>(a, p, BH, s) : launch_scores<true, false>(a, p, BH, s);
+  return trans ? launch_scores<false, true>(a, p, BH, s) : launch_scores<false, false>(a, p, BH, s);
 }
 
-template <bool BF, typename TV, typename TO>
+template <typename TV, typename TO>
 int launch_score_v(const ScoreVArgs& a, int64_t nt, int64_t BH, hipStream_t s) {
   if (nt - a.s0 <= 0) return BDH_OK;
   dim3 grid((unsigned)(nt - a.s0), unsigned((a.Dv + kTile - 1) / kTile), unsigned(BH));
-  BDH_LAUNCH("k_score_v", (k_score_v<BF, TV, TO>), grid, dim3(kNT), 0, s, a);
+  BDH_LAUNCH("k_score_v", (k_score_v<TV, TO>), grid, dim3(kNT), 0, s, a);
   return BDH_OK;
 }
 
-int run_score_v(const ScoreVArgs& a, int64_t nt, int64_t BH, bool bf, int32_t v_dt, int32_t o_dt,
-                hipStream_t s) {
+int run_score_v(const ScoreVArgs& a, int64_t nt, int64_t BH, int32_t v_dt, int32_t o_dt, hipStream_t s) {
   const bool vb = v_dt == BDH_BF16, ob = o_dt == BDH_BF16;
-  if (bf) {
-    if (vb) return ob ? launch_score_v<true, bf16_t, bf16_t>(a, nt, BH, s)
-                      : launch_score_v<true, bf16_t, float>(a, nt, BH, s);
-    return ob ? launch_score_v<true, float, bf16_t>(a, nt, BH, s)
-              : launch_score_v<true, float, float>(a, nt, BH, s);
-  }
-  if (vb) return ob ? launch_score_v<false, bf16_t, bf16_t>(a, nt, BH, s)
-                    : launch_score_v<false, bf16_t, float>(a, nt, BH, s);
-  return ob ? launch_score_v<false, float, bf16_t>(a, nt, BH, s)
-            : launch_score_v<false, float, float>(a, nt, BH, s);
+  if (vb) return ob ? launch_score_v<bf16_t, bf16_t>(a, nt, BH, s) : launch_score_v<bf16_t, float>(a, nt, BH, s);
+  return ob ? launch_score_v<float, bf16_t>(a, nt, BH, s) : launch_score_v<float, float>(a, nt, BH, s);
 }
 
 static bool vec4_rows(const bdh_tensor4* t) {
@@ -244,8 +230,15 @@ static int run_cold(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor
     const int rc = sy_cold(q, k, v, out, freqs, rope_start, qr, ws, ws_bytes, s);
     if (rc != kNotEligible) return rc;
   }
-  const FwdPlan p = plan_fwd(B, H, T, K, bf);
-  if (ws == nullptr || ws_bytes < p.ws_bytes) return BDH_ERR_WORKSPACE;
+  const bool q_is_k = (q->data == k->data && q->stride[0] == k->stride[0] && q->stride[1] == k->stride[1] &&
+                       q->stride[2] == k->stride[2]);
+  FwdPlan p;
+  F32Plan pf;
+  if (bf)
+    p = plan_fwd(B, H, T, K);
+  else
+    pf = plan_f32(B, H, T, K, q_is_k);
+  if (ws == nullptr || ws_bytes < (bf ? p.ws_bytes : pf.m_bytes)) return BDH_ERR_WORKSPACE;
   if (T == 0) return BDH_OK;
 
   ScoresArgs sa;
@@ -256,8 +249,7 @@ static int run_cold(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor
   sa.H = H;
   sa.T = T;
   sa.K = K;
-  sa.q_is_k = (q->data == k->data && q->stride[0] == k->stride[0] && q->stride[1] == k->stride[1] &&
-               q->stride[2] == k->stride[2]);
+  sa.q_is_k = q_is_k;
   sa.vec_q = vec16_ok(q);
   sa.vec_k = vec16_ok(k);
   sa.freqs = freqs;
@@ -271,8 +263,13 @@ static int run_cold(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor
     sa.qr = view_of(qr);
     sa.qr.s1 = qr->stride[1];
     sa.qr_bf = qr->dtype == BDH_BF16;
+    sa.qr_vec = vec4_rows(qr);
   }
-  BDH_TRY(run_scores(sa, p, B * H, bf, freqs != nullptr, false, s));
+  if (!bf) {
+    BDH_TRY(f32_scores(sa, pf, B * H, s));
+    return numel4(out) == 0 ? BDH_OK : f32_score_v(sa.sp, pf, v, out, T, 0, s);
+  }
+  BDH_TRY(run_scores(sa, p, B * H, freqs != nullptr, false, s));
   if (numel4(out) == 0) return BDH_OK;
 
   ScoreVArgs va;
@@ -288,7 +285,7 @@ static int run_cold(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor
   va.vec4_v = vec4_rows(v);
   va.o = view_of(out);
   va.o.s1 = out->stride[1];
-  return run_score_v(va, p.nt, B * H, bf, v->dtype, out->dtype, s);
+  return run_score_v(va, p.nt, B * H, v->dtype, out->dtype, s);
 }
 
 // Queries at an offset (chunked prefill): q (B,H,T,N) are global rows
@@ -320,8 +317,13 @@ static int run_past(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor
   const int64_t Tk = past + T;
   if (numel4(out) == 0) return BDH_OK;
   const bool bf = q->dtype == BDH_BF16;
-  const FwdPlan p = plan_fwd(B, H, Tk, K, bf, past);
-  if (ws == nullptr || ws_bytes < p.ws_bytes) return BDH_ERR_WORKSPACE;
+  FwdPlan p;
+  F32Plan pf;
+  if (bf)
+    p = plan_fwd(B, H, Tk, K, past);
+  else
+    pf = plan_f32(B, H, Tk, K, false, past);
+  if (ws == nullptr || ws_bytes < (bf ? p.ws_bytes : pf.m_bytes)) return BDH_ERR_WORKSPACE;
 
   ScoresArgs sa;
   sa.q = view_of(q);
@@ -343,7 +345,11 @@ static int run_past(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor
   sa.qr_bf = false;
   sa.past = past;
   sa.t0 = int(p.t0);
-  BDH_TRY(run_scores(sa, p, B * H, bf, false, false, s));
+  if (!bf) {
+    BDH_TRY(f32_scores(sa, pf, B * H, s));
+    return f32_score_v(sa.sp, pf, v, out, Tk, past, s);
+  }
+  BDH_TRY(run_scores(sa, p, B * H, false, false, s));
 
   ScoreVArgs va;
   va.sp = sa.sp;
@@ -361,7 +367,7 @@ static int run_past(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor
   va.past = past;
   va.s0 = int(p.s0);
   va.t0 = int(p.t0);
-  return run_score_v(va, p.nt, B * H, bf, v->dtype, out->dtype, s);
+  return run_score_v(va, p.nt, B * H, v->dtype, out->dtype, s);
 }
 
 }  // namespace bdh
@@ -371,9 +377,8 @@ using namespace bdh;
 extern "C" size_t bdh_tril_score_v_past_workspace(int64_t B, int64_t H, int64_t T, int64_t past, int64_t Dk,
                                                   int64_t Dv, int32_t qk_dtype) {
   if (past <= 0) return bdh_tril_score_v_workspace(B, H, T, Dk, Dv, qk_dtype);
-  const size_t generic = plan_fwd(B, H, past + T, Dk, qk_dtype == BDH_BF16, past).ws_bytes;
-  const size_t fast = qk_dtype == BDH_BF16 ? sy_past_workspace(B, H, past + T, past, Dk, Dv) : 0;
-  return generic > fast ? generic : fast;
+  if (qk_dtype != BDH_BF16) return plan_f32(B, H, past + T, Dk, false, past).m_bytes;
+  return std::max(plan_fwd(B, H, past + T, Dk, past).ws_bytes, sy_past_workspace(B, H, past + T, past, Dk, Dv));
 }
 
 extern "C" int bdh_tril_score_v_past(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v,
@@ -389,10 +394,10 @@ extern "C" int bdh_tril_score_v_past(const bdh_tensor4* q, const bdh_tensor4* k,
 
 extern "C" size_t bdh_tril_score_v_workspace(int64_t B, int64_t H, int64_t T, int64_t Dk,
                                              int64_t Dv, int32_t qk_dtype) {
-  const size_t generic = plan_fwd(B, H, T, Dk, qk_dtype == BDH_BF16).ws_bytes;
+  if (qk_dtype != BDH_BF16)  // whether q is k is not known yet
+    return std::max(plan_f32(B, H, T, Dk, true).m_bytes, plan_f32(B, H, T, Dk, false).m_bytes);
   // bf16 operands may take the fast path (with a RoPE table when fused).
-  const size_t fast = qk_dtype == BDH_BF16 ? sy_workspace(B, H, T, Dk, Dv, true) : 0;
-  return generic > fast ? generic : fast;
+  return std::max(plan_fwd(B, H, T, Dk).ws_bytes, sy_workspace(B, H, T, Dk, Dv, true));
 }
 
 extern "C" int bdh_tril_score_v(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v,

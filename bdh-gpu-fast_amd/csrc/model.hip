@@ -298,16 +298,16 @@ struct SmallGemmArgs {
 };
 
 __global__ __launch_bounds__(kNT) void k_small_gemm(SmallGemmArgs a) {
-  __shared__ Smem<true> sm;
+  __shared__ Smem sm;
   const int n0 = blockIdx.x * kTile, split = blockIdx.y, m0 = blockIdx.z * kTile;
-  KRows<bf16_t, true, false, 0> la;
+  KRows<bf16_t, false, 0> la;
   la.base = a.a;
   la.rs = a.as;
   la.r0 = m0;
   la.nrows = a.M;
   la.K = a.K;
   la.vec = a.avec;
-  NRows<bf16_t, true, false> lb;
+  NRows<bf16_t, false> lb;
   lb.base = a.b;
   lb.rs = a.bs;
   lb.n0 = n0;
@@ -322,7 +322,7 @@ __global__ __launch_bounds__(kNT) void k_small_gemm(SmallGemmArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
   const int kb = split * a.kc, ke = min(a.K, kb + a.kc);
-  mainloop<true, false>(sm, la, lb, false, kb, ke, acc, true);
+  mainloop<false>(sm, la, lb, false, kb, ke, acc, true);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = wave >> 1, wn = wave & 1;
   float* dst = a.part + int64_t(split) * a.M * a.D;
@@ -475,7 +475,7 @@ struct SmallGemmPlan {
 inline SmallGemmPlan small_gemm_plan(int64_t M, int64_t K, int64_t D) {
   SmallGemmPlan p;
   const int64_t tiles = ((M + kTile - 1) / kTile) * ((D + kTile - 1) / kTile);
-  const int64_t BK = Mode<true>::BK;
+  const int64_t BK = kBK;
   int64_t S = tiles > 0 ? (256 + tiles - 1) / tiles : 1;
   S = std::max<int64_t>(1, std::min<int64_t>(S, (K + BK - 1) / BK));
   int64_t kc = (K + S - 1) / S;

@@ -1,5 +1,5 @@
-// 128x128 MFMA tile engine for gfx950 (CDNA4), shared by the forward,
-// score x V and backward kernels.
+// 128x128 bf16 MFMA tile engine for gfx950 (CDNA4), shared by the generic
+// forward, score x V and backward kernels.
 //
 // A workgroup is 256 threads = 4 wave64s arranged 2x2; each wave owns a 64x64
 // sub-tile made of 2x2 blocks of 32x32 MFMA accumulators (16 fp32 registers
@@ -8,10 +8,8 @@
 // stage s+1 are issued before the MFMAs of stage s, and transformed (RoPE,
 // masks, dtype conversion) and written to the other LDS buffer after them.
 //
-// bf16 mode: v_mfma_f32_32x32x16_bf16, K-stage 64, LDS pitch 72 elements
-// (144 B: conflict-free 16-byte fragment reads).  fp32 mode:
-// v_mfma_f32_32x32x2f32, K-stage 32, LDS pitch 33 floats (conflict-free
-// 4-byte fragment reads).
+// v_mfma_f32_32x32x16_bf16, K-stage 64, LDS pitch 72 elements (144 B:
+// conflict-free 16-byte fragment reads).  fp32 operands: f32_gemm.h.
 //
 // Accumulator layout of a 32x32 block (lane l, register r = 0..15):
 //   row = 8*(r/4) + 4*(l/32) + r%4, col = l%32.
@@ -29,28 +27,17 @@ constexpr int kNT = 256;    // threads per workgroup
 constexpr int kTile = 128;  // output tile edge
 constexpr int kTileElems = kTile * kTile;
 
-template <bool BF> struct Mode;
-template <> struct Mode<true> {
-  static constexpr int BK = 64;
-  static constexpr int E = 8;  // k elements per 16-byte LDS chunk
-  static constexpr int LDSW = BK + 8;
-  typedef bf16_t lds_t;
-};
-template <> struct Mode<false> {
-  static constexpr int BK = 32;
-  static constexpr int E = 4;
-  static constexpr int LDSW = BK + 1;
-  typedef float lds_t;
+constexpr int kBK = 64;        // k per stage
+constexpr int kE = 8;          // k elements per 16-byte LDS chunk
+constexpr int kLdsW = kBK + 8;
+
+struct Smem {
+  bf16_t a[2][kTile][kLdsW];
+  bf16_t b[2][kTile][kLdsW];
 };
 
-template <bool BF> struct Smem {
-  typedef typename Mode<BF>::lds_t T;
-  T a[2][kTile][Mode<BF>::LDSW];
-  T b[2][kTile][Mode<BF>::LDSW];
-};
-
-template <bool BF> using LdsTile = typename Mode<BF>::lds_t (*)[Mode<BF>::LDSW];
-template <bool BF> using CLdsTile = const typename Mode<BF>::lds_t (*)[Mode<BF>::LDSW];
+typedef bf16_t (*LdsTile)[kLdsW];
+typedef const bf16_t (*CLdsTile)[kLdsW];
 
 // Packed index of lower tile (ti >= tj).
 __device__ __forceinline__ int lower_tile_index(int ti, int tj) { return ti * (ti + 1) / 2 + tj; }
@@ -63,66 +50,38 @@ __device__ __forceinline__ void lower_tile_coords(int t, int& ti, int& tj) {
 }
 
 // Write E floats of one LDS chunk.
-template <bool BF>
-__device__ __forceinline__ void lds_put(LdsTile<BF> dst, int row, int kc, const float* f) {
-  if constexpr (BF) {
-    uint4 w;
-    w.x = pack_bf2(f[0], f[1]);
-    w.y = pack_bf2(f[2], f[3]);
-    w.z = pack_bf2(f[4], f[5]);
-    w.w = pack_bf2(f[6], f[7]);
-    *reinterpret_cast<uint4*>(&dst[row][kc]) = w;
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) dst[row][kc + e] = f[e];
-  }
+__device__ __forceinline__ void lds_put(LdsTile dst, int row, int kc, const float* f) {
+  uint4 w;
+  w.x = pack_bf2(f[0], f[1]);
+  w.y = pack_bf2(f[2], f[3]);
+  w.z = pack_bf2(f[4], f[5]);
+  w.w = pack_bf2(f[6], f[7]);
+  *reinterpret_cast<uint4*>(&dst[row][kc]) = w;
 }
 
 // One LDS stage of MFMAs for this wave's 2x2 blocks.
-template <bool BF, bool TRANS>
-__device__ __forceinline__ void mma_stage(CLdsTile<BF> A, CLdsTile<BF> B, f32x16 (&acc)[2][2],
-                                          int wm, int wn, int lane) {
+template <bool TRANS>
+__device__ __forceinline__ void mma_stage(CLdsTile A, CLdsTile B, f32x16 (&acc)[2][2], int wm, int wn, int lane) {
   const int r = lane & 31;
-  if constexpr (BF) {
-    const int ko = (lane >> 5) * 8;
+  const int ko = (lane >> 5) * 8;
 #pragma unroll
-    for (int kk = 0; kk < Mode<true>::BK; kk += 16) {
-      bf16x8 a[2], b[2];
+  for (int kk = 0; kk < kBK; kk += 16) {
+    bf16x8 a[2], b[2];
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
-        a[i] = *reinterpret_cast<const bf16x8*>(&A[wm * 64 + i * 32 + r][kk + ko]);
+    for (int i = 0; i < 2; ++i)
+      a[i] = *reinterpret_cast<const bf16x8*>(&A[wm * 64 + i * 32 + r][kk + ko]);
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-        b[j] = *reinterpret_cast<const bf16x8*>(&B[wn * 64 + j * 32 + r][kk + ko]);
+    for (int j = 0; j < 2; ++j)
+      b[j] = *reinterpret_cast<const bf16x8*>(&B[wn * 64 + j * 32 + r][kk + ko]);
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          if constexpr (TRANS)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
-          else
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-    }
-  } else {
-    const int ko = lane >> 5;
-#pragma unroll
-    for (int kk = 0; kk < Mode<false>::BK; kk += 2) {
-      float a[2], b[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) a[i] = A[wm * 64 + i * 32 + r][kk + ko];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) b[j] = B[wn * 64 + j * 32 + r][kk + ko];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          if constexpr (TRANS)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[j], a[i], acc[i][j], 0, 0, 0);
-          else
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-    }
+      for (int j = 0; j < 2; ++j) {
+        if constexpr (TRANS)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
+        else
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+      }
   }
 }
 
@@ -130,10 +89,10 @@ __device__ __forceinline__ void mma_stage(CLdsTile<BF> A, CLdsTile<BF> B, f32x16
 // loaders zero-fill past their own limits).  When b_is_a the B operand is the
 // A tile itself (diagonal tiles of Q = K), so B is neither loaded nor stored.
 // Inactive waves load and synchronise but issue no MFMAs.
-template <bool BF, bool TRANS, class LA, class LB>
-__device__ __forceinline__ void mainloop(Smem<BF>& sm, LA& la, LB& lb, bool b_is_a, int kb, int ke,
+template <bool TRANS, class LA, class LB>
+__device__ __forceinline__ void mainloop(Smem& sm, LA& la, LB& lb, bool b_is_a, int kb, int ke,
                                          f32x16 (&acc)[2][2], bool active) {
-  constexpr int BK = Mode<BF>::BK;
+  constexpr int BK = kBK;
   if (kb >= ke) return;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = wave >> 1, wn = wave & 1;
@@ -150,7 +109,7 @@ __device__ __forceinline__ void mainloop(Smem<BF>& sm, LA& la, LB& lb, bool b_is
       if (!b_is_a) lb.load(k0 + BK);
     }
     if (active)
-      mma_stage<BF, TRANS>(sm.a[buf], b_is_a ? sm.a[buf] : sm.b[buf], acc, wm, wn, lane);
+      mma_stage<TRANS>(sm.a[buf], b_is_a ? sm.a[buf] : sm.b[buf], acc, wm, wn, lane);
     if (next) {
       la.store(sm.a[buf ^ 1], k0 + BK);
       if (!b_is_a) lb.store(sm.b[buf ^ 1], k0 + BK);
@@ -179,12 +138,12 @@ __device__ __forceinline__ void acc_coord(int wm, int wn, int lane, int i, int j
 // ROPE rotates adjacent pairs along k with position pos0 + row.
 // MASK 1 keeps k < row, MASK 2 keeps k > row (global indices), MASK 0 none.
 // ------------------------------------------------------------------------
-template <typename TIn, bool BF, bool ROPE, int MASK>
+template <typename TIn, bool ROPE, int MASK>
 struct KRows {
-  static constexpr int BK = Mode<BF>::BK, E = Mode<BF>::E;
+  static constexpr int BK = kBK, E = kE;
   static constexpr int CPR = BK / E;               // chunks per row
   static constexpr int CPT = kTile * CPR / kNT;    // chunks per thread
-  static constexpr bool RAW = BF && std::is_same<TIn, bf16_t>::value && !ROPE && MASK == 0;
+  static constexpr bool RAW = std::is_same<TIn, bf16_t>::value && !ROPE && MASK == 0;
 
   const TIn* base = nullptr;
   int64_t rs = 0;    // row stride (elements)
@@ -231,7 +190,7 @@ struct KRows {
     }
   }
 
-  __device__ __forceinline__ void store(LdsTile<BF> dst, int k0) {
+  __device__ __forceinline__ void store(LdsTile dst, int k0) {
 #pragma unroll
     for (int c = 0; c < CPT; ++c) {
       const int ch = threadIdx.x + c * kNT;
@@ -264,7 +223,7 @@ struct KRows {
           for (int e = 0; e < E; ++e)
             if (!(gk + e > gr)) f[e] = 0.f;
         }
-        lds_put<BF>(dst, row, kc, f);
+        lds_put(dst, row, kc, f);
       }
     }
   }
@@ -289,9 +248,9 @@ struct KRows {
 // [n][k].  One unit of 4 columns x E k-rows per thread per stage.  ROPE
 // rotates adjacent column pairs with position pos0 + k.
 // ------------------------------------------------------------------------
-template <typename TIn, bool BF, bool ROPE>
+template <typename TIn, bool ROPE>
 struct NRows {
-  static constexpr int BK = Mode<BF>::BK, E = Mode<BF>::E;
+  static constexpr int BK = kBK, E = kE;
   static_assert((kTile / 4) * (BK / E) == kNT, "one unit per thread");
 
   const TIn* base = nullptr;
@@ -329,7 +288,7 @@ struct NRows {
     }
   }
 
-  __device__ __forceinline__ void store(LdsTile<BF> dst, int k0) {
+  __device__ __forceinline__ void store(LdsTile dst, int k0) {
     const int nq = threadIdx.x & 31, kg = threadIdx.x >> 5;
     float f[4][E];
 #pragma unroll
@@ -352,7 +311,7 @@ struct NRows {
       for (int c = 0; c < 4; ++c) f[c][e] = x[c];
     }
 #pragma unroll
-    for (int c = 0; c < 4; ++c) lds_put<BF>(dst, nq * 4 + c, kg * E, f[c]);
+    for (int c = 0; c < 4; ++c) lds_put(dst, nq * 4 + c, kg * E, f[c]);
   }
 };
 
@@ -362,9 +321,9 @@ struct NRows {
 // tile (R, C), keep j < i.  DV=true (dV): partials stored transposed, A row
 // j, k = i, tile (C, R), keep i > j.
 // ------------------------------------------------------------------------
-template <bool BF, bool DV>
+template <bool DV>
 struct SplitRows {
-  static constexpr int BK = Mode<BF>::BK, E = Mode<BF>::E;
+  static constexpr int BK = kBK, E = kE;
   static constexpr int CPR = BK / E;
   static constexpr int CPT = kTile * CPR / kNT;
 
@@ -404,7 +363,7 @@ struct SplitRows {
     }
   }
 
-  __device__ __forceinline__ void store(LdsTile<BF> dst, int k0) {
+  __device__ __forceinline__ void store(LdsTile dst, int k0) {
 #pragma unroll
     for (int c = 0; c < CPT; ++c) {
       const int ch = threadIdx.x + c * kNT;
@@ -416,7 +375,7 @@ struct SplitRows {
         const bool keep = DV ? (gk + e > gr) : (gk + e < gr);
         f[e] = keep ? v[c][e] : 0.f;
       }
-      lds_put<BF>(dst, row, kc, f);
+      lds_put(dst, row, kc, f);
     }
   }
 };
