@@ -1,10 +1,10 @@
 // KV-cache decode step for gfx950: out = (q K_past^T) V_past.
 //
 // HBM-bound: every past key row (N = 8192 elements) is read exactly once per
-// query row.  Work is split over the past (chunks of keys per workgroup) so a
-// B*H = 256 row batch still fills the chip; partial outputs over chunks are
-// summed by a second small kernel (the op is linear in the scores, so no
-// renormalisation is needed).
+// query row.  Work is split over the past (chunks of keys per workgroup, from
+// 64 down to 4 so that a small batch or a short past still fills the chip:
+// dec_chunk); partial outputs over chunks are summed by a second small kernel
+// (the op is linear in the scores, so no renormalisation is needed).
 //
 // Three score kernels share that shape: k_decode_bf16 (bf16 q and keys,
 // v_dot2 products), k_decode_f32q (fp32 arithmetic, fp32 or bf16 keys, q of
@@ -12,6 +12,7 @@
 // streams key rows with 16-byte loads, reduces the dot product across the wave
 // with shuffles and records the score in LDS; then all 256 threads form the
 // partial out[d] = sum_s score_s V[s,d] with coalesced V row reads.
+#include <algorithm>
 #include <mutex>
 
 #include "common.h"
@@ -19,7 +20,7 @@
 namespace bdh {
 
 constexpr int kDecNT = 256;
-constexpr int kChunk = 32;  // keys per workgroup
+constexpr int kChunk = 32;  // most keys per workgroup
 
 struct DecodeArgs {
   View q, k, v;
@@ -27,6 +28,7 @@ struct DecodeArgs {
   int vec_k;
   float* part;    // [nchunk][rows][Dv]
   int64_t rows;   // B*H*Tq
+  int chunk;      // keys per workgroup
 };
 
 template <typename TK>
@@ -75,8 +77,8 @@ __global__ __launch_bounds__(kDecNT) void k_decode_partial(DecodeArgs a) {
   for (int64_t e = threadIdx.x; e < a.Dk; e += kDecNT) qs[e] = to_f(qp[e]);
   __syncthreads();
 
-  const int64_t s0 = int64_t(blockIdx.x) * kChunk;
-  const int64_t s1 = min(a.S, s0 + kChunk);
+  const int64_t s0 = int64_t(blockIdx.x) * a.chunk;
+  const int64_t s1 = min(a.S, s0 + a.chunk);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const TK* kb = static_cast<const TK*>(a.k.p) + b * a.k.s0 + h * a.k.s1;
   for (int64_t s = s0 + wave; s < s1; s += kDecNT / 64) {
@@ -99,7 +101,9 @@ __global__ __launch_bounds__(kDecNT) void k_decode_partial(DecodeArgs a) {
 // in flight per lane, accumulating v_dot2_f32_bf16 (exact bf16 products, fp32
 // sums) against the staged q; then the 256 threads form the chunk's partial
 // out[d] = sum_s score_s V[s,d].  Needs Dk a multiple of 2048.
-constexpr int kDecChunkB = 64;  // keys per workgroup
+// HALF (chunks of 4, a key per wave): the eight loads in flight go to the two
+// halves of one key row; Dk a multiple of 4096.
+constexpr int kDecChunkB = 64;  // most keys per workgroup
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 // (The dwords are copied to scalars before the bit cast: this clang lowers
@@ -116,7 +120,7 @@ __device__ __forceinline__ float dot8(u32x4 k, u32x4 q, float acc) {
   return dot2w(k3, q3, acc);
 }
 
-template <typename TV>
+template <typename TV, bool HALF>
 __global__ __launch_bounds__(kDecNT) void k_decode_bf16(DecodeArgs a) {
   extern __shared__ float smem[];
   float* sc = smem;                                         // kDecChunkB scores
@@ -129,16 +133,16 @@ __global__ __launch_bounds__(kDecNT) void k_decode_bf16(DecodeArgs a) {
   for (int64_t i = threadIdx.x; i < a.Dk / 8; i += kDecNT) qs[i] = *reinterpret_cast<const u32x4*>(qp + 8 * i);
   __syncthreads();
 
-  const int64_t s0 = int64_t(blockIdx.x) * kDecChunkB;
-  const int64_t s1 = min(a.S, s0 + kDecChunkB);
+  const int64_t s0 = int64_t(blockIdx.x) * a.chunk;
+  const int64_t s1 = min(a.S, s0 + a.chunk);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const bf16_t* kb = static_cast<const bf16_t*>(a.k.p) + b * a.k.s0 + h * a.k.s1;
-  const int nc = int(a.Dk / 512);  // 16-byte chunks per lane per key row
+  const int nc = int(a.Dk / (HALF ? 1024 : 512));  // 16-byte chunks per lane per key row (or half)
   // keys s0 + wave + 4 j of this wave, in pairs (s, s + 4)
   for (int64_t s = s0 + wave; s < s1; s += 8) {
-    const bool two = s + 4 < s1;
+    const bool two = !HALF && s + 4 < s1;
     const bf16_t* k0 = kb + s * a.k.s2 + lane * 8;
-    const bf16_t* k1 = kb + (two ? s + 4 : s) * a.k.s2 + lane * 8;
+    const bf16_t* k1 = HALF ? k0 + nc * 512 : kb + (two ? s + 4 : s) * a.k.s2 + lane * 8;
     float acc0 = 0.f, acc1 = 0.f;
     for (int c = 0; c < nc; c += 4) {
       u32x4 x0[4], x1[4];
@@ -151,11 +155,15 @@ __global__ __launch_bounds__(kDecNT) void k_decode_bf16(DecodeArgs a) {
       for (int u = 0; u < 4; ++u) {
         const u32x4 q = qs[(c + u) * 64 + lane];
         acc0 = dot8(x0[u], q, acc0);
-        acc1 = dot8(x1[u], q, acc1);
+        acc1 = dot8(x1[u], HALF ? qs[(nc + c + u) * 64 + lane] : q, acc1);
       }
     }
-    acc0 = wave_sum(acc0);
-    acc1 = wave_sum(acc1);
+    if constexpr (HALF) {
+      acc0 = wave_sum(acc0 + acc1);
+    } else {
+      acc0 = wave_sum(acc0);
+      acc1 = wave_sum(acc1);
+    }
     if (lane == 0) {
       sc[s - s0] = acc0;
       if (two) sc[s + 4 - s0] = acc1;
@@ -182,7 +190,8 @@ __global__ __launch_bounds__(kDecNT) void k_decode_bf16(DecodeArgs a) {
 // qs[(NP c + p) 64 + lane].  Each wave scores two key rows at a time with
 // eight 16-byte loads in flight per lane; then the 256 threads form the
 // chunk's partial out[d] = sum_s score_s V[s,d].  Needs Dk a multiple of
-// 64 EK and 16-byte aligned q and key rows.
+// 64 EK and 16-byte aligned q and key rows.  HALF as in k_decode_bf16; Dk a
+// multiple of 512 EK.
 template <typename TK>
 __device__ __forceinline__ float dot_piece(const u32x4& w, const float4* qs4, int np_stride, float acc) {
   if constexpr (sizeof(TK) == 4) {
@@ -205,7 +214,7 @@ __device__ __forceinline__ float dot_piece(const u32x4& w, const float4* qs4, in
   }
 }
 
-template <typename TQ, typename TK, typename TV>
+template <typename TQ, typename TK, typename TV, bool HALF>
 __global__ __launch_bounds__(kDecNT) void k_decode_f32q(DecodeArgs a) {
   constexpr int EK = 16 / int(sizeof(TK));  // key elements per 16-byte piece
   constexpr int NP = EK / 4;                // float4 planes of q per piece
@@ -233,17 +242,17 @@ __global__ __launch_bounds__(kDecNT) void k_decode_f32q(DecodeArgs a) {
   }
   __syncthreads();
 
-  const int64_t s0 = int64_t(blockIdx.x) * kDecChunkB;
-  const int64_t s1 = min(a.S, s0 + kDecChunkB);
+  const int64_t s0 = int64_t(blockIdx.x) * a.chunk;
+  const int64_t s1 = min(a.S, s0 + a.chunk);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const TK* kb = static_cast<const TK*>(a.k.p) + b * a.k.s0 + h * a.k.s1;
-  const int nc = int(a.Dk / (64 * EK));  // 16-byte pieces per lane per key row
+  const int nc = int(a.Dk / ((HALF ? 128 : 64) * EK));  // 16-byte pieces per lane per key row (or half)
   const float4* ql = qs + lane;
   // keys s0 + wave + 4 j of this wave, in pairs (s, s + 4)
   for (int64_t s = s0 + wave; s < s1; s += 8) {
-    const bool two = s + 4 < s1;
+    const bool two = !HALF && s + 4 < s1;
     const TK* k0 = kb + s * a.k.s2 + lane * EK;
-    const TK* k1 = kb + (two ? s + 4 : s) * a.k.s2 + lane * EK;
+    const TK* k1 = HALF ? k0 + nc * 64 * EK : kb + (two ? s + 4 : s) * a.k.s2 + lane * EK;
     float acc0 = 0.f, acc1 = 0.f;
     int c = 0;
     for (; c + 4 <= nc; c += 4) {
@@ -257,18 +266,22 @@ __global__ __launch_bounds__(kDecNT) void k_decode_f32q(DecodeArgs a) {
       for (int u = 0; u < 4; ++u) {
         const float4* q = ql + (NP * (c + u)) * 64;
         acc0 = dot_piece<TK>(x0[u], q, 64, acc0);
-        acc1 = dot_piece<TK>(x1[u], q, 64, acc1);
+        acc1 = dot_piece<TK>(x1[u], HALF ? q + NP * nc * 64 : q, 64, acc1);
       }
     }
-    for (; c < nc; ++c) {
+    for (; !HALF && c < nc; ++c) {
       const u32x4 x0 = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(k0 + c * 64 * EK));
       const u32x4 x1 = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(k1 + c * 64 * EK));
       const float4* q = ql + (NP * c) * 64;
       acc0 = dot_piece<TK>(x0, q, 64, acc0);
       acc1 = dot_piece<TK>(x1, q, 64, acc1);
     }
-    acc0 = wave_sum(acc0);
-    acc1 = wave_sum(acc1);
+    if constexpr (HALF) {
+      acc0 = wave_sum(acc0 + acc1);
+    } else {
+      acc0 = wave_sum(acc0);
+      acc1 = wave_sum(acc1);
+    }
     if (lane == 0) {
       sc[s - s0] = acc0;
       if (two) sc[s + 4 - s0] = acc1;
@@ -285,20 +298,54 @@ __global__ __launch_bounds__(kDecNT) void k_decode_f32q(DecodeArgs a) {
   }
 }
 
+// out = sum over the chunks of their partials: 32 outputs a workgroup, eight
+// groups of lanes each take every eighth chunk with four loads in flight, the
+// groups' sums added through LDS (a few dozen chunks of a small batch are a
+// chain of loads otherwise).
+constexpr int kRedCols = 32, kRedGroups = kDecNT / kRedCols;
 template <typename TO>
 __global__ __launch_bounds__(kDecNT) void k_decode_reduce(const float* part, int64_t nchunk, int64_t rows,
                                                           int64_t Dv, View o, int64_t H, int64_t Tq) {
-  const int64_t idx = int64_t(blockIdx.x) * kDecNT + threadIdx.x;
-  if (idx >= rows * Dv) return;
-  const int64_t row = idx / Dv, d = idx % Dv;
+  __shared__ float sums[kRedGroups][kRedCols];
+  const int g = threadIdx.x / kRedCols, l = threadIdx.x % kRedCols;
+  const int64_t idx = int64_t(blockIdx.x) * kRedCols + l, n = rows * Dv;
   float s = 0.f;
-  for (int64_t c = 0; c < nchunk; ++c) s += part[(c * rows + row) * Dv + d];
+  if (idx < n) {
+    for (int64_t c = g; c < nchunk; c += 4 * kRedGroups) {
+      float w[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[u] = part[min(c + u * kRedGroups, nchunk - 1) * n + idx];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) s += c + u * kRedGroups < nchunk ? w[u] : 0.f;
+    }
+  }
+  sums[g][l] = s;
+  __syncthreads();
+  if (g != 0 || idx >= n) return;
+#pragma unroll
+  for (int u = 1; u < kRedGroups; ++u) s += sums[u][l];
+  const int64_t row = idx / Dv, d = idx % Dv;
   const int64_t t = row % Tq, bh = row / Tq, h = bh % H, b = bh / H;
   TO* op = static_cast<TO*>(const_cast<void*>(o.p)) + b * o.s0 + h * o.s1 + t * o.s2;
   op[d] = from_f<TO>(s);
 }
 
-static int64_t n_chunks(int64_t S) { return S > 0 ? (S + kChunk - 1) / kChunk : 1; }
+// Keys per workgroup: 64 where that already makes three workgroups per CU
+// (8 sequences, 32 rows, S = 1500: 127 us, 145 in 32-key chunks), else the
+// largest of 32 ... 4 that makes eight, as long as the partial sums fit the
+// no-allocation scratch (a call that fits it with 64-key chunks keeps doing
+// so).  N = 8192, nh = 4, 64-key chunks -> this rule: one sequence of fp32
+// keys at S = 301 53.5 -> 14 us, at S = 1500 58 -> 39; 8 sequences of bf16
+// keys at S = 301 40 -> 32, at S = 100 37 -> 15.
+static int dec_chunk(int64_t rows, int64_t S, int64_t Dv) {
+  int chunk = kDecChunkB;
+  if (rows * ((S + chunk - 1) / chunk) >= 768) return chunk;
+  while (chunk > 4 && rows * ((S + chunk - 1) / chunk) < 2048 &&
+         (S + chunk / 2 - 1) / (chunk / 2) * rows * Dv * int64_t(sizeof(float)) <= BDH_NOALLOC_SCRATCH_BYTES)
+    chunk /= 2;
+  return chunk;
+}
+static int64_t n_chunks(int64_t S, int64_t chunk) { return S > 0 ? (S + chunk - 1) / chunk : 1; }
 
 template <typename TQ, typename TK, typename TV>
 static int launch_partial(const DecodeArgs& a, int64_t nchunk, hipStream_t s) {
@@ -323,7 +370,10 @@ template <typename TQ, typename TK, typename TV>
 static int launch_f32q_t(const DecodeArgs& a, int64_t nred, hipStream_t s) {
   const dim3 grid((unsigned)nred, unsigned(a.rows));
   const size_t shm = size_t(kDecChunkB) * sizeof(float) + size_t(a.Dk) * sizeof(float);
-  BDH_LAUNCH("k_decode_f32q", (k_decode_f32q<TQ, TK, TV>), grid, dim3(kDecNT), shm, s, a);
+  if (a.chunk == 4 && a.Dk % (8192 / int(sizeof(TK))) == 0)
+    BDH_LAUNCH("k_decode_f32q", (k_decode_f32q<TQ, TK, TV, true>), grid, dim3(kDecNT), shm, s, a);
+  else
+    BDH_LAUNCH("k_decode_f32q", (k_decode_f32q<TQ, TK, TV, false>), grid, dim3(kDecNT), shm, s, a);
   return BDH_OK;
 }
 
@@ -345,7 +395,8 @@ using namespace bdh;
 extern "C" size_t bdh_tril_decode_workspace(int64_t B, int64_t H, int64_t Tq, int64_t S, int64_t Dk,
                                             int64_t Dv) {
   (void)Dk;
-  return size_t(n_chunks(S)) * size_t(B * H * Tq) * size_t(Dv) * sizeof(float);
+  const int64_t chunk = std::min(kChunk, dec_chunk(B * H * Tq, S, Dv));
+  return size_t(n_chunks(S, chunk)) * size_t(B * H * Tq) * size_t(Dv) * sizeof(float);
 }
 
 namespace bdh {
@@ -376,7 +427,7 @@ int decode_plan(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v
   if (out->size[0] != B || out->size[1] != H || out->size[2] != Tq || out->size[3] != Dv)
     return BDH_ERR_SHAPE;
   if (views_overlap(out, q) || views_overlap(out, k) || views_overlap(out, v)) return BDH_ERR_ALIAS;
-  if (B * H * Tq > 65535 || n_chunks(S) > int64_t(1) << 30) return BDH_ERR_SHAPE;
+  if (B * H * Tq > 65535 || n_chunks(S, kChunk) > int64_t(1) << 30) return BDH_ERR_SHAPE;
   if ((Dk + kChunk) * int64_t(sizeof(float)) > 64 * 1024) return BDH_ERR_SHAPE;
   DecodeArgs& a = p.a;
   a.q = view_of(q);
@@ -402,7 +453,9 @@ int decode_plan(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v
     p.kind = kDecF32q;
   else
     p.kind = kDecGeneric;
-  p.nred = p.kind == kDecGeneric ? n_chunks(S) : (S + kDecChunkB - 1) / kDecChunkB;
+  a.chunk = dec_chunk(a.rows, S, Dv);
+  if (p.kind == kDecGeneric) a.chunk = std::min(kChunk, a.chunk);
+  p.nred = n_chunks(S, a.chunk);
   p.part_bytes = size_t(p.nred) * size_t(a.rows) * size_t(Dv) * sizeof(float);
   return BDH_OK;
 }
@@ -416,10 +469,18 @@ int decode_run(const DecodePlan& p, const bdh_tensor4* q, const bdh_tensor4* k, 
   if (p.kind == kDecBf16) {
     const dim3 grid((unsigned)p.nred, unsigned(a.rows));
     const size_t shm = size_t(kDecChunkB) * sizeof(float) + size_t(a.Dk) * 2;
-    if (v->dtype == BDH_BF16)
-      BDH_LAUNCH("k_decode_bf16", k_decode_bf16<bf16_t>, grid, dim3(kDecNT), shm, st, a);
-    else
-      BDH_LAUNCH("k_decode_bf16", k_decode_bf16<float>, grid, dim3(kDecNT), shm, st, a);
+    const bool half = a.chunk == 4 && a.Dk % 4096 == 0;
+    if (v->dtype == BDH_BF16) {
+      if (half)
+        BDH_LAUNCH("k_decode_bf16", (k_decode_bf16<bf16_t, true>), grid, dim3(kDecNT), shm, st, a);
+      else
+        BDH_LAUNCH("k_decode_bf16", (k_decode_bf16<bf16_t, false>), grid, dim3(kDecNT), shm, st, a);
+    } else {
+      if (half)
+        BDH_LAUNCH("k_decode_bf16", (k_decode_bf16<float, true>), grid, dim3(kDecNT), shm, st, a);
+      else
+        BDH_LAUNCH("k_decode_bf16", (k_decode_bf16<float, false>), grid, dim3(kDecNT), shm, st, a);
+    }
   } else if (p.kind == kDecF32q) {
     const int rc = launch_f32q(a, p.nred, q->dtype, k->dtype, v->dtype, st);
     if (rc != BDH_OK) return rc;
@@ -431,7 +492,7 @@ int decode_run(const DecodePlan& p, const bdh_tensor4* q, const bdh_tensor4* k, 
   View o = view_of(out);
   o.s1 = out->stride[1];
   const int64_t total = a.rows * a.Dv;
-  dim3 grid((unsigned)((total + kDecNT - 1) / kDecNT));
+  dim3 grid((unsigned)((total + kRedCols - 1) / kRedCols));
   if (out->dtype == BDH_BF16)
     BDH_LAUNCH("k_decode_reduce", k_decode_reduce<bf16_t>, grid, dim3(kDecNT), 0, st, a.part, p.nred, a.rows,
                a.Dv, o, a.H, a.Tq);
