@@ -37,6 +37,8 @@ from torch import nn
 
 import kernels
 from bdh_cache import CacheManager
+from kernels import hip_attn
+from kernels.attention_bwd import _save_scores
 
 
 @dataclasses.dataclass
@@ -211,6 +213,121 @@ def _chains_decoder(x_bthn: torch.Tensor, y_ln: torch.Tensor, dec: torch.Tensor)
             and D == 256 and dec.size(1) == 256 and N % 32 == 0 and B * T > 256 and N * D * 2 < 2**32)
 
 
+# Training forms on the HIP path under bf16 autocast: the layer's latent-sized
+# work as two autograd functions, so that the backward writes and reads each
+# latent-sized tensor (1.07 GB a layer at 16384 tokens, nh*N = 32768) as few
+# times as its products need: torch's own graph of the same layer makes
+# separate passes for each ReLU, product, stack, add and threshold.
+def _padded_rows(B: int, T: int, nh: int, N: int, dtype: torch.dtype, device) -> torch.Tensor:
+    """A (B, T, nh, N) tensor whose token rows lie nh*N + _XS_PAD elements apart."""
+    return torch.empty(B, T, nh * N + _XS_PAD, dtype=dtype, device=device).narrow(2, 0, nh * N).unflatten(2, (nh, N))
+
+
+class _EncodeAttend(torch.autograd.Function):
+    """x (B, T, D) -> the latent relu(x @ encoder) (B, T, nh, N) and its attention over x,
+    (B, nh, T, D).  ``enc_t`` is ``encoder`` in bf16 as (nh, N, D)."""
+
+    @staticmethod
+    def forward(ctx, x, encoder, enc_t, freqs):  # type: ignore[override]
+        B, T, D = x.shape
+        nh, N, _ = enc_t.shape
+        xb = x.to(torch.bfloat16).contiguous()
+        lat = kernels.relu_gemm(xb.unsqueeze(1).expand(B, nh, T, D), enc_t,
+                                out=_padded_rows(B, T, nh, N, torch.bfloat16, x.device))
+        xs = lat.permute(0, 2, 1, 3)
+        scores = None
+        if _save_scores():
+            y, scores = hip_attn.tril_rope_score_v_save(xs, xb.unsqueeze(1), freqs, 0)
+        else:
+            y = hip_attn.tril_rope_score_v(xs, xb.unsqueeze(1), freqs, 0)
+        ctx.has_scores = scores is not None
+        ctx.save_for_backward(xb, lat, enc_t, freqs, *((scores,) if scores is not None else ()))
+        ctx.dtypes = x.dtype, encoder.dtype
+        return lat, y
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, g_lat, g_y):  # type: ignore[override]
+        xb, lat, enc_t, freqs, *kept = ctx.saved_tensors
+        B, T, nh, N = lat.shape
+        D = xb.size(-1)
+        xs, v = lat.permute(0, 2, 1, 3), xb.unsqueeze(1)
+        g_y = g_y.to(torch.bfloat16).contiguous()
+        d_lat = _padded_rows(B, T, nh, N, torch.bfloat16, lat.device)
+        d_v = torch.empty(B, 1, T, D, dtype=torch.float32, device=lat.device)
+        g_lat, d_xs = g_lat.to(torch.bfloat16), d_lat.permute(0, 2, 1, 3)
+        if ctx.has_scores:
+            hip_attn.tril_rope_score_v_bwd_saved(xs, v, g_y, freqs, 0, kept[0], dx=d_xs, dv=d_v,
+                                                 relu_add=g_lat.permute(0, 2, 1, 3))
+        else:
+            hip_attn.tril_rope_score_v_bwd(xs, v, g_y, freqs, 0, dx=d_xs, dv=d_v)
+            kernels.relu_bwd_add(d_lat, g_lat, lat, out=d_lat)
+        dz = d_lat.flatten(2).flatten(0, 1)
+        dx = dw = None
+        if ctx.needs_input_grad[0]:
+            dx = (d_v.view(B * T, D) + dz @ enc_t.view(nh * N, D)).view(B, T, D).to(ctx.dtypes[0])
+        if ctx.needs_input_grad[1]:
+            dw = (xb.view(B * T, D).t() @ dz).view(D, nh, N).permute(1, 0, 2).to(ctx.dtypes[1])
+        return dx, dw, None, None
+
+
+class _GateDecode(torch.autograd.Function):
+    """(latent, LN(attention) (B, nh, T, D)) -> (latent * relu(y @ encoder_v)) @ decoder (B, T, D).
+    ``encv_t`` is ``encoder_v`` in bf16 as (nh, N, D), ``dec`` the decoder in bf16."""
+
+    @staticmethod
+    def forward(ctx, lat, y, encoder_v, decoder, encv_t, dec):  # type: ignore[override]
+        B, T, nh, N = lat.shape
+        # head-major rows: each head's tokens are one matrix for the backward's products
+        yb = y.permute(1, 0, 2, 3).to(torch.bfloat16, memory_format=torch.contiguous_format)
+        yv = yb.permute(1, 0, 2, 3)
+        # (kept for the decoder's gradient, which contracts it over the tokens)
+        xy = kernels.gated_gemm(yv, encv_t, lat, out=_padded_rows(B, T, nh, N, lat.dtype, lat.device))
+        out = (xy.flatten(2).flatten(0, 1) @ dec).view(B, T, -1)
+        ctx.save_for_backward(lat, yb, xy, encv_t, dec)
+        ctx.dtypes = y.dtype, encoder_v.dtype, decoder.dtype
+        return out
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, g):  # type: ignore[override]
+        lat, yb, xy, encv_t, dec = ctx.saved_tensors
+        B, T, nh, N = lat.shape
+        M, D = B * T, yb.size(-1)
+        gb = g.to(torch.bfloat16).contiguous()
+        # dz head-major: each head's rows are the operand of two products
+        zh = torch.empty(nh, M, N + _XS_PAD, dtype=lat.dtype, device=lat.device).narrow(2, 0, N)
+        d_lat, _ = kernels.gated_bwd(yb.permute(1, 0, 2, 3), encv_t, lat, dec, gb,
+                                     dx=_padded_rows(B, T, nh, N, lat.dtype, lat.device),
+                                     dz=zh.unflatten(1, (B, T)).permute(1, 2, 0, 3))
+        yh = yb.view(nh, M, D)
+        dy = dw = dd = None
+        if ctx.needs_input_grad[1]:
+            dy = torch.empty_like(yh)
+            for h in range(nh):
+                torch.mm(zh[h], encv_t[h], out=dy[h])
+            dy = dy.view(nh, B, T, D).permute(1, 0, 2, 3).to(ctx.dtypes[0])
+        if ctx.needs_input_grad[2]:
+            dw = torch.empty(nh, D, N, dtype=torch.bfloat16, device=lat.device)
+            for h in range(nh):
+                torch.mm(yh[h].t(), zh[h], out=dw[h])
+            dw = dw.to(ctx.dtypes[1])
+        if ctx.needs_input_grad[3]:
+            dd = (xy.flatten(2).flatten(0, 1).t() @ gb.view(M, D)).to(ctx.dtypes[2])
+        return d_lat, dy, dw, dd, None, None
+
+
+def _trains_fused(x: torch.Tensor, encoder: torch.Tensor) -> bool:
+    """Whether a training layer takes the fused functions: bf16 autocast on the
+    GPU, n_embd a multiple of 32 and N of 8 (the gated kernels' K stages and
+    16-byte rows), one head's rows of every operand under 4 GiB."""
+    nh, D, N = encoder.shape
+    B, T, _ = x.shape
+    return (x.is_cuda and torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16
+            and x.dtype == torch.float32 and D % 32 == 0 and N % 8 == 0 and B * T * D * 2 <= 2**32
+            and N * D * 2 < 2**32 and B * T > 0)
+
+
 def _follows(past: torch.Tensor, new: torch.Tensor) -> Optional[torch.Tensor]:
     """past||new as one view when ``new`` is the rows right after ``past`` in the
     same buffer (the reserved slot after the committed rows), else None."""
@@ -353,6 +470,12 @@ class BDH(nn.Module):
 
         fast = impl == "hip" and not torch.is_grad_enabled()
         x = _ln(self.embed(idx))  # (B, T, D)
+        fused = impl == "hip" and torch.is_grad_enabled() and cache is None and _trains_fused(x, self.encoder)
+        if fused:  # (laid out anew for every forward: a training step changes them)
+            with torch.no_grad():
+                enc_t, encv_t = (w.transpose(1, 2).to(torch.bfloat16, memory_format=torch.contiguous_format)
+                                 for w in (self.encoder, self.encoder_v))
+                dec = self.decoder.to(torch.bfloat16).contiguous()
         prep = self._prepared(_compute_dtype(x)) if fast else None
         # Under bf16 compute the encoder and the attention's V take the fp32 residual
         # stream x rounded to bf16 (autocast's matmuls, bdh.py:396-413, 861-912).  From
@@ -362,6 +485,11 @@ class BDH(nn.Module):
         xb = None
         v_bf16 = fast and (cache is None or (isinstance(cache, KVCache) and cache.dtype == torch.bfloat16))
         for level in range(cfg.n_layer):
+            if fused:
+                lat, y_kv = _EncodeAttend.apply(x, self.encoder, enc_t, self.freqs)
+                y_mlp = _GateDecode.apply(lat, _ln(y_kv), self.encoder_v, self.decoder, encv_t, dec)
+                x = _ln(x + _ln(y_mlp))
+                continue
             if fast:
                 x_bthn = _encode_fast(x if xb is None else xb, prep, nh)
             else:

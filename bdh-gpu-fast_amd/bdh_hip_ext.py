@@ -51,6 +51,8 @@ __all__ = [
     "gated_gemm",
     "relu_gemm",
     "gated_decoder",
+    "gated_bwd",
+    "relu_bwd_add",
     "small_gemm",
     "layer_norm_rows",
     "profile_enable",
@@ -84,11 +86,14 @@ EXPORTED_SYMBOLS = (
     "bdh_tril_rope_score_v_keeps_scores",
     "bdh_tril_rope_score_v_bwd_saved_workspace",
     "bdh_tril_rope_score_v_bwd_saved",
+    "bdh_tril_rope_score_v_bwd_saved_relu",
     "bdh_relu_mul",
     "bdh_gated_gemm",
     "bdh_relu_gemm",
     "bdh_gated_decoder_workspace",
     "bdh_gated_decoder",
+    "bdh_gated_bwd",
+    "bdh_relu_bwd_add",
     "bdh_small_gemm_workspace",
     "bdh_small_gemm",
     "bdh_layer_norm_rows",
@@ -151,6 +156,7 @@ def _load():
         "bdh_tril_rope_score_v_keeps_scores": (ctypes.c_int, [P, P, ctypes.POINTER(sz)]),
         "bdh_tril_rope_score_v_bwd_saved_workspace": (sz, [i64, i64, i64, i64, i64, i64, i32]),
         "bdh_tril_rope_score_v_bwd_saved": (ctypes.c_int, [P, P, P, fp, i64, P, P, vp, sz, vp, sz, vp]),
+        "bdh_tril_rope_score_v_bwd_saved_relu": (ctypes.c_int, [P, P, P, P, fp, i64, P, P, vp, sz, vp, sz, vp]),
         "bdh_relu_mul": (ctypes.c_int, [P, P, P, vp]),
         "bdh_layer_norm_rows": (ctypes.c_int, [P, P, P, vp]),
         "bdh_layer_norm_rows2": (ctypes.c_int, [P, P, P, P, vp]),
@@ -158,6 +164,8 @@ def _load():
         "bdh_relu_gemm": (ctypes.c_int, [P, P, P, vp]),
         "bdh_gated_decoder_workspace": (sz, [i64, i64]),
         "bdh_gated_decoder": (ctypes.c_int, [P, P, P, P, P, vp, sz, vp]),
+        "bdh_gated_bwd": (ctypes.c_int, [P, P, P, P, P, P, P, vp]),
+        "bdh_relu_bwd_add": (ctypes.c_int, [P, P, P, P, vp]),
         "bdh_small_gemm_workspace": (sz, [i64, i64, i64]),
         "bdh_small_gemm": (ctypes.c_int, [P, P, P, vp, sz, vp]),
         "bdh_profile_enable": (None, [i32]),
@@ -389,25 +397,32 @@ def tril_rope_score_v_bwd_saved(
     rope_start: int,
     scores: torch.Tensor,
     *,
+    dx: Optional[torch.Tensor] = None,
     dv: Optional[torch.Tensor] = None,
+    relu_add: Optional[torch.Tensor] = None,
 ) -> Tuple[torch.Tensor, torch.Tensor]:
     """``(dx, dv)`` of :func:`tril_rope_score_v` from the score tiles kept by
     :func:`tril_rope_score_v_save` on the same ``x``, ``v``, ``freqs`` and
-    ``rope_start`` (no recompute of the tiles)."""
-    dev = _require_device(x, v, dout, scores, dv)
+    ``rope_start`` (no recompute of the tiles).  ``relu_add`` (the gradient of
+    another use of ``x``, itself a ReLU's output): ``dx`` is ``gradient +
+    relu_add`` where ``x > 0``, else 0 (bf16)."""
+    dev = _require_device(x, v, dout, scores, dx, dv, relu_add)
     B, H, T, N = x.shape
     f, fptr = _freqs_ptr(freqs, N, dev)
-    dx = torch.empty_like(x, memory_format=torch.contiguous_format)
+    if dx is None:
+        dx = torch.empty_like(x, memory_format=torch.contiguous_format)
     if dv is None:
         dv = torch.empty_like(v, memory_format=torch.contiguous_format)
     with torch.cuda.device(dev):
         need = _lib.bdh_tril_rope_score_v_bwd_saved_workspace(B, H, v.size(1), T, N, v.size(-1), _dtype_code(x))
         ws, nb = _workspace(need, dev)
-        rc = _lib.bdh_tril_rope_score_v_bwd_saved(
-            ctypes.byref(_t4(x)), ctypes.byref(_t4(v)), ctypes.byref(_t4(dout)), fptr, int(rope_start),
-            ctypes.byref(_t4(dx)), ctypes.byref(_t4(dv)), scores.data_ptr(), scores.numel() * scores.element_size(),
-            ws.data_ptr() if ws is not None else None, nb, _stream(dev),
-        )
+        head = (ctypes.byref(_t4(x)), ctypes.byref(_t4(v)), ctypes.byref(_t4(dout)))
+        tail = (fptr, int(rope_start), ctypes.byref(_t4(dx)), ctypes.byref(_t4(dv)), scores.data_ptr(),
+                scores.numel() * scores.element_size(), ws.data_ptr() if ws is not None else None, nb, _stream(dev))
+        if relu_add is None:
+            rc = _lib.bdh_tril_rope_score_v_bwd_saved(*head, *tail)
+        else:
+            rc = _lib.bdh_tril_rope_score_v_bwd_saved_relu(*head, ctypes.byref(_t4(relu_add)), *tail)
     _check(rc, "tril_rope_score_v_bwd_saved")
     return dx, dv
 
@@ -562,14 +577,16 @@ def tril_rope_score_v_bwd(
     freqs: torch.Tensor,
     rope_start: int = 0,
     *,
+    dx: Optional[torch.Tensor] = None,
     dv: Optional[torch.Tensor] = None,
 ) -> Tuple[torch.Tensor, torch.Tensor]:
     """Gradients ``(dx, dv)`` of :func:`tril_rope_score_v` (``dv`` may be passed
     in any float dtype; it defaults to ``v``'s)."""
-    dev = _require_device(x, v, dout, dv)
+    dev = _require_device(x, v, dout, dx, dv)
     B, H, T, N = x.shape
     f, fptr = _freqs_ptr(freqs, N, dev)
-    dx = torch.empty_like(x, memory_format=torch.contiguous_format)
+    if dx is None:
+        dx = torch.empty_like(x, memory_format=torch.contiguous_format)
     if dv is None:
         dv = torch.empty_like(v, memory_format=torch.contiguous_format)
     with torch.cuda.device(dev):
@@ -710,6 +727,40 @@ def gated_decoder(y: torch.Tensor, wt: torch.Tensor, x: torch.Tensor, dec: torch
                                     ctypes.byref(_t4(out.view(B, T, 1, -1))),
                                     ws.data_ptr() if ws is not None else None, nb, _stream(dev))
     _check(rc, "gated_decoder")
+    return out
+
+
+def gated_bwd(y: torch.Tensor, wt: torch.Tensor, x: torch.Tensor, dec: torch.Tensor, dout: torch.Tensor, *,
+              dx: Optional[torch.Tensor] = None,
+              dz: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Backward of ``(x * relu(y @ wt^T)).view(B, T, nh*N) @ dec`` up to its weight products, bf16:
+    y (B, nh, T, K), wt (nh, N, K), x (B, T, nh, N), dec (nh*N, K), dout (B, T, K) ->
+    ``(dx, dz)`` (B, T, nh, N) with dz the gradient of ``y @ wt^T``; both may be passed
+    in (any strides, 16-byte rows)."""
+    dev = _require_device(y, wt, x, dec, dout, dx, dz)
+    if wt.dim() != 3 or dec.dim() != 2 or x.dim() != 4 or dout.dim() != 3:
+        raise ValueError(f"gated_bwd: wt (nh, N, K), dec (nh*N, K), x (B, T, nh, N), dout (B, T, K); got "
+                         f"{tuple(wt.shape)}, {tuple(dec.shape)}, {tuple(x.shape)}, {tuple(dout.shape)}")
+    nh, N, K = wt.shape
+    dx, dz = (torch.empty(x.shape, dtype=x.dtype, device=dev) if t is None else t for t in (dx, dz))
+    with torch.cuda.device(dev):
+        rc = _lib.bdh_gated_bwd(ctypes.byref(_t4(y)), ctypes.byref(_t4(wt.unsqueeze(0))), ctypes.byref(_t4(x)),
+                                ctypes.byref(_t4(dec.view(1, nh, N, K))), ctypes.byref(_t4(dout.unsqueeze(1))),
+                                ctypes.byref(_t4(dx)), ctypes.byref(_t4(dz)), _stream(dev))
+    _check(rc, "gated_bwd")
+    return dx, dz
+
+
+def relu_bwd_add(a: torch.Tensor, b: torch.Tensor, x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``a + b`` where ``x > 0``, else 0: bf16 4-D views of one shape; ``out`` (which may be
+    one of them) defaults to a contiguous tensor."""
+    dev = _require_device(a, b, x, out)
+    if out is None:
+        out = torch.empty(x.shape, dtype=x.dtype, device=dev)
+    with torch.cuda.device(dev):
+        rc = _lib.bdh_relu_bwd_add(ctypes.byref(_t4(a)), ctypes.byref(_t4(b)), ctypes.byref(_t4(x)),
+                                   ctypes.byref(_t4(out)), _stream(dev))
+    _check(rc, "relu_bwd_add")
     return out
 
 

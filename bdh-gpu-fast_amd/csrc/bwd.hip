@@ -340,7 +340,7 @@ size_t rope_saved_bwd_bytes(int64_t B, int64_t H, int64_t T, int64_t N, size_t* 
 
 int rope_saved_bwd(const bdh_tensor4* x, const bdh_tensor4* v, const bdh_tensor4* dout, const bdh_tensor4* dx,
                    const bdh_tensor4* dv, const float* freqs, int64_t rope_start, const void* scores,
-                   size_t scores_bytes, void* ws, size_t ws_bytes, hipStream_t s) {
+                   size_t scores_bytes, void* ws, size_t ws_bytes, hipStream_t s, const bdh_tensor4* add = nullptr) {
   const int64_t B = x->size[0], H = x->size[1], T = x->size[2], N = x->size[3];
   const int64_t D = v->size[3];
   size_t off = 0, kept = 0;
@@ -365,7 +365,7 @@ int rope_saved_bwd(const bdh_tensor4* x, const bdh_tensor4* v, const bdh_tensor4
   if (numel4(dv) > 0) BDH_TRY(step(sy_bwd_dv(x, v, dout, dv, nullptr, 0, s, tiles, rel)));
   if (numel4(dx) == 0) return BDH_OK;
   BDH_TRY(step(sy_bwd_g(dout, v, w + g_off, tpad, s)));
-  return step(sy_dq(w + g_off, tpad, true, x, dx, s, freqs, rope_start, true));
+  return step(sy_dq(w + g_off, tpad, true, x, dx, s, freqs, rope_start, true, add));
 }
 
 bool vec4_rows(const bdh_tensor4* t) {
@@ -710,6 +710,25 @@ extern "C" int bdh_tril_rope_score_v_bwd_saved(const bdh_tensor4* x, const bdh_t
   if (numel4(dx) == 0 && numel4(dv) == 0) return BDH_OK;
   return rope_saved_bwd(x, v, dout, dx, dv, freqs, rope_start, scores, scores_bytes, workspace, workspace_bytes,
                         static_cast<hipStream_t>(stream));
+}
+
+extern "C" int bdh_tril_rope_score_v_bwd_saved_relu(const bdh_tensor4* x, const bdh_tensor4* v,
+                                                    const bdh_tensor4* dout, const bdh_tensor4* add,
+                                                    const float* freqs, int64_t rope_start, const bdh_tensor4* dx,
+                                                    const bdh_tensor4* dv, const void* scores, size_t scores_bytes,
+                                                    void* workspace, size_t workspace_bytes, bdh_stream stream) {
+  BDH_TRY(check_bwd(x, nullptr, v, dout, dx, nullptr, dv));
+  BDH_TRY(check_view(add));
+  if (!same4(add, x)) return BDH_ERR_SHAPE;
+  if (add->dtype != BDH_BF16 || dx->dtype != BDH_BF16) return BDH_ERR_DTYPE;
+  if (views_overlap(dx, add) || views_overlap(dv, add)) return BDH_ERR_ALIAS;
+  if (!rows16b(add)) return BDH_ERR_STRIDE;
+  if (freqs == nullptr && x->size[3] > 0) return BDH_ERR_ARG;
+  if (x->size[3] % 2 != 0) return BDH_ERR_SHAPE;
+  if (rope_start < 0 || rope_start + x->size[2] > (int64_t(1) << 24)) return BDH_ERR_ARG;
+  if (numel4(dx) == 0 && numel4(dv) == 0) return BDH_OK;
+  return rope_saved_bwd(x, v, dout, dx, dv, freqs, rope_start, scores, scores_bytes, workspace, workspace_bytes,
+                        static_cast<hipStream_t>(stream), add);
 }
 
 extern "C" int bdh_tril_rope_score_v_bwd(const bdh_tensor4* x, const bdh_tensor4* v, const bdh_tensor4* dout,

@@ -997,6 +997,8 @@ struct DqsArgs {
   int H, T, N, tpad, nslab, nti, ntn;
   const float* freqs = nullptr;  // RoPE: the output is R^T(G X), positions rope_start + t
   int64_t rope_start = 0;
+  const bf16_t* add = nullptr;  // RADD: the other gradient of x, its strides over (b, h, t)
+  int64_t a0 = 0, a1 = 0, a2 = 0;
 };
 
 __device__ __forceinline__ bf16x4 lds_tr4(const uint8_t* p) {
@@ -1018,9 +1020,15 @@ __device__ __forceinline__ bf16x4 lds_tr4(const lds_u8* p) {
 // barrier that hands the stage to the fragment reads, with the table
 // kernel's (cos, sin) entries and the score kernel's rotation, so the
 // product sees the bits of the R(x) copy the absolute score pass writes.
-template <typename TO, bool ROPE = false, bool ROTB = false, bool KM = false>
+// RADD (with ROTB, bf16): the output is the gradient through the ReLU that
+// made x, (R^T(G X) + add) where x > 0: the sum and the mask are formed on the
+// fp32 values in the epilogue, instead of a pass of its own that reads the
+// product back (three latent-sized reads and a write: 1.14-1.24 ms at 16384
+// tokens, nh N = 32768; the epilogue's two reads add 300 us).
+template <typename TO, bool ROPE = false, bool ROTB = false, bool KM = false, bool RADD = false>
 __global__ __launch_bounds__(kSyThreads, 1) void k_dq_sy(const DqsArgs a) {
   static_assert(!ROTB || ROPE, "B rotation: RoPE output");
+  static_assert(!RADD || (ROTB && sizeof(TO) == 2), "ReLU gradient: X is x, bf16 output");
   const int bid = blockIdx.x;
   const int xcd = bid & 7, kk = bid >> 3;
   const int tiles = a.nti * a.ntn;
@@ -1223,6 +1231,11 @@ __global__ __launch_bounds__(kSyThreads, 1) void k_dq_sy(const DqsArgs a) {
   char* const ob = reinterpret_cast<char*>(o + int64_t(i0 + 128 * wm) * a.o2 + (n0 + 64 * wn));
   const int64_t o2b = a.o2 * int64_t(sizeof(TO));
   const uint32_t lofs = uint32_t(4 * (lane >> 5)) * uint32_t(o2b) + uint32_t((lane & 31) * sizeof(TO));
+  // bf16 with RoPE: lanes l and l ^ 1 hold both columns of a pair, so the even
+  // lane stores the pair of row r and the odd lane that of row r + 1, 4 bytes each
+  constexpr bool PAIR = ROPE && sizeof(TO) == 2;
+  const uint32_t plane = uint32_t(4 * (lane >> 5) + (lane & 1)), pcol = uint32_t(((lane & 31) & ~1) * 2);
+  const uint32_t pofs = plane * uint32_t(o2b) + pcol;
   auto epilogue = [&](auto fullc) __attribute__((always_inline)) {
     constexpr bool FULL = decltype(fullc)::value;
     auto put = [&](int m, int r, float y) __attribute__((always_inline)) {
@@ -1233,6 +1246,22 @@ __global__ __launch_bounds__(kSyThreads, 1) void k_dq_sy(const DqsArgs a) {
         const int row = i0 + 128 * wm + rr_of(m, r) + 4 * (lane >> 5);
         const int col = n0 + 64 * wn + 32 * (m & 1) + (lane & 31);
         if (row < a.T) o[int64_t(row) * a.o2 + col] = from_f<TO>(y);
+      }
+    };
+    // the dword of this lane's column pair in row rr_of(m, r) + (lane & 1) of a view
+    auto pair_at = [&](const bf16_t* base, int64_t s0, int64_t s1, int64_t s2, int m, int r) __attribute__((always_inline)) {
+      const int row = i0 + 128 * wm + rr_of(m, r) + int(plane);
+      const bf16_t* t = base + b * s0 + h * s1 + int64_t(FULL ? row : min(row, a.T - 1)) * s2;
+      return *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(t + n0 + 64 * wn + 32 * (m & 1)) + pcol);
+    };
+    auto put2 = [&](int m, int r, uint32_t v) __attribute__((always_inline)) {
+      if constexpr (FULL) {
+        char* const rp = ob + int64_t(rr_of(m, r)) * o2b + 64 * (m & 1);
+        *reinterpret_cast<uint32_t*>(rp + pofs) = v;
+      } else {
+        const int row = i0 + 128 * wm + rr_of(m, r) + int(plane);
+        if (row < a.T)
+          *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(o + int64_t(row) * a.o2 + n0 + 64 * wn + 32 * (m & 1)) + pcol) = v;
       }
     };
     if constexpr (ROPE) {
@@ -1249,7 +1278,15 @@ __global__ __launch_bounds__(kSyThreads, 1) void k_dq_sy(const DqsArgs a) {
 #pragma unroll
       for (int u = 0; u < 2; ++u) fq[u] = a.freqs[(n0 + 64 * wn + 32 * u + (lane & 31)) & ~1];
 #pragma unroll
-      for (int m = 0; m < 8; ++m)
+      for (int m = 0; m < 8; ++m) {
+        uint32_t ad[8], xm[8];
+        if constexpr (RADD) {
+#pragma unroll
+          for (int r = 0; r < 8; ++r) {
+            ad[r] = pair_at(a.add, a.a0, a.a1, a.a2, m, 2 * r);
+            xm[r] = pair_at(a.x, a.x0, a.x1, a.x2, m, 2 * r);
+          }
+        }
 #pragma unroll
         for (int r = 0; r < 16; r += 2) {
           const int row0 = i0 + 128 * wm + rr_of(m, r) + 4 * (lane >> 5);
@@ -1257,15 +1294,30 @@ __global__ __launch_bounds__(kSyThreads, 1) void k_dq_sy(const DqsArgs a) {
           const uint32_t mine = rope_cs(float(a.rope_start + row0 + (odd ? 1 : 0)), fq[m & 1]);
           const uint32_t theirs = swap1(mine);
           const uint32_t cws[2] = {odd ? theirs : mine, odd ? mine : theirs};
+          float ys[2];
 #pragma unroll
           for (int e = 0; e < 2; ++e) {
             const float v = acc[m][r + e];
             const float pv = __uint_as_float(swap1(__float_as_uint(v)));
             const float c = __uint_as_float(cws[e] << 16), sn = __uint_as_float(cws[e] & 0xffff0000u);
             const float y = odd ? fmaf(v, c, -(pv * sn)) : fmaf(v, c, pv * sn);
-            put(m, r + e, y);
+            if constexpr (PAIR)
+              ys[e] = y;
+            else
+              put(m, r + e, y);
+          }
+          if constexpr (PAIR) {
+            const float got = __uint_as_float(swap1(__float_as_uint(odd ? ys[0] : ys[1])));
+            float lo = odd ? got : ys[0], hi = odd ? ys[1] : got;
+            if constexpr (RADD) {
+              const uint32_t av = ad[r / 2], xv = xm[r / 2];
+              lo = __uint_as_float(xv << 16) <= 0.f ? 0.f : lo + __uint_as_float(av << 16);
+              hi = __uint_as_float(xv & 0xffff0000u) <= 0.f ? 0.f : hi + __uint_as_float(av & 0xffff0000u);
+            }
+            put2(m, r, pack_bf2(lo, hi));
           }
         }
+      }
     } else {
 #pragma unroll
       for (int m = 0; m < 8; ++m)
@@ -2455,7 +2507,9 @@ int sy_past(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v, co
 namespace {
 template <bool KM>
 int launch_dq(const DqsArgs& a, bool bf_out, bool rope, bool rot_b, dim3 gs, hipStream_t s) {
-  if (rope && rot_b) {
+  if (a.add != nullptr) {  // (sy_dq: RoPE, rot_b, bf16 output)
+    BDH_LAUNCH("k_dq_sy", (k_dq_sy<bf16_t, true, true, KM, true>), gs, dim3(kSyThreads), 0, s, a);
+  } else if (rope && rot_b) {
     if (bf_out)
       BDH_LAUNCH("k_dq_sy", (k_dq_sy<bf16_t, true, true, KM>), gs, dim3(kSyThreads), 0, s, a);
     else
@@ -2475,8 +2529,10 @@ int launch_dq(const DqsArgs& a, bool bf_out, bool rope, bool rot_b, dim3 gs, hip
 }  // namespace
 
 int sy_dq(const void* g, int64_t tpad, bool g_sym, const bdh_tensor4* x, const bdh_tensor4* out, hipStream_t s,
-          const float* freqs, int64_t rope_start, bool rot_b) {
+          const float* freqs, int64_t rope_start, bool rot_b, const bdh_tensor4* add) {
   const int64_t B = x->size[0], H = x->size[1], T = x->size[2], N = x->size[3];
+  if (add != nullptr && !(freqs != nullptr && rot_b && out->dtype == BDH_BF16 && add->dtype == BDH_BF16 && rows16(add)))
+    return kNotEligible;
   if (x->dtype != BDH_BF16 || N % kSyTile != 0 || T < 1 || !rows16(x)) return kNotEligible;
   if (out->size[0] != B || out->size[1] != H || out->size[2] != T || out->size[3] != N) return kNotEligible;
   if (tpad % 32 != 0 || tpad * tpad * 2 >= (int64_t(1) << 31)) return kNotEligible;
@@ -2505,6 +2561,12 @@ int sy_dq(const void* g, int64_t tpad, bool g_sym, const bdh_tensor4* x, const b
   a.ntn = int(ntn);
   a.freqs = freqs;
   a.rope_start = rope_start;
+  if (add != nullptr) {
+    a.add = static_cast<const bf16_t*>(add->data);
+    a.a0 = add->stride[0];
+    a.a1 = add->stride[1];
+    a.a2 = add->stride[2];
+  }
   const dim3 gs{unsigned(grid)};
   if (g_sym) return launch_dq<true>(a, out->dtype == BDH_BF16, freqs != nullptr, rot_b, gs, s);
   return launch_dq<false>(a, out->dtype == BDH_BF16, freqs != nullptr, rot_b, gs, s);

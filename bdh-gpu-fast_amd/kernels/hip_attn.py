@@ -134,10 +134,11 @@ def relu_mul(x: torch.Tensor, y: torch.Tensor, out: Optional[torch.Tensor] = Non
     return ext.relu_mul(_last_dim_unit(x), _last_dim_unit(y), out)
 
 
-def gated_gemm(y: torch.Tensor, wt: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
-    """``x * relu(y @ wt^T)`` per head on the GPU (encoder_v GEMM + gated product, bdh.py:914-945)."""
-    ext = _require(y, wt, x)
-    return ext.gated_gemm(y, wt, x)
+def gated_gemm(y: torch.Tensor, wt: torch.Tensor, x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``x * relu(y @ wt^T)`` per head on the GPU (encoder_v GEMM + gated product, bdh.py:914-945);
+    ``out`` may be a strided view (padded rows)."""
+    ext = _require(y, wt, x, out)
+    return ext.gated_gemm(y, wt, x, out)
 
 
 def relu_gemm(y: torch.Tensor, wt: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -154,6 +155,20 @@ def gated_decoder(y: torch.Tensor, wt: torch.Tensor, x: torch.Tensor, dec: torch
     product never stored; fp32 output unless ``out_dtype`` says otherwise."""
     ext = _require(y, wt, x, dec)
     return ext.gated_decoder(y, wt, x, dec, out_dtype)
+
+
+def gated_bwd(y: torch.Tensor, wt: torch.Tensor, x: torch.Tensor, dec: torch.Tensor, dout: torch.Tensor, *,
+              dx: Optional[torch.Tensor] = None, dz: Optional[torch.Tensor] = None):
+    """``(dx, dz)`` of the gated product chained into the decoder (bdh.py:914-945), from
+    the gradient of its output; ``dz`` is the gradient of ``y @ wt^T``."""
+    ext = _require(y, wt, x, dec, dout)
+    return ext.gated_bwd(y, wt, x, dec, dout, dx=dx, dz=dz)
+
+
+def relu_bwd_add(a: torch.Tensor, b: torch.Tensor, x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``a + b`` where ``x > 0``, else 0: the encoder ReLU's gradient from the latent's two uses."""
+    ext = _require(a, b, x, out)
+    return ext.relu_bwd_add(a, b, x, out)
 
 
 def layer_norm_rows(y: torch.Tensor, x: Optional[torch.Tensor] = None,
@@ -230,19 +245,22 @@ def tril_rope_score_v_save(x: torch.Tensor, v: torch.Tensor, freqs: torch.Tensor
     return ext.tril_rope_score_v_save(_last_dim_unit(x), _last_dim_unit(v), freqs, int(rope_start))
 
 
-def tril_rope_score_v_bwd_saved(x, v, dout, freqs, rope_start: int, scores, *, dv=None):
+def tril_rope_score_v_bwd_saved(x, v, dout, freqs, rope_start: int, scores, *, dx=None, dv=None,
+                                relu_add=None):
     """dx and dv of the fused RoPE op from the score tiles saved by
-    :func:`tril_rope_score_v_save`."""
-    ext = _require(x, v, dout, scores)
+    :func:`tril_rope_score_v_save`; with ``relu_add`` dx is ``gradient +
+    relu_add`` where ``x > 0``, else 0."""
+    ext = _require(x, v, dout, scores, relu_add)
     return ext.tril_rope_score_v_bwd_saved(
-        _last_dim_unit(x), _last_dim_unit(v), _last_dim_unit(dout), freqs, int(rope_start), scores, dv=dv
+        _last_dim_unit(x), _last_dim_unit(v), _last_dim_unit(dout), freqs, int(rope_start), scores, dx=dx, dv=dv,
+        relu_add=relu_add
     )
 
 
-def tril_rope_score_v_bwd(x, v, dout, freqs, rope_start: int = 0, *, dv=None):
+def tril_rope_score_v_bwd(x, v, dout, freqs, rope_start: int = 0, *, dx=None, dv=None):
     ext = _require(x, v, dout)
     return ext.tril_rope_score_v_bwd(
-        _last_dim_unit(x), _last_dim_unit(v), _last_dim_unit(dout), freqs, int(rope_start), dv=dv
+        _last_dim_unit(x), _last_dim_unit(v), _last_dim_unit(dout), freqs, int(rope_start), dx=dx, dv=dv
     )
 
 
@@ -284,6 +302,8 @@ __all__ = [
     "relu_mul",
     "gated_gemm",
     "gated_decoder",
+    "gated_bwd",
+    "relu_bwd_add",
     "relu_gemm",
     "small_gemm",
     "tril_rope_score_v",

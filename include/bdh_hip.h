@@ -244,6 +244,17 @@ int bdh_tril_rope_score_v_bwd_saved(const bdh_tensor4* x, const bdh_tensor4* v,
                                     size_t workspace_bytes, bdh_stream stream);
 
 /*
+ * The same with the gradient taken on through the ReLU that made x, when x
+ * has another use with gradient add (bf16, x's shape, 16-byte rows): dx =
+ * (gradient + add) where x > 0, else 0, bf16.  dx may not overlap add.
+ */
+int bdh_tril_rope_score_v_bwd_saved_relu(const bdh_tensor4* x, const bdh_tensor4* v, const bdh_tensor4* dout,
+                                         const bdh_tensor4* add, const float* freqs, int64_t rope_start,
+                                         const bdh_tensor4* dx, const bdh_tensor4* dv, const void* scores,
+                                         size_t scores_bytes, void* workspace, size_t workspace_bytes,
+                                         bdh_stream stream);
+
+/*
  * Consumer of the attention in the BDH layer: out = x * max(y, 0), elementwise.
  * Replaces the ReLU of encoder_v's output (bdh.py:914-925, `_bias_relu_`) and
  * the sparse product of _mlp_merge (bdh.py:927-945, `x_bthn * y_bthn`) in one
@@ -302,6 +313,27 @@ size_t bdh_gated_decoder_workspace(int64_t nh, int64_t M);
 int bdh_gated_decoder(const bdh_tensor4* y, const bdh_tensor4* wt, const bdh_tensor4* x,
                       const bdh_tensor4* dec, const bdh_tensor4* out, void* workspace,
                       size_t workspace_bytes, bdh_stream stream);
+
+/*
+ * Backward of the gated product, all bf16: with s = y wt^T and g = dout dec^T
+ * per head,
+ *   dx = g relu(s),  dz = g x where s > 0 (else 0).
+ * y (B, nh, T, K); wt (1, nh, N, K) encoder_v transposed; x, dx, dz
+ * (B, T, nh, N); dec (1, nh, N, K) the decoder's rows; dout (B, 1, T, K).
+ * K a multiple of 32, N of 8, 16-byte rows; one head's rows of y, wt, dec and
+ * dout within 4 GiB.  The remaining gradients are products of these tensors:
+ * d wt = dz^T y, dy = dz wt, and d dec = (x relu(s))^T dout.
+ */
+int bdh_gated_bwd(const bdh_tensor4* y, const bdh_tensor4* wt, const bdh_tensor4* x, const bdh_tensor4* dec,
+                  const bdh_tensor4* dout, const bdh_tensor4* dx, const bdh_tensor4* dz, bdh_stream stream);
+
+/*
+ * The ReLU gradient of a latent with two uses, bf16, one shape: out = a + b
+ * where x > 0, else 0 (x the ReLU's output).  The last dimension a multiple
+ * of 8, 16-byte rows; out may be one of the inputs itself.
+ */
+int bdh_relu_bwd_add(const bdh_tensor4* a, const bdh_tensor4* b, const bdh_tensor4* x, const bdh_tensor4* out,
+                     bdh_stream stream);
 
 /*
  * Few-row GEMM with split K, bf16 operands, fp32 accumulation:

@@ -1,0 +1,117 @@
+"""The training layer's kernels (csrc/gated_bwd.hip, the ReLU form of the
+saved RoPE backward) against float64, and the fused autograd functions.
+
+Tolerance: bf16 operands are exact in float64; each result is rounded to bf16
+once (2^-9 relative) from fp32 sums, and relu(s) once more inside dx, so 8e-3
+covers two roundings of every element; the compared tensors differ by their
+norm, where roundings average to about 3e-3.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if not torch.cuda.is_available():
+    pytest.skip("needs a ROCm GPU", allow_module_level=True)
+
+import bdh_harness as H  # noqa: E402
+import bdh_hip_ext as ext  # noqa: E402
+import kernels  # noqa: E402
+
+BF = torch.bfloat16
+TOL = 8e-3
+
+
+def _randn(*shape, seed, std=1.0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return (torch.randn(*shape, generator=g, device="cuda") * std).to(BF)
+
+
+def _rel(got, want):
+    return float((got.double() - want).norm() / want.norm().clamp_min(1e-300))
+
+
+# tokens around the 128-row tile, N around the 128-column tile (a multiple of
+# 8), one and several K stages of 32
+@pytest.mark.parametrize("B,T,nh,N,K", [(1, 1, 1, 8, 32), (1, 127, 2, 128, 64), (3, 43, 4, 136, 96), (2, 150, 3, 1000, 256),
+                                        (1, 257, 2, 264, 512)])
+@pytest.mark.parametrize("padded", [False, True])
+def test_gated_backward_matches_float64(B, T, nh, N, K, padded):
+    y, wt = _randn(B, nh, T, K, seed=0), _randn(nh, N, K, seed=1, std=0.05)
+    dec, dout = _randn(nh * N, K, seed=2, std=0.05), _randn(B, T, K, seed=3)
+    x = torch.relu(_randn(B, T, nh, N, seed=4))
+    s = torch.einsum("bhtk,hnk->bthn", y.double(), wt.double())
+    g = torch.einsum("btk,hnk->bthn", dout.double(), dec.double().view(nh, N, K))
+    dx, dz = None, None
+    if padded:  # padded token rows and head-major rows
+        x = H._padded_rows(B, T, nh, N, BF, "cuda").copy_(x)
+        dx = H._padded_rows(B, T, nh, N, BF, "cuda")
+        dz = torch.empty(nh, B, T, N + 8, dtype=BF, device="cuda")[..., :N].permute(1, 2, 0, 3)
+    dx, dz = ext.gated_bwd(y, wt, x, dec, dout, dx=dx, dz=dz)
+    sure = s.abs() > 1e-3  # (the sign of a sum near zero is its rounding's)
+    assert _rel(dx, g * s.clamp_min(0)) <= TOL
+    assert _rel(dz[sure], (g * x.double() * (s > 0))[sure]) <= TOL
+    with pytest.raises(RuntimeError):
+        ext.gated_bwd(y, wt, x, dec, dout, dx=dx, dz=dx)
+
+
+@pytest.mark.parametrize("B,T,nh,N", [(1, 1, 1, 8), (2, 33, 3, 2056), (1, 5, 4, 4096)])
+def test_relu_backward_add_is_exact(B, T, nh, N):
+    a, b = _randn(B, nh, T, N, seed=0).permute(0, 2, 1, 3), _randn(B, T, nh, N, seed=1)
+    x = torch.relu(_randn(B, T, nh, N, seed=2))
+    x[0, 0, 0, 1] = float("nan")
+    want = torch.where(x <= 0, torch.zeros_like(b), a + b)
+    assert torch.equal(ext.relu_bwd_add(a, b, x), want)
+    assert torch.equal(ext.relu_bwd_add(a, b, x, out=b), want)  # in place
+
+
+@pytest.mark.parametrize("B,T,nh,N,D", [(2, 100, 2, 256, 64), (1, 300, 4, 512, 256), (2, 512, 1, 256, 128)])
+def test_saved_backward_through_the_relu(B, T, nh, N, D):
+    """The fused sum and mask equal the separate pass up to its extra rounding."""
+    xt = H._padded_rows(B, T, nh, N, BF, "cuda").copy_(torch.relu(_randn(B, T, nh, N, seed=0, std=0.3)))
+    x, v, do = xt.permute(0, 2, 1, 3), _randn(B, 1, T, D, seed=1), _randn(B, nh, T, D, seed=2)
+    add = _randn(B, T, nh, N, seed=3, std=3.0)
+    freqs = kernels.get_freqs(N).cuda()
+    _, scores = ext.tril_rope_score_v_save(x, v, freqs, 2)
+    assert scores is not None
+    dx, dv = ext.tril_rope_score_v_bwd_saved(x, v, do, freqs, 2, scores)
+    out = H._padded_rows(B, T, nh, N, BF, "cuda")
+    got, dv2 = ext.tril_rope_score_v_bwd_saved(x, v, do, freqs, 2, scores, dx=out.permute(0, 2, 1, 3),
+                                               relu_add=add.permute(0, 2, 1, 3))
+    assert torch.equal(dv, dv2)
+    want = ext.relu_bwd_add(dx.permute(0, 2, 1, 3), add, xt)
+    assert not out[xt <= 0].any()
+    # the separate pass rounds dx to bf16 before the sum: 2^-9 of dx, as the sum's own rounding
+    assert _rel(out, want.double()) <= 4e-3
+
+
+# the fused functions and, with n_embd = 48 (not a multiple of 32), the plain graph
+@pytest.mark.parametrize("D,nh,mult,B,T", [(64, 2, 8, 2, 33), (128, 4, 16, 3, 130), (48, 2, 16, 2, 40)])
+@pytest.mark.parametrize("frozen", [(), ("encoder",), ("encoder_v", "decoder")])
+def test_training_step_gradients_follow_eager_attention(D, nh, mult, B, T, frozen, monkeypatch):
+    """Against the same step on the plain autograd graph (the layer's masks see
+    the same bits): gradients within bf16 rounding of each other."""
+    torch.manual_seed(0)
+    m = H.BDH(H.BDHConfig(n_layer=2, n_embd=D, n_head=nh, mlp_internal_dim_multiplier=mult)).cuda()
+    for n in frozen:
+        getattr(m, n).requires_grad_(False)
+    idx = torch.randint(0, 256, (B, T), device="cuda")
+
+    def grads():
+        m.zero_grad(set_to_none=True)
+        with torch.autocast("cuda", dtype=BF):
+            loss = m(idx, idx.roll(-1, 1), impl="hip")[1]
+        loss.backward()
+        return loss.detach(), {n: p.grad for n, p in m.named_parameters() if p.requires_grad}
+
+    loss, got = grads()
+    monkeypatch.setattr(H, "_trains_fused", lambda *a: False)
+    want_loss, want = grads()
+    assert abs(float(loss - want_loss)) <= 1e-4 * float(want_loss)
+    assert set(got) == set(want)
+    for n, g in want.items():
+        assert got[n].shape == g.shape and got[n].dtype == g.dtype
+        assert _rel(got[n], g.double()) <= 3e-2, n
