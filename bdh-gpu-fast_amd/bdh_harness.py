@@ -328,6 +328,18 @@ def _trains_fused(x: torch.Tensor, encoder: torch.Tensor) -> bool:
             and N * D * 2 < 2**32 and B * T > 0)
 
 
+def _steps_native(x: torch.Tensor, cache, prep: dict) -> bool:
+    """Whether one token after a cached past takes the native step: the packed
+    bf16 cache and bf16 weights, and the limits of the kernels it launches
+    (row LayerNorm, 32-wide K stages, 16-byte rows, q in LDS, 32-bit offsets
+    over one layer's V rows), few enough rows for the split-K decoder."""
+    B, T, D = x.shape
+    N = prep["enc_t"].size(1)
+    return (isinstance(cache, KVCache) and T == 1 and cache.seq_len > 0 and cache.dtype == torch.bfloat16
+            and x.dtype == torch.float32 and prep["enc_t"].dtype == torch.bfloat16 and _ln_rows_ok(x)
+            and N % 8 == 0 and N <= 16320 and 0 < B <= 256 and B * cache.capacity * D * 2 <= 2**32)
+
+
 def _follows(past: torch.Tensor, new: torch.Tensor) -> Optional[torch.Tensor]:
     """past||new as one view when ``new`` is the rows right after ``past`` in the
     same buffer (the reserved slot after the committed rows), else None."""
@@ -483,8 +495,13 @@ class BDH(nn.Module):
         # cache's V slot when the cache stores bf16, so a decode step makes neither a
         # cast nor a slot copy.  The bits are those of x.to(bf16).
         xb = None
+        native = fast and _steps_native(x, cache, prep)
+        if native:
+            cache.slot(0, 1)[1].copy_(x.unsqueeze(1))
+            x = kernels.decode_step(x.view(B, -1), prep["enc_t"], prep["encv_t"], prep["dec"], *cos_sin, cache.kr,
+                                    cache.v, cache.seq_len).view(B, 1, -1)
         v_bf16 = fast and (cache is None or (isinstance(cache, KVCache) and cache.dtype == torch.bfloat16))
-        for level in range(cfg.n_layer):
+        for level in range(0 if native else cfg.n_layer):
             if fused:
                 lat, y_kv = _EncodeAttend.apply(x, self.encoder, enc_t, self.freqs)
                 y_mlp = _GateDecode.apply(lat, _ln(y_kv), self.encoder_v, self.decoder, encv_t, dec)

@@ -17,8 +17,10 @@ is missing or does not export the expected symbols.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
+import struct
 from pathlib import Path
 from typing import Optional, Sequence, Tuple
 
@@ -54,6 +56,7 @@ __all__ = [
     "gated_bwd",
     "relu_bwd_add",
     "small_gemm",
+    "decode_step",
     "layer_norm_rows",
     "profile_enable",
     "profile_collect",
@@ -96,6 +99,8 @@ EXPORTED_SYMBOLS = (
     "bdh_relu_bwd_add",
     "bdh_small_gemm_workspace",
     "bdh_small_gemm",
+    "bdh_decode_step_workspace",
+    "bdh_decode_step",
     "bdh_layer_norm_rows",
     "bdh_layer_norm_rows2",
     "bdh_profile_enable",
@@ -131,9 +136,10 @@ def _load():
     missing = [s for s in EXPORTED_SYMBOLS if not hasattr(lib, s)]
     if missing:
         raise ImportError(f"bdh_hip_ext: {path} lacks symbols {missing}")
-    P = ctypes.POINTER(Tensor4)
+    # descriptors go in as the bytes of a Tensor4 (_t4) or by reference to one
+    P = ctypes.c_void_p
     vp, i32, i64, sz = ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64, ctypes.c_size_t
-    fp = ctypes.POINTER(ctypes.c_float)
+    fp = ctypes.c_void_p
     sig = {
         "bdh_version": (ctypes.c_char_p, []),
         "bdh_error_string": (ctypes.c_char_p, [ctypes.c_int]),
@@ -168,6 +174,8 @@ def _load():
         "bdh_relu_bwd_add": (ctypes.c_int, [P, P, P, P, vp]),
         "bdh_small_gemm_workspace": (sz, [i64, i64, i64]),
         "bdh_small_gemm": (ctypes.c_int, [P, P, P, vp, sz, vp]),
+        "bdh_decode_step_workspace": (sz, [i64, i64, i64, i64, i64]),
+        "bdh_decode_step": (ctypes.c_int, [P, P, P, P, P, P, P, P, i64, P, i64, i32, i64, vp, sz, vp]),
         "bdh_profile_enable": (None, [i32]),
         "bdh_profile_collect": (ctypes.c_int, [ctypes.c_char_p, i32, fp, i32]),
     }
@@ -196,24 +204,28 @@ def launch_count() -> int:
     return _launches
 
 
+_DTYPE_CODES = {torch.float32: BDH_F32, torch.bfloat16: BDH_BF16}
+
+
 def _dtype_code(t: torch.Tensor) -> int:
-    if t.dtype == torch.float32:
-        return BDH_F32
-    if t.dtype == torch.bfloat16:
-        return BDH_BF16
-    raise TypeError(f"bdh_hip_ext supports float32 and bfloat16 tensors, got {t.dtype}")
+    code = _DTYPE_CODES.get(t.dtype)
+    if code is None:
+        raise TypeError(f"bdh_hip_ext supports float32 and bfloat16 tensors, got {t.dtype}")
+    return code
 
 
-def _t4(t: torch.Tensor) -> Tensor4:
-    if t.dim() != 4:
-        raise ValueError(f"bdh_hip_ext expects 4-D tensors, got shape {tuple(t.shape)}")
-    s = Tensor4()
-    s.data = t.data_ptr() if t.numel() > 0 else None
-    for i in range(4):
-        s.size[i] = t.size(i)
-        s.stride[i] = t.stride(i)
-    s.dtype = _dtype_code(t)
-    return s
+# Tensor4's fields as one packed struct: a call's descriptors cost half of what
+# filling ctypes structures member by member did.
+_pack4 = struct.Struct("@P4q4qii").pack
+assert struct.calcsize("@P4q4qii") == ctypes.sizeof(Tensor4)
+
+
+def _t4(t: torch.Tensor) -> bytes:
+    """The Tensor4 of a 4-D tensor, as bytes."""
+    shape = t.shape
+    if len(shape) != 4:
+        raise ValueError(f"bdh_hip_ext expects 4-D tensors, got shape {tuple(shape)}")
+    return _pack4(t.data_ptr() if t.numel() > 0 else 0, *shape, *t.stride(), _dtype_code(t), 0)
 
 
 def _require_device(*ts: Optional[torch.Tensor]) -> torch.device:
@@ -234,8 +246,16 @@ def _require_device(*ts: Optional[torch.Tensor]) -> torch.device:
     return dev
 
 
-def _stream(dev: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+def _stream(dev: torch.device) -> int:
+    return torch._C._cuda_getCurrentRawStream(dev.index)
+
+
+_HERE = contextlib.nullcontext()
+
+
+def _on(dev: torch.device):
+    """``torch.cuda.device(dev)``, skipped when ``dev`` is current already."""
+    return _HERE if torch._C._cuda_getDevice() == dev.index else torch.cuda.device(dev)
 
 
 def _check(rc: int, what: str) -> None:
@@ -260,7 +280,7 @@ def _freqs_ptr(freqs: torch.Tensor, n: int, dev: torch.device):
     if f.device != dev:
         raise RuntimeError(f"freqs on {f.device}, tensors on {dev}")
     f = f.contiguous()
-    return f, ctypes.cast(ctypes.c_void_p(f.data_ptr()), ctypes.POINTER(ctypes.c_float))
+    return f, f.data_ptr()
 
 
 # ------------------------------------------------------------------- forward
@@ -269,11 +289,11 @@ def tril_score_v(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Ten
     dev = _require_device(q, k, v)
     B, H, T, Dk = q.shape
     out = torch.empty(B, H, T, v.size(-1), dtype=q.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         need = _lib.bdh_tril_score_v_workspace(B, H, T, Dk, v.size(-1), _dtype_code(q))
         ws, nb = _workspace(need, dev)
         rc = _lib.bdh_tril_score_v(
-            ctypes.byref(_t4(q)), ctypes.byref(_t4(k)), ctypes.byref(_t4(v)), ctypes.byref(_t4(out)),
+            _t4(q), _t4(k), _t4(v), _t4(out),
             ws.data_ptr() if ws is not None else None, nb, _stream(dev),
         )
     _check(rc, "tril_score_v")
@@ -293,11 +313,11 @@ def tril_score_v_past(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, past: i
     B, H, T, Dk = q.shape
     past = int(past)
     out = torch.empty(B, H, T, v.size(-1), dtype=q.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         need = _lib.bdh_tril_score_v_past_workspace(B, H, T, past, Dk, v.size(-1), _dtype_code(q))
         ws, nb = _workspace(need, dev)
         rc = _lib.bdh_tril_score_v_past(
-            ctypes.byref(_t4(q)), ctypes.byref(_t4(k)), ctypes.byref(_t4(v)), ctypes.byref(_t4(out)),
+            _t4(q), _t4(k), _t4(v), _t4(out),
             past, ws.data_ptr() if ws is not None else None, nb, _stream(dev),
         )
     _check(rc, "tril_score_v_past")
@@ -308,7 +328,7 @@ def keeps_scores(x: torch.Tensor, v: torch.Tensor) -> bool:
     """Whether ``tril_score_v(x, x, v)`` leaves reusable score tiles in its workspace."""
     if not (x.is_cuda and v.is_cuda) or x.dim() != 4 or v.dim() != 4:
         return False
-    return bool(_lib.bdh_tril_score_v_keeps_scores(ctypes.byref(_t4(x)), ctypes.byref(_t4(v)), None))
+    return bool(_lib.bdh_tril_score_v_keeps_scores(_t4(x), _t4(v), None))
 
 
 def tril_score_v_save(x: torch.Tensor, v: torch.Tensor) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
@@ -318,11 +338,11 @@ def tril_score_v_save(x: torch.Tensor, v: torch.Tensor) -> Tuple[torch.Tensor, O
     dev = _require_device(x, v)
     B, H, T, N = x.shape
     out = torch.empty(B, H, T, v.size(-1), dtype=x.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         need = _lib.bdh_tril_score_v_workspace(B, H, T, N, v.size(-1), _dtype_code(x))
         ws, nb = _workspace(need, dev)
         rc = _lib.bdh_tril_score_v(
-            ctypes.byref(_t4(x)), ctypes.byref(_t4(x)), ctypes.byref(_t4(v)), ctypes.byref(_t4(out)),
+            _t4(x), _t4(x), _t4(v), _t4(out),
             ws.data_ptr() if ws is not None else None, nb, _stream(dev),
         )
     _check(rc, "tril_score_v")
@@ -348,12 +368,12 @@ def tril_rope_score_v(
     f, fptr = _freqs_ptr(freqs, N, dev)
     if out is None:
         out = torch.empty(B, H, T, v.size(-1), dtype=x.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         need = _lib.bdh_tril_score_v_workspace(B, H, T, N, v.size(-1), _dtype_code(x))
         ws, nb = _workspace(need, dev)
         rc = _lib.bdh_tril_rope_score_v(
-            ctypes.byref(_t4(x)), ctypes.byref(_t4(v)), ctypes.byref(_t4(out)), fptr, int(rope_start),
-            ctypes.byref(_t4(qr_out)) if qr_out is not None else None,
+            _t4(x), _t4(v), _t4(out), fptr, int(rope_start),
+            _t4(qr_out) if qr_out is not None else None,
             ws.data_ptr() if ws is not None else None, nb, _stream(dev),
         )
     _check(rc, "tril_rope_score_v")
@@ -365,7 +385,7 @@ def rope_keeps_scores(x: torch.Tensor, v: torch.Tensor) -> bool:
     score tiles in its workspace."""
     if not (x.is_cuda and v.is_cuda) or x.dim() != 4 or v.dim() != 4:
         return False
-    return bool(_lib.bdh_tril_rope_score_v_keeps_scores(ctypes.byref(_t4(x)), ctypes.byref(_t4(v)), None))
+    return bool(_lib.bdh_tril_rope_score_v_keeps_scores(_t4(x), _t4(v), None))
 
 
 def tril_rope_score_v_save(
@@ -378,11 +398,11 @@ def tril_rope_score_v_save(
     B, H, T, N = x.shape
     f, fptr = _freqs_ptr(freqs, N, dev)
     out = torch.empty(B, H, T, v.size(-1), dtype=x.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         need = _lib.bdh_tril_score_v_workspace(B, H, T, N, v.size(-1), _dtype_code(x))
         ws, nb = _workspace(need, dev)
         rc = _lib.bdh_tril_rope_score_v(
-            ctypes.byref(_t4(x)), ctypes.byref(_t4(v)), ctypes.byref(_t4(out)), fptr, int(rope_start), None,
+            _t4(x), _t4(v), _t4(out), fptr, int(rope_start), None,
             ws.data_ptr() if ws is not None else None, nb, _stream(dev),
         )
     _check(rc, "tril_rope_score_v")
@@ -413,16 +433,16 @@ def tril_rope_score_v_bwd_saved(
         dx = torch.empty_like(x, memory_format=torch.contiguous_format)
     if dv is None:
         dv = torch.empty_like(v, memory_format=torch.contiguous_format)
-    with torch.cuda.device(dev):
+    with _on(dev):
         need = _lib.bdh_tril_rope_score_v_bwd_saved_workspace(B, H, v.size(1), T, N, v.size(-1), _dtype_code(x))
         ws, nb = _workspace(need, dev)
-        head = (ctypes.byref(_t4(x)), ctypes.byref(_t4(v)), ctypes.byref(_t4(dout)))
-        tail = (fptr, int(rope_start), ctypes.byref(_t4(dx)), ctypes.byref(_t4(dv)), scores.data_ptr(),
+        head = (_t4(x), _t4(v), _t4(dout))
+        tail = (fptr, int(rope_start), _t4(dx), _t4(dv), scores.data_ptr(),
                 scores.numel() * scores.element_size(), ws.data_ptr() if ws is not None else None, nb, _stream(dev))
         if relu_add is None:
             rc = _lib.bdh_tril_rope_score_v_bwd_saved(*head, *tail)
         else:
-            rc = _lib.bdh_tril_rope_score_v_bwd_saved_relu(*head, ctypes.byref(_t4(relu_add)), *tail)
+            rc = _lib.bdh_tril_rope_score_v_bwd_saved_relu(*head, _t4(relu_add), *tail)
     _check(rc, "tril_rope_score_v_bwd_saved")
     return dx, dv
 
@@ -468,11 +488,11 @@ def tril_decode(q: torch.Tensor, k_past: torch.Tensor, v_past: torch.Tensor) -> 
     S = k_past.size(2)
     Dv = v_past.size(-1)
     out = torch.empty(B, H, Tq, Dv, dtype=q.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         need = _lib.bdh_tril_decode_workspace(B, H, Tq, S, Dk, Dv)
         ws, nb = _workspace(need, dev)
         rc = _lib.bdh_tril_decode(
-            ctypes.byref(_t4(q)), ctypes.byref(_t4(k_past)), ctypes.byref(_t4(v_past)), ctypes.byref(_t4(out)),
+            _t4(q), _t4(k_past), _t4(v_past), _t4(out),
             ws.data_ptr() if ws is not None else None, nb, _stream(dev),
         )
     _check(rc, "tril_decode")
@@ -493,9 +513,9 @@ def tril_decode_noalloc(
     B, H, Tq, _ = q.shape
     if out is None:
         out = torch.empty(B, H, Tq, v_past.size(-1), dtype=q.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.bdh_tril_decode_noalloc(
-            ctypes.byref(_t4(q)), ctypes.byref(_t4(k_past)), ctypes.byref(_t4(v_past)), ctypes.byref(_t4(out)),
+            _t4(q), _t4(k_past), _t4(v_past), _t4(out),
             _stream(dev),
         )
     _check(rc, "tril_decode_noalloc")
@@ -529,13 +549,13 @@ def tril_score_v_bwd(
         dk = None
     if dv is None:
         dv = torch.empty_like(v, memory_format=torch.contiguous_format)
-    with torch.cuda.device(dev):
+    with _on(dev):
         need = _lib.bdh_tril_score_v_bwd_workspace(B, H, v.size(1), T, N, v.size(-1), _dtype_code(q))
         ws, nb = _workspace(need, dev)
         rc = _lib.bdh_tril_score_v_bwd(
-            ctypes.byref(_t4(q)), ctypes.byref(_t4(k)) if k is not None else None, ctypes.byref(_t4(v)),
-            ctypes.byref(_t4(dout)), ctypes.byref(_t4(dq)), ctypes.byref(_t4(dk)) if dk is not None else None,
-            ctypes.byref(_t4(dv)), ws.data_ptr() if ws is not None else None, nb, _stream(dev),
+            _t4(q), _t4(k) if k is not None else None, _t4(v),
+            _t4(dout), _t4(dq), _t4(dk) if dk is not None else None,
+            _t4(dv), ws.data_ptr() if ws is not None else None, nb, _stream(dev),
         )
     _check(rc, "tril_score_v_bwd")
     return dq, dk, dv
@@ -558,12 +578,12 @@ def tril_score_v_bwd_saved(
         dx = torch.empty_like(x, memory_format=torch.contiguous_format)
     if dv is None:
         dv = torch.empty_like(v, memory_format=torch.contiguous_format)
-    with torch.cuda.device(dev):
+    with _on(dev):
         need = _lib.bdh_tril_score_v_bwd_saved_workspace(B, H, v.size(1), T, N, v.size(-1), _dtype_code(x))
         ws, nb = _workspace(need, dev)
         rc = _lib.bdh_tril_score_v_bwd_saved(
-            ctypes.byref(_t4(x)), ctypes.byref(_t4(v)), ctypes.byref(_t4(dout)), ctypes.byref(_t4(dx)),
-            ctypes.byref(_t4(dv)), scores.data_ptr(), scores.numel() * scores.element_size(),
+            _t4(x), _t4(v), _t4(dout), _t4(dx),
+            _t4(dv), scores.data_ptr(), scores.numel() * scores.element_size(),
             ws.data_ptr() if ws is not None else None, nb, _stream(dev),
         )
     _check(rc, "tril_score_v_bwd_saved")
@@ -589,12 +609,12 @@ def tril_rope_score_v_bwd(
         dx = torch.empty_like(x, memory_format=torch.contiguous_format)
     if dv is None:
         dv = torch.empty_like(v, memory_format=torch.contiguous_format)
-    with torch.cuda.device(dev):
+    with _on(dev):
         need = _lib.bdh_tril_rope_score_v_bwd_workspace(B, H, v.size(1), T, N, v.size(-1), _dtype_code(x))
         ws, nb = _workspace(need, dev)
         rc = _lib.bdh_tril_rope_score_v_bwd(
-            ctypes.byref(_t4(x)), ctypes.byref(_t4(v)), ctypes.byref(_t4(dout)), fptr, int(rope_start),
-            ctypes.byref(_t4(dx)), ctypes.byref(_t4(dv)), ws.data_ptr() if ws is not None else None, nb,
+            _t4(x), _t4(v), _t4(dout), fptr, int(rope_start),
+            _t4(dx), _t4(dv), ws.data_ptr() if ws is not None else None, nb,
             _stream(dev),
         )
     _check(rc, "tril_rope_score_v_bwd")
@@ -626,9 +646,9 @@ def rope_rotate(
     if out is None:
         out = torch.empty(shape, dtype=v.dtype, device=dev)
     o4 = out.view(pad + shape) if pad else out
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.bdh_rope_rotate(
-            ctypes.byref(_t4(v4)), ctypes.byref(_t4(c4)), ctypes.byref(_t4(s4)), ctypes.byref(_t4(o4)),
+            _t4(v4), _t4(c4), _t4(s4), _t4(o4),
             1 if backward else 0, _stream(dev),
         )
     _check(rc, "rope_rotate")
@@ -644,8 +664,8 @@ def relu_mul(x: torch.Tensor, y: torch.Tensor, out: Optional[torch.Tensor] = Non
         raise ValueError(f"relu_mul: x and y must be 4-D of one shape, got {tuple(x.shape)} and {tuple(y.shape)}")
     if out is None:
         out = torch.empty(x.shape, dtype=x.dtype, device=dev)
-    with torch.cuda.device(dev):
-        rc = _lib.bdh_relu_mul(ctypes.byref(_t4(x)), ctypes.byref(_t4(y)), ctypes.byref(_t4(out)), _stream(dev))
+    with _on(dev):
+        rc = _lib.bdh_relu_mul(_t4(x), _t4(y), _t4(out), _stream(dev))
     _check(rc, "relu_mul")
     return out
 
@@ -665,16 +685,16 @@ def layer_norm_rows(y: torch.Tensor, x: Optional[torch.Tensor] = None, out_dtype
     def v4(t: torch.Tensor) -> torch.Tensor:
         return t.reshape((1,) * (4 - t.dim()) + tuple(t.shape)) if t.dim() < 4 else t
 
-    with torch.cuda.device(dev):
+    with _on(dev):
         if out_bf16 is None:
-            rc = _lib.bdh_layer_norm_rows(ctypes.byref(_t4(v4(x))) if x is not None else None,
-                                          ctypes.byref(_t4(v4(y))), ctypes.byref(_t4(v4(out))), _stream(dev))
+            rc = _lib.bdh_layer_norm_rows(_t4(v4(x)) if x is not None else None,
+                                          _t4(v4(y)), _t4(v4(out)), _stream(dev))
         else:
             if out_bf16.shape != y.shape:
                 raise ValueError(f"layer_norm_rows: out_bf16 {tuple(out_bf16.shape)} and y {tuple(y.shape)} differ")
-            rc = _lib.bdh_layer_norm_rows2(ctypes.byref(_t4(v4(x))) if x is not None else None,
-                                           ctypes.byref(_t4(v4(y))), ctypes.byref(_t4(v4(out))),
-                                           ctypes.byref(_t4(v4(out_bf16))), _stream(dev))
+            rc = _lib.bdh_layer_norm_rows2(_t4(v4(x)) if x is not None else None,
+                                           _t4(v4(y)), _t4(v4(out)),
+                                           _t4(v4(out_bf16)), _stream(dev))
     _check(rc, "layer_norm_rows")
     return out
 
@@ -686,9 +706,9 @@ def gated_gemm(y: torch.Tensor, wt: torch.Tensor, x: torch.Tensor, out: Optional
         raise ValueError(f"gated_gemm: wt must be (nh, N, K), got {tuple(wt.shape)}")
     if out is None:
         out = torch.empty(x.shape, dtype=x.dtype, device=dev)
-    with torch.cuda.device(dev):
-        rc = _lib.bdh_gated_gemm(ctypes.byref(_t4(y)), ctypes.byref(_t4(wt.unsqueeze(0))), ctypes.byref(_t4(x)),
-                                 ctypes.byref(_t4(out)), _stream(dev))
+    with _on(dev):
+        rc = _lib.bdh_gated_gemm(_t4(y), _t4(wt.unsqueeze(0)), _t4(x),
+                                 _t4(out), _stream(dev))
     _check(rc, "gated_gemm")
     return out
 
@@ -702,8 +722,8 @@ def relu_gemm(y: torch.Tensor, wt: torch.Tensor, out: Optional[torch.Tensor] = N
     B, nh, T, _ = y.shape
     if out is None:
         out = torch.empty(B, T, nh, wt.size(1), dtype=y.dtype, device=dev)
-    with torch.cuda.device(dev):
-        rc = _lib.bdh_relu_gemm(ctypes.byref(_t4(y)), ctypes.byref(_t4(wt.unsqueeze(0))), ctypes.byref(_t4(out)),
+    with _on(dev):
+        rc = _lib.bdh_relu_gemm(_t4(y), _t4(wt.unsqueeze(0)), _t4(out),
                                 _stream(dev))
     _check(rc, "relu_gemm")
     return out
@@ -720,11 +740,11 @@ def gated_decoder(y: torch.Tensor, wt: torch.Tensor, x: torch.Tensor, dec: torch
                          f"{tuple(wt.shape)}, {tuple(dec.shape)}, {tuple(x.shape)}")
     B, T, nh, N = x.shape
     out = torch.empty(B, T, dec.size(1), dtype=out_dtype or torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ws, nb = _workspace(_lib.bdh_gated_decoder_workspace(nh, B * T), dev)
-        rc = _lib.bdh_gated_decoder(ctypes.byref(_t4(y)), ctypes.byref(_t4(wt.unsqueeze(0))), ctypes.byref(_t4(x)),
-                                    ctypes.byref(_t4(dec.view(1, 1, *dec.shape))),
-                                    ctypes.byref(_t4(out.view(B, T, 1, -1))),
+        rc = _lib.bdh_gated_decoder(_t4(y), _t4(wt.unsqueeze(0)), _t4(x),
+                                    _t4(dec.view(1, 1, *dec.shape)),
+                                    _t4(out.view(B, T, 1, -1)),
                                     ws.data_ptr() if ws is not None else None, nb, _stream(dev))
     _check(rc, "gated_decoder")
     return out
@@ -743,10 +763,10 @@ def gated_bwd(y: torch.Tensor, wt: torch.Tensor, x: torch.Tensor, dec: torch.Ten
                          f"{tuple(wt.shape)}, {tuple(dec.shape)}, {tuple(x.shape)}, {tuple(dout.shape)}")
     nh, N, K = wt.shape
     dx, dz = (torch.empty(x.shape, dtype=x.dtype, device=dev) if t is None else t for t in (dx, dz))
-    with torch.cuda.device(dev):
-        rc = _lib.bdh_gated_bwd(ctypes.byref(_t4(y)), ctypes.byref(_t4(wt.unsqueeze(0))), ctypes.byref(_t4(x)),
-                                ctypes.byref(_t4(dec.view(1, nh, N, K))), ctypes.byref(_t4(dout.unsqueeze(1))),
-                                ctypes.byref(_t4(dx)), ctypes.byref(_t4(dz)), _stream(dev))
+    with _on(dev):
+        rc = _lib.bdh_gated_bwd(_t4(y), _t4(wt.unsqueeze(0)), _t4(x),
+                                _t4(dec.view(1, nh, N, K)), _t4(dout.unsqueeze(1)),
+                                _t4(dx), _t4(dz), _stream(dev))
     _check(rc, "gated_bwd")
     return dx, dz
 
@@ -757,9 +777,9 @@ def relu_bwd_add(a: torch.Tensor, b: torch.Tensor, x: torch.Tensor, out: Optiona
     dev = _require_device(a, b, x, out)
     if out is None:
         out = torch.empty(x.shape, dtype=x.dtype, device=dev)
-    with torch.cuda.device(dev):
-        rc = _lib.bdh_relu_bwd_add(ctypes.byref(_t4(a)), ctypes.byref(_t4(b)), ctypes.byref(_t4(x)),
-                                   ctypes.byref(_t4(out)), _stream(dev))
+    with _on(dev):
+        rc = _lib.bdh_relu_bwd_add(_t4(a), _t4(b), _t4(x),
+                                   _t4(out), _stream(dev))
     _check(rc, "relu_bwd_add")
     return out
 
@@ -772,12 +792,32 @@ def small_gemm(a: torch.Tensor, b: torch.Tensor, out_dtype: Optional[torch.dtype
     M, K = a.shape
     D = b.size(1)
     out = torch.empty(M, D, dtype=out_dtype or a.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         ws, nb = _workspace(_lib.bdh_small_gemm_workspace(M, K, D), dev)
-        rc = _lib.bdh_small_gemm(ctypes.byref(_t4(a.view(1, 1, M, K))), ctypes.byref(_t4(b.view(1, 1, K, D))),
-                                 ctypes.byref(_t4(out.view(1, 1, M, D))),
+        rc = _lib.bdh_small_gemm(_t4(a.view(1, 1, M, K)), _t4(b.view(1, 1, K, D)),
+                                 _t4(out.view(1, 1, M, D)),
                                  ws.data_ptr() if ws is not None else None, nb, _stream(dev))
     _check(rc, "small_gemm")
+    return out
+
+
+def decode_step(x: torch.Tensor, enc_t: torch.Tensor, encv_t: torch.Tensor, dec: torch.Tensor, cos: torch.Tensor,
+                sin: torch.Tensor, kr: torch.Tensor, v: torch.Tensor, seq_len: int) -> torch.Tensor:
+    """All layers of one generate step: x (B, D) fp32 the token's embedding, already in
+    layer 0's V slot as bf16; enc_t and encv_t (nh, N, D), dec (nh*N, D) bf16; cos, sin (1, 1, 1, N);
+    kr (L, B, nh, cap, N) and v (L, B, 1, cap, D) the bf16 cache with ``seq_len`` rows.
+    Returns the last layer's x (B, D); the rows at ``seq_len`` are written."""
+    dev = _require_device(x, enc_t, encv_t, dec, cos, sin, kr, v)
+    B, D = x.shape
+    nh, N, _ = enc_t.shape
+    out = torch.empty(B, D, dtype=torch.float32, device=dev)
+    with _on(dev):
+        ws, nb = _workspace(_lib.bdh_decode_step_workspace(B, nh, N, D, seq_len), dev)
+        rc = _lib.bdh_decode_step(_t4(x.view(1, 1, B, D)), _t4(out.view(1, 1, B, D)), _t4(enc_t.unsqueeze(0)),
+                                  _t4(encv_t.unsqueeze(0)), _t4(dec.view(1, 1, nh * N, D)), _t4(cos), _t4(sin),
+                                  _t4(kr[0]), kr.stride(0), _t4(v[0]), v.stride(0), kr.size(0), int(seq_len),
+                                  ws.data_ptr() if ws is not None else None, nb, _stream(dev))
+    _check(rc, "decode_step")
     return out
 
 

@@ -186,6 +186,13 @@ def small_gemm(a: torch.Tensor, b: torch.Tensor, out_dtype: Optional[torch.dtype
     return ext.small_gemm(a, b, out_dtype)
 
 
+def decode_step(x, enc_t, encv_t, dec, cos, sin, kr, v, seq_len: int) -> torch.Tensor:
+    """All layers of one generate step over the packed bf16 cache in one native call
+    (bdh.py:992-1052 for one token); returns the last layer's x (B, D)."""
+    ext = _require(x, enc_t, encv_t, dec, cos, sin, kr, v)
+    return ext.decode_step(x, enc_t, encv_t, dec, cos, sin, kr, v, seq_len)
+
+
 def tril_rope_score_v(
     x: torch.Tensor,
     v: torch.Tensor,
@@ -306,6 +313,7 @@ __all__ = [
     "relu_bwd_add",
     "relu_gemm",
     "small_gemm",
+    "decode_step",
     "tril_rope_score_v",
     "tril_decode",
     "tril_score_v_bwd",

@@ -374,6 +374,26 @@ int bdh_layer_norm_rows2(const bdh_tensor4* x, const bdh_tensor4* y,
                          bdh_stream stream);
 
 /*
+ * One generate step of every layer in one call (the launches of the entries
+ * above, in the order of the model's cached forward): for l = 0 .. n_layer-1
+ *   lat = relu(row_l enc_t^T), KR slot = RoPE(lat), y = decode(KR slot, past),
+ *   x <- LN(x + LN((lat * relu(LN(y) encv_t^T)) dec)),
+ * where row_l is the bf16 row at seq_len of layer l's V: the caller writes
+ * layer 0's (x rounded), the call the others.  x, out (1, 1, B, D) fp32; enc_t,
+ * encv_t (1, nh, N, D), dec (1, 1, nh*N, D) bf16; cos, sin (1, 1, 1, N); kr
+ * (B, nh, cap, N) and v (B, 1, cap, D) bf16, layer 0 of n_layer that lie
+ * kr_layer and v_layer elements apart, rows [0, seq_len) filled, seq_len >= 1.
+ * The shapes are those of the entries it calls (D = 64 * 2^k <= 1024, N <=
+ * 16320 a multiple of 8).
+ */
+size_t bdh_decode_step_workspace(int64_t B, int64_t nh, int64_t N, int64_t D, int64_t seq_len);
+int bdh_decode_step(const bdh_tensor4* x, const bdh_tensor4* out, const bdh_tensor4* enc_t,
+                    const bdh_tensor4* encv_t, const bdh_tensor4* dec, const bdh_tensor4* cos,
+                    const bdh_tensor4* sin, const bdh_tensor4* kr, int64_t kr_layer, const bdh_tensor4* v,
+                    int64_t v_layer, int32_t n_layer, int64_t seq_len, void* workspace, size_t workspace_bytes,
+                    bdh_stream stream);
+
+/*
  * Per-kernel timing (measurement support; no counterpart in the reference).
  * While enabled, every kernel the library launches is bracketed by HIP events
  * on its stream.  bdh_profile_collect() waits for the recorded events and
