@@ -406,7 +406,12 @@ def tril_rope_score_v_save(
             ws.data_ptr() if ws is not None else None, nb, _stream(dev),
         )
     _check(rc, "tril_rope_score_v")
-    return out, (ws if rope_keeps_scores(x, v) else None)
+    kept = ctypes.c_size_t()
+    if ws is None or not _lib.bdh_tril_rope_score_v_keeps_scores(_t4(x), _t4(v), ctypes.byref(kept)):
+        return out, None
+    # fp32: the sum of the splits is the first split's part of the workspace;
+    # only that much is kept
+    return out, (ws[:kept.value].clone() if x.dtype == torch.float32 and 2 * kept.value <= nb else ws)
 
 
 def tril_rope_score_v_bwd_saved(

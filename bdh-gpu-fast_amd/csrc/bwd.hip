@@ -259,17 +259,18 @@ BwdPlan plan_bwd(int64_t B, int64_t H, int64_t T, int64_t K, bool saved = false,
   return p;
 }
 
-// fp32: [score tiles | dV pieces | G].
+// fp32: [score tiles | dV pieces | G]; saved: the tiles come from the forward.
 struct F32BwdPlan {
   F32Plan f;
   int64_t tpad;
   size_t dv_off, g_off, ws_bytes;
 };
-F32BwdPlan plan_f32_bwd(int64_t B, int64_t H, int64_t Hv, int64_t T, int64_t K, int64_t Dv, bool self) {
+F32BwdPlan plan_f32_bwd(int64_t B, int64_t H, int64_t Hv, int64_t T, int64_t K, int64_t Dv, bool self,
+                        bool saved = false) {
   F32BwdPlan p;
   p.f = plan_f32(B, H, T, K, self);
   p.tpad = (T + kTile - 1) / kTile * kTile;
-  p.dv_off = align_up(p.f.m_bytes, 256);
+  p.dv_off = saved ? 0 : align_up(p.f.m_bytes, 256);
   p.g_off = align_up(p.dv_off + f32_dv_bytes(B, H, Hv, T, Dv), 256);
   p.ws_bytes = p.g_off + size_t(B * H) * size_t(p.tpad) * size_t(p.tpad) * 4;
   return p;
@@ -452,13 +453,13 @@ int check_bwd(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v, 
   return BDH_OK;
 }
 
-// fp32 operands (f32.hip).
+// fp32 operands (f32.hip).  saved: the forward's score tiles.
 int run_f32_bwd(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v, const bdh_tensor4* dout,
                 const bdh_tensor4* dq, const bdh_tensor4* dk, const bdh_tensor4* dv, const float* freqs,
-                int64_t rope_start, void* ws, size_t ws_bytes, hipStream_t s) {
+                int64_t rope_start, void* ws, size_t ws_bytes, hipStream_t s, const float* saved = nullptr) {
   const int64_t B = q->size[0], H = q->size[1], T = q->size[2], N = q->size[3];
   const bool self = k == nullptr;
-  const F32BwdPlan p = plan_f32_bwd(B, H, v->size[1], T, N, v->size[3], self);
+  const F32BwdPlan p = plan_f32_bwd(B, H, v->size[1], T, N, v->size[3], self, saved != nullptr);
   if (ws == nullptr || ws_bytes < p.ws_bytes) return BDH_ERR_WORKSPACE;
   char* w = static_cast<char*>(ws);
   float* g = reinterpret_cast<float*>(w + p.g_off);
@@ -479,8 +480,8 @@ int run_f32_bwd(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v
     sa.sp = reinterpret_cast<float*>(w);
     sa.qr.p = nullptr;
     sa.qr_bf = false;
-    BDH_TRY(f32_scores(sa, p.f, B * H, s));
-    BDH_TRY(f32_dv(sa.sp, p.f, dout, dv, reinterpret_cast<float*>(w + p.dv_off), s));
+    if (saved == nullptr) BDH_TRY(f32_scores(sa, p.f, B * H, s));
+    BDH_TRY(f32_dv(saved != nullptr ? saved : sa.sp, p.f, dout, dv, reinterpret_cast<float*>(w + p.dv_off), s));
   }
   if (numel4(dq) == 0) return BDH_OK;
   BDH_TRY(f32_g(dout, v, g, p.tpad, s));
@@ -675,6 +676,12 @@ extern "C" size_t bdh_tril_rope_score_v_bwd_workspace(int64_t B, int64_t H, int6
 extern "C" int bdh_tril_rope_score_v_keeps_scores(const bdh_tensor4* x, const bdh_tensor4* v, size_t* scores_bytes) {
   size_t off = 0, kept = 0;
   int rel = 0;
+  if (check_view(x) == BDH_OK && check_view(v) == BDH_OK && x->dtype == BDH_F32 && v->size[0] == x->size[0] &&
+      v->size[2] == x->size[2] && (v->size[1] == 1 || v->size[1] == x->size[1]) && x->size[3] % 2 == 0) {
+    // fp32: every shape of the forward, the summed tiles at the start
+    if (scores_bytes) *scores_bytes = plan_f32(x->size[0], x->size[1], x->size[2], x->size[3], true).tile_bytes;
+    return 1;
+  }
   // the limits rope_saved_bwd applies to what the forward already knows (G's
   // padded T x T tile and V's row span), so tiles are kept only when the
   // saved backward will take them; dO is passed with contiguous rows
@@ -693,9 +700,7 @@ extern "C" int bdh_tril_rope_score_v_keeps_scores(const bdh_tensor4* x, const bd
 
 extern "C" size_t bdh_tril_rope_score_v_bwd_saved_workspace(int64_t B, int64_t H, int64_t Hv, int64_t T,
                                                             int64_t N, int64_t Dv, int32_t x_dtype) {
-  (void)Hv;
-  (void)Dv;
-  if (x_dtype != BDH_BF16) return 0;
+  if (x_dtype != BDH_BF16) return plan_f32_bwd(B, H, Hv, T, N, Dv, true, true).ws_bytes;
   return rope_saved_bwd_bytes(B, H, T, N, nullptr, nullptr);
 }
 
@@ -708,6 +713,13 @@ extern "C" int bdh_tril_rope_score_v_bwd_saved(const bdh_tensor4* x, const bdh_t
   if (x->size[3] % 2 != 0) return BDH_ERR_SHAPE;
   if (rope_start < 0 || rope_start + x->size[2] > (int64_t(1) << 24)) return BDH_ERR_ARG;
   if (numel4(dx) == 0 && numel4(dv) == 0) return BDH_OK;
+  if (x->dtype == BDH_F32) {
+    if (scores == nullptr || (reinterpret_cast<uintptr_t>(scores) & 15) != 0) return BDH_ERR_ARG;
+    if (scores_bytes < plan_f32(x->size[0], x->size[1], x->size[2], x->size[3], true).tile_bytes)
+      return BDH_ERR_WORKSPACE;
+    return run_f32_bwd(x, nullptr, v, dout, dx, nullptr, dv, freqs, rope_start, workspace, workspace_bytes,
+                       static_cast<hipStream_t>(stream), static_cast<const float*>(scores));
+  }
   return rope_saved_bwd(x, v, dout, dx, dv, freqs, rope_start, scores, scores_bytes, workspace, workspace_bytes,
                         static_cast<hipStream_t>(stream));
 }

@@ -143,8 +143,8 @@ class TrilRopeSelfAttnFn(torch.autograd.Function):
 
     The backward returns dx (RoPE^T of the merged dQR) and dV; ``freqs`` is a
     constant buffer (no gradient), like the reference's detached cos/sin.
-    Without ``qr_out`` the forward's bf16 score tiles are kept for the
-    backward when the shapes allow it (``BDH_ATTN_SAVE_SCORES=0`` turns this
+    Without ``qr_out`` the forward's score tiles (bf16, or fp32 for fp32 x)
+    are kept for the backward when the shapes allow it (``BDH_ATTN_SAVE_SCORES=0`` turns this
     off), so the backward recomputes none of them.
     """
 
@@ -153,7 +153,7 @@ class TrilRopeSelfAttnFn(torch.autograd.Function):
         ctx.rope_start = int(rope_start)
         scores = None
         with torch.no_grad():
-            if qr_out is None and x.dtype == torch.bfloat16 and _save_scores():
+            if qr_out is None and _save_scores():
                 out, scores = hip_attn.tril_rope_score_v_save(x, V, freqs, rope_start)
             else:
                 out = hip_attn.tril_rope_score_v(x, V, freqs, rope_start, qr_out=qr_out)

@@ -223,13 +223,14 @@ int bdh_tril_rope_score_v_bwd(const bdh_tensor4* x, const bdh_tensor4* v,
  * default autograd keeps S, attention_bwd.py:259-291).
  * bdh_tril_rope_score_v_keeps_scores returns 1 when bdh_tril_rope_score_v(x, v,
  * out, freqs, rope_start, NULL, ...) on these views runs the bf16 MFMA path
- * and leaves its score tiles in its workspace, of which the backward needs
- * the first *scores_bytes; else 0.  bdh_tril_rope_score_v_bwd_saved takes
+ * (or x is fp32: any shape) and leaves its score tiles in its workspace, of
+ * which the backward needs the first *scores_bytes; else 0.  bdh_tril_rope_score_v_bwd_saved takes
  * that workspace as `scores` (x, v, freqs and rope_start those of the
  * forward, x unchanged since) and recomputes no score tile: dv from the kept
  * tiles, dx as above with x rotated (absolute positions) as the dQ product
  * stages it, so R(x) is never written.  Other views
- * give BDH_ERR_ARG.  bf16 x, dout and v; D a multiple of 64 up to 256.
+ * give BDH_ERR_ARG.  bf16 x, dout and v with D a multiple of 64 up to 256, or
+ * fp32 x (scores 16-byte aligned).
  */
 int bdh_tril_rope_score_v_keeps_scores(const bdh_tensor4* x, const bdh_tensor4* v,
                                        size_t* scores_bytes);

@@ -74,6 +74,10 @@ def test_forward_and_backward_at_tile_edges(T, N, D, rope):
         assert torch.equal(got, ext.tril_rope_score_v(xd, vd, fd, start))  # the copy changes nothing
         assert _rel(qr, r64.detach()) <= TOL
         dx, dv = ext.tril_rope_score_v_bwd(xd, vd, dd, fd, start)
+        out, scores = ext.tril_rope_score_v_save(xd, vd, fd, start)
+        assert torch.equal(out, got)
+        for a, b in zip(ext.tril_rope_score_v_bwd_saved(xd, vd, dd, fd, start, scores), (dx, dv)):
+            assert torch.equal(a, b)  # the kept tiles are those the backward would make
     else:
         got = ext.tril_score_v(xd, xd, vd)
         dx, _, dv = ext.tril_score_v_bwd(xd, None, vd, dd)
