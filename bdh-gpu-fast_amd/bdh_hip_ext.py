@@ -55,6 +55,7 @@ __all__ = [
     "gated_decoder",
     "gated_bwd",
     "relu_bwd_add",
+    "tn_gemm",
     "small_gemm",
     "decode_step",
     "layer_norm_rows",
@@ -97,6 +98,7 @@ EXPORTED_SYMBOLS = (
     "bdh_gated_decoder",
     "bdh_gated_bwd",
     "bdh_relu_bwd_add",
+    "bdh_tn_gemm",
     "bdh_small_gemm_workspace",
     "bdh_small_gemm",
     "bdh_decode_step_workspace",
@@ -172,6 +174,7 @@ def _load():
         "bdh_gated_decoder": (ctypes.c_int, [P, P, P, P, P, vp, sz, vp]),
         "bdh_gated_bwd": (ctypes.c_int, [P, P, P, P, P, P, P, vp]),
         "bdh_relu_bwd_add": (ctypes.c_int, [P, P, P, P, vp]),
+        "bdh_tn_gemm": (ctypes.c_int, [P, P, P, vp]),
         "bdh_small_gemm_workspace": (sz, [i64, i64, i64]),
         "bdh_small_gemm": (ctypes.c_int, [P, P, P, vp, sz, vp]),
         "bdh_decode_step_workspace": (sz, [i64, i64, i64, i64, i64]),
@@ -787,6 +790,20 @@ def relu_bwd_add(a: torch.Tensor, b: torch.Tensor, x: torch.Tensor, out: Optiona
                                    _t4(out), _stream(dev))
     _check(rc, "relu_bwd_add")
     return out
+
+
+def tn_gemm(a: torch.Tensor, b: torch.Tensor, splits: int = 1) -> torch.Tensor:
+    """``a^T b`` per head, contracted over rows: a (H, K, M), b (H, K, N) bf16 -> (H, M, N) fp32;
+    K (in ``splits`` equal parts, added up) a multiple of 32 ``splits``, N of 256."""
+    dev = _require_device(a, b)
+    H, K, M = a.shape
+    out = torch.empty(splits, H, M, b.size(2), dtype=torch.float32, device=dev)
+    with _on(dev):
+        rc = _lib.bdh_tn_gemm(_t4(a.unsqueeze(0)), _t4(b.unsqueeze(0)), _t4(out), _stream(dev))
+    _check(rc, "tn_gemm")
+    for s in range(1, splits):
+        out[0].add_(out[s])
+    return out[0]
 
 
 def small_gemm(a: torch.Tensor, b: torch.Tensor, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:

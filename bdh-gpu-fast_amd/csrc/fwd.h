@@ -94,6 +94,8 @@ int sy_bwd_g(const bdh_tensor4* dout, const bdh_tensor4* v, void* g, int64_t tpa
 // for its columns and both operands stream as whole 128-byte lines.
 int sy_dq(const void* g, int64_t tpad, bool g_sym, const bdh_tensor4* x, const bdh_tensor4* out, hipStream_t s,
           const float* freqs = nullptr, int64_t rope_start = 0, bool rot_b = false, const bdh_tensor4* add = nullptr);
+// Products over rows on the same kernel (bdh_tn_gemm, checked there).
+int sy_tn(const bdh_tensor4* a, const bdh_tensor4* b, const bdh_tensor4* out, hipStream_t s);
 // Backward of the fused RoPE op on the MFMA path (syrk.hip): the score tiles
 // of R(x) R(x)^T with R(x) written to qr (absolute positions; ws starts with
 // their (cos, sin) table, *tiles points at the tiles).

@@ -5,7 +5,7 @@
 //   dz = g x where s > 0     (d y = dz wt, d wt = dz^T y)
 // and the ReLU gradient that joins the two uses of x:
 //   out = (a + b) where x > 0.
-#include "common.h"
+#include "fwd.h"
 #include "lds_dma.h"
 
 namespace bdh {
@@ -285,7 +285,7 @@ __global__ __launch_bounds__(256) void k_relu_bwd_add(ReluAddArgs p) {
   }
 }
 
-bool rows16(const bdh_tensor4* t) {
+bool rows_16(const bdh_tensor4* t) {
   if ((reinterpret_cast<uintptr_t>(t->data) & 15) != 0) return false;
   for (int i = 0; i < 3; ++i)
     if (t->size[i] > 1 && t->stride[i] % 8 != 0) return false;
@@ -331,7 +331,7 @@ extern "C" int bdh_gated_bwd(const bdh_tensor4* y, const bdh_tensor4* wt, const 
   if (numel4(x) == 0) return BDH_OK;
   if (K < kBK32 || K % kBK32 != 0 || N % 8 != 0) return BDH_ERR_SHAPE;
   for (const bdh_tensor4* t : all)
-    if (!rows16(t)) return BDH_ERR_STRIDE;
+    if (!rows_16(t)) return BDH_ERR_STRIDE;
   const int64_t M = B * T;
   if (M >= (int64_t(1) << 31) || T >= (int64_t(1) << 31)) return BDH_ERR_SHAPE;
   // the DMA takes 32-bit byte offsets from the per-head bases
@@ -389,7 +389,7 @@ extern "C" int bdh_relu_bwd_add(const bdh_tensor4* a, const bdh_tensor4* b, cons
   if (numel4(x) == 0) return BDH_OK;
   if (x->size[3] % 8 != 0) return BDH_ERR_SHAPE;
   for (const bdh_tensor4* t : {a, b, x, out})
-    if (!rows16(t)) return BDH_ERR_STRIDE;
+    if (!rows_16(t)) return BDH_ERR_STRIDE;
   // out may be one of the inputs itself (each element is read before it is written)
   auto same = [&](const bdh_tensor4* t) {
     if (t->data != out->data) return false;
@@ -414,4 +414,22 @@ extern "C" int bdh_relu_bwd_add(const bdh_tensor4* a, const bdh_tensor4* b, cons
   BDH_LAUNCH("k_relu_bwd_add", k_relu_bwd_add, dim3(unsigned((rows + kReluRows - 1) / kReluRows), unsigned(ncol)),
              dim3(256), 0, static_cast<hipStream_t>(stream), p);
   return BDH_OK;
+}
+
+extern "C" int bdh_tn_gemm(const bdh_tensor4* a, const bdh_tensor4* b, const bdh_tensor4* out, bdh_stream stream) {
+  for (const bdh_tensor4* t : {a, b, out}) BDH_TRY(check_view(t));
+  if (a->dtype != BDH_BF16 || b->dtype != BDH_BF16 || out->dtype != BDH_F32) return BDH_ERR_DTYPE;
+  const int64_t S = out->size[0], H = a->size[1], K = a->size[2], M = a->size[3], N = b->size[3];
+  if (a->size[0] != 1 || b->size[0] != 1 || b->size[1] != H || b->size[2] != K) return BDH_ERR_SHAPE;
+  if (out->size[1] != H || out->size[2] != M || out->size[3] != N) return BDH_ERR_SHAPE;
+  if (views_overlap(out, a) || views_overlap(out, b)) return BDH_ERR_ALIAS;
+  if (numel4(out) == 0) return BDH_OK;
+  if (K <= 0 || K % (32 * S) != 0 || M % 8 != 0 || N % 256 != 0) return BDH_ERR_SHAPE;
+  if (!rows_16(a) || !rows_16(b)) return BDH_ERR_STRIDE;
+  // 32-bit DMA offsets inside one split of one head; 4 rows of out below 2^31 bytes
+  const int64_t ks = K / S, lim = int64_t(1) << 31;
+  if ((ks * a->stride[2] + M) * 2 >= lim || (ks * b->stride[2] + N) * 2 >= lim || out->stride[2] >= (int64_t(1) << 26) ||
+      K >= lim || S * H > (int64_t(1) << 24))
+    return BDH_ERR_SHAPE;
+  return sy_tn(a, b, out, static_cast<hipStream_t>(stream));
 }

@@ -994,7 +994,11 @@ struct DqsArgs {
   int64_t x0, x1, x2;  // element strides of X over (b, h, t)
   void* o;
   int64_t o0, o1, o2;
-  int H, T, N, tpad, nslab, nti, ntn;
+  int H, T, N, nslab, nti, ntn;
+  int64_t g0, g1;   // element strides of G over (b, h)
+  int lda, nst;     // G's row stride; stages of 32 contracted
+  int acols, mrows; // G columns readable (a multiple of 8); output rows
+  int ksplit = 0;   // > 0: b is a split of the contraction, ksplit rows each (of T in all)
   const float* freqs = nullptr;  // RoPE: the output is R^T(G X), positions rope_start + t
   int64_t rope_start = 0;
   const bf16_t* add = nullptr;  // RADD: the other gradient of x, its strides over (b, h, t)
@@ -1032,17 +1036,26 @@ __global__ __launch_bounds__(kSyThreads, 1) void k_dq_sy(const DqsArgs a) {
   const int bid = blockIdx.x;
   const int xcd = bid & 7, kk = bid >> 3;
   const int tiles = a.nti * a.ntn;
-  const int grp = kk / tiles;
-  const int slab = grp * 8 + xcd;
-  if (slab >= a.nslab) return;
-  const int tt = kk - grp * tiles;
+  int slab, tt;
+  if (a.ksplit > 0) {  // few slabs: the XCDs share their tiles in contiguous ranges
+    const int per = (a.nslab * tiles + 7) / 8, t = xcd * per + kk;
+    if (kk >= per || t >= a.nslab * tiles) return;
+    slab = t / tiles;
+    tt = t - slab * tiles;
+  } else {
+    const int grp = kk / tiles;
+    slab = grp * 8 + xcd;
+    if (slab >= a.nslab) return;
+    tt = kk - grp * tiles;
+  }
   const int tn = tt / a.nti, ti = tt - tn * a.nti;
   const int b = slab / a.H, h = slab - b * a.H;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nst = a.tpad / 32;
+  const int nst = a.nst;
+  const int T = a.ksplit > 0 ? min(a.ksplit, a.T - b * a.ksplit) : a.T;
   const int i0 = ti * kSyTile, n0 = tn * kSyTile;
-  const void* gbase = sgpr_ptr(a.g + int64_t(slab) * a.tpad * a.tpad);
+  const void* gbase = sgpr_ptr(a.g + b * a.g0 + h * a.g1);
   const void* xbase = sgpr_ptr(a.x + b * a.x0 + h * a.x1);
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_u8*)sy_lds);
 
@@ -1054,14 +1067,14 @@ __global__ __launch_bounds__(kSyThreads, 1) void k_dq_sy(const DqsArgs a) {
     const int q = (u * 8 + w) * 1024 + lane * 16;
     const int rb = q >> 9, pb = (q >> 4) & 31, pc = pb ^ (4 * (rb & 3));
     if constexpr (KM) {
-      // row rb of the stage, columns i0 + 8 pc ..; columns past tpad (output
-      // rows past tpad): garbage, not stored
-      aoff[u] = uint32_t((rb * a.tpad + min(i0 + 8 * pc, a.tpad - 8)) * 2);
+      // row rb of the stage, columns i0 + 8 pc ..; columns past acols (output
+      // rows past it): garbage, not stored
+      aoff[u] = uint32_t((rb * a.lda + min(i0 + 8 * pc, a.acols - 8)) * 2);
     } else {
       const int row = q >> 6;
       const int c = ((q >> 4) & 3) ^ ((row >> 2) & 3);
-      const int gi = min(i0 + row, a.tpad - 1);  // rows past tpad: garbage, not stored
-      aoff[u] = uint32_t((gi * a.tpad + 8 * c) * 2);
+      const int gi = min(i0 + row, a.acols - 1);  // rows past it: garbage, not stored
+      aoff[u] = uint32_t((gi * a.lda + 8 * c) * 2);
     }
     brow[u] = rb;
     bcol[u] = uint32_t((n0 + 8 * pc) * 2);
@@ -1079,7 +1092,7 @@ __global__ __launch_bounds__(kSyThreads, 1) void k_dq_sy(const DqsArgs a) {
     StageDma d;
     d.m0 = wl + uint32_t(k * kSySlot);
     const int sc = min(st, nst - 1);
-    d.ka = KM ? uint32_t(sc) * uint32_t(64 * a.tpad) : uint32_t(sc * 64);  // tpad^2 * 2 < 2^31
+    d.ka = KM ? uint32_t(sc) * uint32_t(64 * a.lda) : uint32_t(sc * 64);  // (the host keeps G below 2^31 bytes)
     d.krow = uint32_t(sc * 32);
     return d;
   };
@@ -1089,7 +1102,7 @@ __global__ __launch_bounds__(kSyThreads, 1) void k_dq_sy(const DqsArgs a) {
   };
   auto dma_b = [&](const StageDma& d, auto uc) {
     constexpr int u = decltype(uc)::value;
-    const int row = min(int(d.krow) + brow[u], a.T - 1);  // rows past T meet zero G columns
+    const int row = min(int(d.krow) + brow[u], T - 1);  // rows past T meet zero G columns
     dma16<kSyBlk + u * 8192>(d.m0, xbase, uint32_t(int64_t(row) * a.x2 * 2) + bcol[u]);
   };
 
@@ -1223,7 +1236,7 @@ __global__ __launch_bounds__(kSyThreads, 1) void k_dq_sy(const DqsArgs a) {
   TO* o = static_cast<TO*>(a.o) + b * a.o0 + h * a.o1;
   // Element (m, r) of this lane: row i0 + 128 wm + rr(m, r) + 4 (lane >> 5),
   // column n0 + 64 wn + 32 (m & 1) + (lane & 31).  On a full row block (every
-  // row below T; wave-uniform) each store's row base is a scalar pointer and
+  // row below mrows; wave-uniform) each store's row base is a scalar pointer and
   // the lane's part a 32-bit offset (the host keeps 4 rows of out below 2^31
   // bytes), so the stores need no per-lane 64-bit address arithmetic and no
   // exec-mask branch; the last, partial row block keeps the per-row check.
@@ -1245,13 +1258,13 @@ __global__ __launch_bounds__(kSyThreads, 1) void k_dq_sy(const DqsArgs a) {
       } else {
         const int row = i0 + 128 * wm + rr_of(m, r) + 4 * (lane >> 5);
         const int col = n0 + 64 * wn + 32 * (m & 1) + (lane & 31);
-        if (row < a.T) o[int64_t(row) * a.o2 + col] = from_f<TO>(y);
+        if (row < a.mrows) o[int64_t(row) * a.o2 + col] = from_f<TO>(y);
       }
     };
     // the dword of this lane's column pair in row rr_of(m, r) + (lane & 1) of a view
     auto pair_at = [&](const bf16_t* base, int64_t s0, int64_t s1, int64_t s2, int m, int r) __attribute__((always_inline)) {
       const int row = i0 + 128 * wm + rr_of(m, r) + int(plane);
-      const bf16_t* t = base + b * s0 + h * s1 + int64_t(FULL ? row : min(row, a.T - 1)) * s2;
+      const bf16_t* t = base + b * s0 + h * s1 + int64_t(FULL ? row : min(row, a.mrows - 1)) * s2;
       return *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(t + n0 + 64 * wn + 32 * (m & 1)) + pcol);
     };
     auto put2 = [&](int m, int r, uint32_t v) __attribute__((always_inline)) {
@@ -1260,7 +1273,7 @@ __global__ __launch_bounds__(kSyThreads, 1) void k_dq_sy(const DqsArgs a) {
         *reinterpret_cast<uint32_t*>(rp + pofs) = v;
       } else {
         const int row = i0 + 128 * wm + rr_of(m, r) + int(plane);
-        if (row < a.T)
+        if (row < a.mrows)
           *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(o + int64_t(row) * a.o2 + n0 + 64 * wn + 32 * (m & 1)) + pcol) = v;
       }
     };
@@ -1325,7 +1338,7 @@ __global__ __launch_bounds__(kSyThreads, 1) void k_dq_sy(const DqsArgs a) {
         for (int r = 0; r < 16; ++r) put(m, r, acc[m][r]);
     }
   };
-  if (i0 + kSyTile <= a.T)
+  if (i0 + kSyTile <= a.mrows)
     epilogue(std::true_type());
   else
     epilogue(std::false_type());
@@ -2555,7 +2568,11 @@ int sy_dq(const void* g, int64_t tpad, bool g_sym, const bdh_tensor4* x, const b
   a.H = int(H);
   a.T = int(T);
   a.N = int(N);
-  a.tpad = int(tpad);
+  a.g0 = H * tpad * tpad;
+  a.g1 = tpad * tpad;
+  a.lda = a.acols = int(tpad);
+  a.nst = int(tpad / 32);
+  a.mrows = int(T);
   a.nslab = int(nslab);
   a.nti = int(nti);
   a.ntn = int(ntn);
@@ -2570,6 +2587,42 @@ int sy_dq(const void* g, int64_t tpad, bool g_sym, const bdh_tensor4* x, const b
   const dim3 gs{unsigned(grid)};
   if (g_sym) return launch_dq<true>(a, out->dtype == BDH_BF16, freqs != nullptr, rot_b, gs, s);
   return launch_dq<false>(a, out->dtype == BDH_BF16, freqs != nullptr, rot_b, gs, s);
+}
+
+// out[s][h] = sum over the rows k of split s of a[h][k]^T b[h][k]: the same
+// kernel, a's rows (k) in the place of G's.  Weight gradients contract over
+// the tokens, and with few output rows a grid of whole contractions leaves
+// CUs idle; splits fill it.
+int sy_tn(const bdh_tensor4* at, const bdh_tensor4* bt, const bdh_tensor4* out, hipStream_t s) {
+  const int64_t S = out->size[0], H = at->size[1], K = at->size[2], M = at->size[3], N = bt->size[3];
+  const int64_t ks = K / S;
+  DqsArgs a;
+  a.g = static_cast<const bf16_t*>(at->data);
+  a.g0 = ks * at->stride[2];
+  a.g1 = at->stride[1];
+  a.lda = int(at->stride[2]);
+  a.nst = int(ks / 32);
+  a.acols = int(M);
+  a.mrows = int(M);
+  a.ksplit = int(ks);
+  a.x = static_cast<const bf16_t*>(bt->data);
+  a.x0 = ks * bt->stride[2];
+  a.x1 = bt->stride[1];
+  a.x2 = bt->stride[2];
+  a.o = out->data;
+  a.o0 = out->stride[0];
+  a.o1 = out->stride[1];
+  a.o2 = out->stride[2];
+  a.H = int(H);
+  a.T = int(K);
+  a.N = int(N);
+  a.nslab = int(S * H);
+  a.nti = int((M + kSyTile - 1) / kSyTile);
+  a.ntn = int(N / kSyTile);
+  const int64_t grid = (S * H * a.nti * a.ntn + 7) / 8 * 8;
+  if (grid >= (int64_t(1) << 31)) return BDH_ERR_SHAPE;
+  BDH_LAUNCH("k_dq_sy_tn", (k_dq_sy<float, false, false, true>), dim3(unsigned(grid)), dim3(kSyThreads), 0, s, a);
+  return BDH_OK;
 }
 
 

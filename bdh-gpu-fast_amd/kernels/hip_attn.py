@@ -171,6 +171,12 @@ def relu_bwd_add(a: torch.Tensor, b: torch.Tensor, x: torch.Tensor, out: Optiona
     return ext.relu_bwd_add(a, b, x, out)
 
 
+def tn_gemm(a: torch.Tensor, b: torch.Tensor, splits: int = 1) -> torch.Tensor:
+    """``a^T b`` per head over many rows, fp32 (the layer's weight gradients)."""
+    ext = _require(a, b)
+    return ext.tn_gemm(a, b, splits)
+
+
 def layer_norm_rows(y: torch.Tensor, x: Optional[torch.Tensor] = None,
                     out_dtype: Optional[torch.dtype] = None, out_bf16: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``LN(y)`` or ``LN(x + LN(y))`` over the last dim on the GPU (bdh.py:565-574, 731-750);
@@ -311,6 +317,7 @@ __all__ = [
     "gated_decoder",
     "gated_bwd",
     "relu_bwd_add",
+    "tn_gemm",
     "relu_gemm",
     "small_gemm",
     "decode_step",

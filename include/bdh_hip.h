@@ -329,6 +329,14 @@ int bdh_gated_bwd(const bdh_tensor4* y, const bdh_tensor4* wt, const bdh_tensor4
                   const bdh_tensor4* dout, const bdh_tensor4* dx, const bdh_tensor4* dz, bdh_stream stream);
 
 /*
+ * out[s][h] = sum over the rows k of split s of a[0][h][k]^T b[0][h][k]: a (1, H,
+ * K, M), b (1, H, K, N) bf16, out (S, H, M, N) fp32, split s the rows
+ * [s K/S, (s+1) K/S).  K a multiple of 32 S, M of 8, N of 256, 16-byte rows;
+ * one split of one head within 2 GiB.  (Weight gradients: K the tokens.)
+ */
+int bdh_tn_gemm(const bdh_tensor4* a, const bdh_tensor4* b, const bdh_tensor4* out, bdh_stream stream);
+
+/*
  * The ReLU gradient of a latent with two uses, bf16, one shape: out = a + b
  * where x > 0, else 0 (x the ReLU's output).  The last dimension a multiple
  * of 8, 16-byte rows; out may be one of the inputs itself.

@@ -115,3 +115,17 @@ def test_training_step_gradients_follow_eager_attention(D, nh, mult, B, T, froze
     for n, g in want.items():
         assert got[n].shape == g.shape and got[n].dtype == g.dtype
         assert _rel(got[n], g.double()) <= 3e-2, n
+
+
+# rows in one and several 32-row stages and splits; output rows below, at and
+# over a 256-row tile; row pitches wider than the row
+@pytest.mark.parametrize("nh,K,M,N,splits", [(1, 32, 8, 256, 1), (2, 192, 264, 512, 3), (4, 2048, 256, 1024, 2),
+                                             (1, 4096, 64, 256, 8)])
+def test_row_contraction_matches_float64(nh, K, M, N, splits):
+    """fp32 sums of exact bf16 products: K roundings of 2^-24, in norm below 1e-5."""
+    a, b = _randn(nh, K, M + 8, seed=0)[..., :M], _randn(nh, K, N + 128, seed=1)[..., :N]
+    got = ext.tn_gemm(a, b, splits)
+    want = torch.stack([a[h].double().t() @ b[h].double() for h in range(nh)])
+    assert got.dtype == torch.float32 and _rel(got, want) <= 1e-5
+    with pytest.raises(RuntimeError):
+        ext.tn_gemm(a, b, splits + 4)  # K is not a multiple of 32 (splits + 4)
