@@ -23,6 +23,8 @@
 //  * The 64 x 256 fp32 output of each wave stays in accumulator registers
 //    over all chunks; the heads' partials go to a workspace [h][m][D] and
 //    k_head_sum adds them in head order (deterministic).
+//  * A short prompt has few (head, block) pairs: its N columns are then cut
+//    into splits, each a workgroup with a partial of its own (gd_splits).
 //  * Fragment addresses are a per-lane base XOR a compile-time offset (the
 //    swizzles flip only bits the bases leave clear), which frees the address
 //    registers for reads two steps ahead of their MFMAs, with scheduling
@@ -30,6 +32,8 @@
 //    read each fragment just before its MFMA and waited for it).
 // Workgroups of one head run on the same XCD, so the head's weight chunks
 // stream through that XCD's L2 once for its token blocks.
+#include <algorithm>
+
 #include "common.h"
 #include "lds_dma.h"
 
@@ -53,8 +57,8 @@ struct GatedDecArgs {
   int64_t x0, x1, x2;  // (B, T, nh, N)
   const bf16_t* dec;
   int64_t dr;          // (nh N, D): row stride
-  float* part;         // [nh][M][D]
-  int T, M, N, nh, ntb;
+  float* part;         // [nh][split][M][D]
+  int T, M, N, nh, ntb, nsplit;
   int64_t total, per_xcd;
 };
 
@@ -75,7 +79,8 @@ __global__ __launch_bounds__(256, 1) void k_gated_dec(const GatedDecArgs a) {
   if (kk0 >= a.per_xcd) return;
   const int64_t t = int64_t(xcd) * a.per_xcd + kk0;
   if (t >= a.total) return;
-  const int h = int(t / a.ntb), tb = int(t - int64_t(h) * a.ntb);
+  const int hs = int(t / a.ntb), tb = int(t - int64_t(hs) * a.ntb);
+  const int h = hs / a.nsplit, split = hs - h * a.nsplit;
   const int m0 = tb * kGdMT;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -190,11 +195,13 @@ __global__ __launch_bounds__(256, 1) void k_gated_dec(const GatedDecArgs a) {
     return __builtin_shufflevector(gd_tr4(pb), gd_tr4(pb + 8 * 512), 0, 1, 2, 3, 4, 5, 6, 7);
   };
 
+  // this split's chunks
   const int nck = a.N / kGdNC;
-  issue(0, 0);
-  issue(1, 1);
+  const int ck0 = split * nck / a.nsplit, ck1 = (split + 1) * nck / a.nsplit;
+  issue(ck0, 0);
+  issue(ck0 + 1, 1);
   int slot = 0;
-  for (int ck = 0; ck < nck; ++ck) {
+  for (int ck = ck0; ck < ck1; ++ck) {
     sy_wait<12>();  // chunk ck landed (chunk ck + 1 may be in flight)
     __syncthreads();  // every wave's part of chunk ck landed; chunk ck - 1's reads done
     const int s2 = slot == 0 ? 2 : slot - 1;  // slot of chunk ck - 1 = slot of chunk ck + 2
@@ -263,7 +270,7 @@ __global__ __launch_bounds__(256, 1) void k_gated_dec(const GatedDecArgs a) {
   sy_wait<0>();  // the re-loads past the end landed before the LDS is released
 
   // ---- partial out of head h: rows m0 + 64 w + 32 j + 8 (r / 4) + 4 hl + r % 4
-  float* const pp = a.part + (int64_t(h) * a.M) * kGdD;
+  float* const pp = a.part + (int64_t(hs) * a.M) * kGdD;
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -276,22 +283,38 @@ __global__ __launch_bounds__(256, 1) void k_gated_dec(const GatedDecArgs a) {
     }
 }
 
-// out[m, d] = sum over heads of part[h][m][d], heads in order; four columns a
-// thread, 16-byte loads.
-template <typename TO>
-__global__ __launch_bounds__(256) void k_head_sum(const float* __restrict__ part, int nh, int64_t M, TO* out,
+// out[m, d] = sum over the np partials (heads, their splits) of part[p][m][d]:
+// four columns a thread, 16-byte loads, four partials in flight; G groups of
+// threads take every G-th partial and add up through LDS (many partials of
+// few tokens are a chain of loads otherwise).
+template <typename TO, int G>
+__global__ __launch_bounds__(256) void k_head_sum(const float* __restrict__ part, int np, int64_t M, TO* out,
                                                   int64_t o_rs) {
-  const int64_t e = (int64_t(blockIdx.x) * 256 + threadIdx.x) * 4;
-  if (e >= M * kGdD) return;
-  const int64_t m = e / kGdD, d = e - m * kGdD;
-  f32x4 s = *reinterpret_cast<const f32x4*>(part + e);
-  for (int hh = 1; hh < nh; ++hh) {
-    const f32x4 v = *reinterpret_cast<const f32x4*>(part + int64_t(hh) * M * kGdD + e);
-    s[0] += v[0];
-    s[1] += v[1];
-    s[2] += v[2];
-    s[3] += v[3];
+  constexpr int Q = 256 / G;  // quads a workgroup
+  __shared__ f32x4 sums[G > 1 ? G : 1][G > 1 ? Q : 1];
+  const int g = threadIdx.x / Q, l = threadIdx.x % Q;
+  const int64_t e = (int64_t(blockIdx.x) * Q + l) * 4;
+  const bool live = e < M * kGdD;
+  f32x4 s{0.f, 0.f, 0.f, 0.f};
+  if (live)
+    for (int p = g; p < np; p += 4 * G) {
+      f32x4 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        v[u] = *reinterpret_cast<const f32x4*>(part + int64_t(min(p + u * G, np - 1)) * M * kGdD + e);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (p + u * G < np) s += v[u];
+    }
+  if constexpr (G > 1) {
+    sums[g][l] = s;
+    __syncthreads();
+    if (g != 0) return;
+#pragma unroll
+    for (int u = 1; u < G; ++u) s += sums[u][l];
   }
+  if (!live) return;
+  const int64_t m = e / kGdD, d = e - m * kGdD;
   TO* op = out + m * o_rs + d;
   if constexpr (sizeof(TO) == 4) {
     *reinterpret_cast<f32x4*>(op) = s;
@@ -300,9 +323,46 @@ __global__ __launch_bounds__(256) void k_head_sum(const float* __restrict__ part
   }
 }
 
+template <typename TO>
+int launch_head_sum(const float* part, int np, int64_t M, TO* out, int64_t o_rs, hipStream_t s) {
+  const int64_t quads = M * kGdD / 4;
+  if (np >= 16)
+    BDH_LAUNCH("k_head_sum", (k_head_sum<TO, 8>), dim3(unsigned((quads + 31) / 32)), dim3(256), 0, s, part, np, M, out,
+               o_rs);
+  else
+    BDH_LAUNCH("k_head_sum", (k_head_sum<TO, 1>), dim3(unsigned((quads + 255) / 256)), dim3(256), 0, s, part, np, M,
+               out, o_rs);
+  return BDH_OK;
+}
+
 }  // namespace
 
-size_t gated_dec_workspace(int64_t nh, int64_t M) { return size_t(nh) * size_t(M) * kGdD * sizeof(float); }
+// Column splits of a head, in microseconds of the launch's estimated end: the
+// (head, 256-token block, split) workgroups in rounds of one per CU at 2.2 us
+// a chunk of 32 columns, and the splits' partials (1 KB a token and head)
+// written and read at 4.8 TB/s.  nh = 4, N = 8192: 40 tokens 467 -> 25 us (32
+// splits), 2400 tokens 470 -> 103 (6), 4096 tokens 480 -> 186 (4).
+int64_t gd_splits(int64_t nh, int64_t M, int64_t N, int64_t most) {
+  const int64_t wgs = (M + kGdMT - 1) / kGdMT * nh;
+  int64_t best = 1;
+  double best_t = 0;
+  for (int64_t s = 1; s <= most; ++s) {
+    const double t = double((wgs * s + 255) / 256) * (double(N / kGdNC) / double(s) * 2.2 + 4.) +
+                     (s > 1 ? double(s) * double(M * nh) * 2048. / 4.8e6 : 0.);
+    if (s == 1 || t < best_t * 0.97) {
+      best = s;
+      best_t = t;
+    }
+  }
+  return best;
+}
+constexpr int64_t kGdMostSplits = 32;
+
+// Partials of the splits that N = 8192 takes; the launch stays within them.
+size_t gated_dec_bytes(int64_t nh, int64_t M) { return size_t(nh) * size_t(M) * kGdD * sizeof(float); }
+size_t gated_dec_workspace(int64_t nh, int64_t M) {
+  return size_t(gd_splits(nh, M, 8192, kGdMostSplits)) * gated_dec_bytes(nh, M);
+}
 
 }  // namespace bdh
 
@@ -372,7 +432,10 @@ extern "C" int bdh_gated_decoder(const bdh_tensor4* y, const bdh_tensor4* wt, co
   a.N = int(N);
   a.nh = int(H);
   a.ntb = int((M + kGdMT - 1) / kGdMT);
-  a.total = int64_t(a.ntb) * H;
+  // (never more than the workspace was sized for; four chunks each at least)
+  a.nsplit = int(gd_splits(H, M, N, std::max<int64_t>(1, std::min<int64_t>({int64_t(need / gated_dec_bytes(H, M)),
+                                                                           N / (4 * kGdNC), kGdMostSplits}))));
+  a.total = int64_t(a.ntb) * H * a.nsplit;
   a.per_xcd = (a.total + 7) / 8;
   const int64_t grid = 8 * a.per_xcd;
   if (grid >= (int64_t(1) << 31)) return BDH_ERR_SHAPE;
@@ -380,12 +443,7 @@ extern "C" int bdh_gated_decoder(const bdh_tensor4* y, const bdh_tensor4* wt, co
   BDH_LAUNCH("k_gated_dec", k_gated_dec, dim3(unsigned(grid)), dim3(256), 0, s, a);
   // out rows: (b, t) at b * stride0 + t * stride1; evenly spaced, so row m at m * stride1
   const int64_t o_rs = out->size[1] > 1 ? out->stride[1] : out->stride[0];
-  const int64_t nthr = (M * kGdD / 4 + 255) / 256;
   if (out->dtype == BDH_F32)
-    BDH_LAUNCH("k_head_sum", k_head_sum<float>, dim3(unsigned(nthr)), dim3(256), 0, s, a.part, int(H), M,
-               static_cast<float*>(out->data), o_rs);
-  else
-    BDH_LAUNCH("k_head_sum", k_head_sum<bf16_t>, dim3(unsigned(nthr)), dim3(256), 0, s, a.part, int(H), M,
-               static_cast<bf16_t*>(out->data), o_rs);
-  return BDH_OK;
+    return launch_head_sum(a.part, int(H) * a.nsplit, M, static_cast<float*>(out->data), o_rs, s);
+  return launch_head_sum(a.part, int(H) * a.nsplit, M, static_cast<bf16_t*>(out->data), o_rs, s);
 }

@@ -91,3 +91,16 @@ def test_gated_decoder_rejects_bad_shapes():
         ext.gated_decoder(y[..., :128].contiguous(), wt[..., :128].contiguous(), x, dec)  # K != 256
     with pytest.raises(RuntimeError):
         ext.gated_decoder(y, wt[:, :48].contiguous(), x[..., :48].contiguous(), dec[:96].contiguous())  # N % 32
+
+
+# N columns in splits (few tokens): chunk counts that the splits do not divide,
+# and tokens around the points where the number of splits changes
+@pytest.mark.parametrize("shape", [(1, 40, 1, 544), (5, 60, 2, 1184), (1, 2500, 4, 2080), (1, 1025, 8, 416)])
+def test_column_splits_match_float64(shape):
+    B, T, nh, N = shape
+    y, wt, x, dec = (t.to(DEV) for t in _inputs(B, T, nh, N, seed=3))
+    got = ext.gated_decoder(y, wt, x, dec)
+    assert torch.equal(got, ext.gated_decoder(y, wt, x, dec))
+    xy = (x.double() * torch.relu(torch.stack([y[:, h].double() @ wt[h].double().t() for h in range(nh)], 2)))
+    want = xy.float().to(BF).double().reshape(B, T, nh * N) @ dec.double()
+    assert float((got.double() - want).norm() / want.norm()) <= 2e-3  # as above: its own rounding of xy
