@@ -21,7 +21,7 @@ ROOT = HERE.parent
 CSRC = HERE / "csrc"
 BUILD = HERE / "_build"
 LIB = HERE / "libbdh_hip.so"
-SOURCES = ["api.hip", "fwd.hip", "syrk.hip", "bwd.hip", "f32.hip", "decode.hip", "decode_step.hip", "rope.hip", "model.hip", "gated_dec.hip", "gated_bwd.hip", "enc.hip"]
+SOURCES = ["api.hip", "fwd.hip", "syrk.hip", "bwd.hip", "f32.hip", "decode.hip", "decode_step.hip", "rope.hip", "model.hip", "gated_dec.hip", "gated_bwd.hip", "few.hip", "enc.hip"]
 ARCH = os.environ.get("BDH_OFFLOAD_ARCH", "gfx950")
 
 

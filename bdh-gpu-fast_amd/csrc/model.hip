@@ -629,6 +629,11 @@ namespace bdh {
 bool relu_enc_takes(int64_t K, int64_t N);
 int relu_enc_launch(const bdh_tensor4* y, const bdh_tensor4* wt, const bdh_tensor4* x, const bdh_tensor4* out,
                     hipStream_t s);
+bool few_gemm_takes(int64_t M, int64_t K);
+int few_gemm_launch(const bdh_tensor4* y, const bdh_tensor4* wt, const bdh_tensor4* x, const bdh_tensor4* out,
+                    hipStream_t s);
+bool few_dec_takes(const bdh_tensor4* a, const bdh_tensor4* b);
+int few_dec_launch(const bdh_tensor4* a, const bdh_tensor4* b, const bdh_tensor4* out, float* part, hipStream_t s);
 }  // namespace bdh
 
 // out = [x *] relu(y @ wt^T) per head (x null: the ReLU GEMM alone, k_relu_enc
@@ -696,6 +701,8 @@ static int gated_gemm_launch(const bdh_tensor4* y, const bdh_tensor4* wt, const 
   // few tokens take the tile kernel, whose grid spans the columns too).
   if (relu_enc_takes(K, N) && (M + 255) / 256 * H >= 128 && ((N - 1) * wt->stride[2] + K) * 2 < (int64_t(1) << 32))
     return relu_enc_launch(y, wt, x, out, static_cast<hipStream_t>(stream));
+  // a generate step's few tokens
+  if (few_gemm_takes(M, K)) return few_gemm_launch(y, wt, x, out, static_cast<hipStream_t>(stream));
   if (x != nullptr)
     BDH_LAUNCH("k_gated_gemm", k_gated_gemm<true>, dim3(unsigned(grid)), dim3(512), 0,
                static_cast<hipStream_t>(stream), a);
@@ -719,7 +726,8 @@ extern "C" int bdh_relu_gemm(const bdh_tensor4* y, const bdh_tensor4* wt, const 
 
 extern "C" size_t bdh_small_gemm_workspace(int64_t M, int64_t K, int64_t D) {
   if (M <= 0 || K <= 0 || D <= 0) return 0;
-  return small_gemm_plan(M, K, D).ws_bytes;
+  const size_t few = M <= 64 && D == 256 && K % 128 == 0 ? size_t(K / 128) * size_t(M) * size_t(D) * sizeof(float) : 0;
+  return std::max(small_gemm_plan(M, K, D).ws_bytes, few);
 }
 
 // out (1, 1, M, D) = a (1, 1, M, K) @ b (1, 1, K, D); see k_small_gemm.
@@ -754,6 +762,10 @@ extern "C" int bdh_small_gemm(const bdh_tensor4* a, const bdh_tensor4* b, const 
   g.avec = (reinterpret_cast<uintptr_t>(a->data) & 15) == 0 && a->stride[2] % 8 == 0 && K % 8 == 0;
   g.bvec = (reinterpret_cast<uintptr_t>(b->data) & 7) == 0 && b->stride[2] % 4 == 0 && D % 4 == 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // few rows and D = 256: one-shot splits of 128 rows, where they fit the workspace
+  if (few_dec_takes(a, b) && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
+      size_t(K / 128) * size_t(M) * size_t(D) * sizeof(float) <= workspace_bytes)
+    return few_dec_launch(a, b, out, g.part, s);
   const dim3 grid{unsigned((D + kTile - 1) / kTile), unsigned(p.nsplit), unsigned((M + kTile - 1) / kTile)};
   BDH_LAUNCH("k_small_gemm", k_small_gemm, grid, dim3(kNT), 0, s, g);
   // the 16-byte reduce needs 16-byte aligned partial rows: D % 4 == 0 and an
