@@ -411,7 +411,8 @@ extern "C" int bdh_gated_decoder(const bdh_tensor4* y, const bdh_tensor4* wt, co
   if (((N - 1) * wt->stride[2] + K) * 2 >= (int64_t(1) << 32)) return BDH_ERR_SHAPE;
   if (((N - 1) * dec->stride[2] + kGdD) * 2 >= (int64_t(1) << 32)) return BDH_ERR_SHAPE;
   const size_t need = gated_dec_workspace(H, M);
-  if (workspace == nullptr || workspace_bytes < need) return BDH_ERR_WORKSPACE;
+  const size_t one = gated_dec_bytes(H, M);  // one split is enough; as many as fit
+  if (workspace == nullptr || workspace_bytes < one) return BDH_ERR_WORKSPACE;
   GatedDecArgs a;
   a.y = static_cast<const bf16_t*>(y->data);
   a.y0 = y->stride[0];
@@ -432,8 +433,8 @@ extern "C" int bdh_gated_decoder(const bdh_tensor4* y, const bdh_tensor4* wt, co
   a.N = int(N);
   a.nh = int(H);
   a.ntb = int((M + kGdMT - 1) / kGdMT);
-  // (never more than the workspace was sized for; four chunks each at least)
-  a.nsplit = int(gd_splits(H, M, N, std::max<int64_t>(1, std::min<int64_t>({int64_t(need / gated_dec_bytes(H, M)),
+  // (never more than the workspace holds; four chunks each at least)
+  a.nsplit = int(gd_splits(H, M, N, std::max<int64_t>(1, std::min<int64_t>({int64_t(std::min(need, workspace_bytes) / one),
                                                                            N / (4 * kGdNC), kGdMostSplits}))));
   a.total = int64_t(a.ntb) * H * a.nsplit;
   a.per_xcd = (a.total + 7) / 8;

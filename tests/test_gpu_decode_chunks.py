@@ -36,3 +36,27 @@ def test_chunked_past_matches_float64(B, H, S, N, qdt, kdt):
     err = float((got.double() - want).norm() / want.norm())
     assert err <= (1e-5 if qdt == torch.float32 else 4e-3), err
     assert torch.equal(got, ext.tril_decode_noalloc(q, ks, vs))
+
+
+# a workspace of the 32-key partials alone (sized for a longer past, say): larger chunks, nothing past its end
+@pytest.mark.parametrize("S", [5, 301, 1024])
+@pytest.mark.parametrize("N,dt", [(8192, torch.bfloat16), (512, torch.float32), (200, torch.float32)])
+def test_smallest_workspace(S, N, dt):
+    H, Dv = 4, 64
+    g = torch.Generator(device="cuda").manual_seed(S)
+    k = torch.randn(1, H, S, N, generator=g, device="cuda").to(dt)
+    v = torch.randn(1, 1, S, Dv, generator=g, device="cuda").to(dt)
+    q = torch.randn(1, H, 1, N, generator=g, device="cuda").to(dt)
+    n = (S + 31) // 32 * H * Dv
+    ws = torch.full((n + 64,), 7.0, device="cuda")
+    out = torch.empty(1, H, 1, Dv, dtype=dt, device="cuda")
+
+    def call(nbytes):
+        return ext._lib.bdh_tril_decode(ext._t4(q), ext._t4(k), ext._t4(v), ext._t4(out), ws.data_ptr(), nbytes,
+                                        ext._stream(out.device))
+
+    assert call(4 * n) == 0
+    want = (q[0].double() @ k[0].double().transpose(-2, -1).contiguous()) @ v[0].double()
+    assert float((out[0].double() - want).norm() / want.norm()) <= (1e-5 if dt == torch.float32 else 4e-3)
+    assert bool((ws[n:] == 7.0).all())
+    assert call(4 * n - 4) != 0

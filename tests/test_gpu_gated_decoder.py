@@ -104,3 +104,27 @@ def test_column_splits_match_float64(shape):
     xy = (x.double() * torch.relu(torch.stack([y[:, h].double() @ wt[h].double().t() for h in range(nh)], 2)))
     want = xy.float().to(BF).double().reshape(B, T, nh * N) @ dec.double()
     assert float((got.double() - want).norm() / want.norm()) <= 2e-3  # as above: its own rounding of xy
+
+
+@pytest.mark.parametrize("room", [1, 3])
+def test_column_splits_stay_within_the_workspace(room):
+    """A workspace for fewer splits than the launch would take (one is enough)."""
+    nh, N, T = 4, 1024, 40
+    g = torch.Generator(device="cuda").manual_seed(1)
+    y, wt, dec = (torch.randn(*s, generator=g, device="cuda").bfloat16()
+                  for s in ((1, nh, T, 256), (nh, N, 256), (nh * N, 256)))
+    x = torch.relu(torch.randn(1, T, nh, N, generator=g, device="cuda")).bfloat16()
+    n = nh * T * 256
+    ws = torch.full((room * n + 64,), 7.0, device="cuda")
+    out = torch.empty(1, T, 256, device="cuda")
+
+    def call(nbytes):
+        return ext._lib.bdh_gated_decoder(ext._t4(y), ext._t4(wt.unsqueeze(0)), ext._t4(x),
+                                          ext._t4(dec.view(1, 1, *dec.shape)), ext._t4(out.view(1, T, 1, -1)),
+                                          ws.data_ptr(), nbytes, ext._stream(out.device))
+
+    assert call(4 * room * n) == 0
+    want = ext.gated_decoder(y, wt, x, dec)
+    assert float((out - want).norm() / want.norm()) <= 1e-5  # the splits' fp32 sums in another order
+    assert bool((ws[room * n:] == 7.0).all())
+    assert call(4 * n - 4) != 0
