@@ -58,6 +58,28 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// A row of D = 64 E values, E a lane: LayerNorm without weights, eps 1e-5.
+template <int E>
+__device__ __forceinline__ void ln_row(float (&v)[E], int D) {
+  float s = 0.f;
+#pragma unroll
+  for (int e = 0; e < E; ++e) s += v[e];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  const float mean = s / float(D);
+  float q = 0.f;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    v[e] -= mean;
+    q += v[e] * v[e];
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) q += __shfl_xor(q, off, 64);
+  const float r = rsqrtf(q / float(D) + 1e-5f);
+#pragma unroll
+  for (int e = 0; e < E; ++e) v[e] *= r;
+}
+
 // A strided 4-D view as seen by kernels: base pointer + element strides of the
 // three outer dimensions (the last dimension is unit-stride).
 struct View {

@@ -18,6 +18,7 @@
 #include <mutex>
 
 #include "common.h"
+#include "few.h"
 
 namespace bdh {
 
@@ -332,6 +333,46 @@ __global__ __launch_bounds__(kDecNT) void k_decode_reduce(const float* part, int
   op[d] = from_f<TO>(s);
 }
 
+// The same with LN(row) behind it (one query a head, Dv = 64 E): a workgroup of
+// eight waves a row, a wave takes every eighth chunk, four in flight.  What it
+// saves is a launch: 32 rows of 256, 75 chunks: 4.8 us and 4.6 for the row
+// LayerNorm before, 4.8 now.
+template <int E>
+__global__ __launch_bounds__(512) void k_decode_ln(const float* part, int64_t nchunk, int64_t rows, View o, int64_t H) {
+  __shared__ float sums[8][64 * E];
+  const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
+  const int64_t row = blockIdx.x, n = rows * 64 * E;
+  const float* pr = part + row * 64 * E + lane;
+  float s[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) s[e] = 0.f;
+  for (int64_t c = g; c < nchunk; c += 32) {
+    float w[4][E];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int e = 0; e < E; ++e) w[u][e] = pr[min(c + 8 * u, nchunk - 1) * n + 64 * e];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int e = 0; e < E; ++e) s[e] += c + 8 * u < nchunk ? w[u][e] : 0.f;
+  }
+#pragma unroll
+  for (int e = 0; e < E; ++e) sums[g][64 * e + lane] = s[e];
+  __syncthreads();
+  if (g != 0) return;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+#pragma unroll
+    for (int u = 1; u < 8; ++u) s[e] += sums[u][64 * e + lane];
+    s[e] = bf_round(s[e]);
+  }
+  ln_row<E>(s, 64 * E);
+  bf16_t* op = static_cast<bf16_t*>(const_cast<void*>(o.p)) + (row / H) * o.s0 + (row % H) * o.s1 + lane;
+#pragma unroll
+  for (int e = 0; e < E; ++e) op[64 * e] = f2bf(s[e]);
+}
+
 // Keys per workgroup: 64 where that already makes three workgroups per CU
 // (8 sequences, 32 rows, S = 1500: 127 us, 145 in 32-key chunks), else the
 // largest of 32 ... 4 that makes eight, as long as the partial sums fit the
@@ -464,8 +505,8 @@ int decode_plan(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v
 
 // The partial kernels write every (chunk, row, column) of part, so part needs
 // no clearing between calls.
-int decode_run(const DecodePlan& p, const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v,
-               const bdh_tensor4* out, float* part, hipStream_t st) {
+int decode_parts(const DecodePlan& p, const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v, float* part,
+                 hipStream_t st) {
   DecodeArgs a = p.a;
   a.part = part;
   if (p.kind == kDecBf16) {
@@ -491,20 +532,63 @@ int decode_run(const DecodePlan& p, const bdh_tensor4* q, const bdh_tensor4* k, 
                                         : pick_k<float>(a, p.nred, k->dtype, v->dtype, st);
     if (rc != BDH_OK) return rc;
   }
+  return BDH_OK;
+}
+
+int decode_run(const DecodePlan& p, const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v,
+               const bdh_tensor4* out, float* part, hipStream_t st) {
+  BDH_TRY(decode_parts(p, q, k, v, part, st));
+  const DecodeArgs& a = p.a;
   View o = view_of(out);
   o.s1 = out->stride[1];
   const int64_t total = a.rows * a.Dv;
   dim3 grid((unsigned)((total + kRedCols - 1) / kRedCols));
   if (out->dtype == BDH_BF16)
-    BDH_LAUNCH("k_decode_reduce", k_decode_reduce<bf16_t>, grid, dim3(kDecNT), 0, st, a.part, p.nred, a.rows,
+    BDH_LAUNCH("k_decode_reduce", k_decode_reduce<bf16_t>, grid, dim3(kDecNT), 0, st, part, p.nred, a.rows,
                a.Dv, o, a.H, a.Tq);
   else
-    BDH_LAUNCH("k_decode_reduce", k_decode_reduce<float>, grid, dim3(kDecNT), 0, st, a.part, p.nred, a.rows,
+    BDH_LAUNCH("k_decode_reduce", k_decode_reduce<float>, grid, dim3(kDecNT), 0, st, part, p.nred, a.rows,
                a.Dv, o, a.H, a.Tq);
   return BDH_OK;
 }
 
+// A workspace of 32-key partials is enough (one sized for a longer past may be
+// smaller than what this one's smaller chunks take): the chunks grow until
+// their partials fit.
+int decode_fit(DecodePlan& p, const void* workspace, size_t workspace_bytes) {
+  auto bytes = [&](int64_t chunk) {
+    return size_t(n_chunks(p.a.S, chunk)) * size_t(p.a.rows) * size_t(p.a.Dv) * sizeof(float);
+  };
+  if (workspace == nullptr || workspace_bytes < bytes(kChunk)) return BDH_ERR_WORKSPACE;
+  while (bytes(p.a.chunk) > workspace_bytes) p.a.chunk *= 2;
+  p.nred = n_chunks(p.a.S, p.a.chunk);
+  p.part_bytes = bytes(p.a.chunk);
+  return BDH_OK;
+}
+
 }  // namespace
+
+int decode_ln(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v, const bdh_tensor4* out, void* workspace,
+              size_t workspace_bytes, hipStream_t s) {
+  DecodePlan p;
+  BDH_TRY(decode_plan(q, k, v, out, p));
+  if (out->dtype != BDH_BF16 || p.a.Tq != 1) return BDH_ERR_ARG;
+  if (numel4(out) == 0) return BDH_OK;
+  BDH_TRY(decode_fit(p, workspace, workspace_bytes));
+  float* part = static_cast<float*>(workspace);
+  BDH_TRY(decode_parts(p, q, k, v, part, s));
+  const View o = view_of(out);
+  const dim3 grid{unsigned(p.a.rows)};
+  switch (p.a.Dv) {
+    case 64: BDH_LAUNCH("k_decode_ln", k_decode_ln<1>, grid, dim3(512), 0, s, part, p.nred, p.a.rows, o, p.a.H); break;
+    case 128: BDH_LAUNCH("k_decode_ln", k_decode_ln<2>, grid, dim3(512), 0, s, part, p.nred, p.a.rows, o, p.a.H); break;
+    case 256: BDH_LAUNCH("k_decode_ln", k_decode_ln<4>, grid, dim3(512), 0, s, part, p.nred, p.a.rows, o, p.a.H); break;
+    case 512: BDH_LAUNCH("k_decode_ln", k_decode_ln<8>, grid, dim3(512), 0, s, part, p.nred, p.a.rows, o, p.a.H); break;
+    case 1024: BDH_LAUNCH("k_decode_ln", k_decode_ln<16>, grid, dim3(512), 0, s, part, p.nred, p.a.rows, o, p.a.H); break;
+    default: return BDH_ERR_SHAPE;
+  }
+  return BDH_OK;
+}
 }  // namespace bdh
 
 extern "C" int bdh_tril_decode(const bdh_tensor4* q, const bdh_tensor4* k, const bdh_tensor4* v,
@@ -513,16 +597,7 @@ extern "C" int bdh_tril_decode(const bdh_tensor4* q, const bdh_tensor4* k, const
   DecodePlan p;
   BDH_TRY(decode_plan(q, k, v, out, p));
   if (numel4(out) == 0) return BDH_OK;
-  // A workspace of 32-key partials is enough (one sized for a longer past may
-  // be smaller than what this one's smaller chunks take): the chunks grow
-  // until their partials fit.
-  auto bytes = [&](int64_t chunk) {
-    return size_t(n_chunks(p.a.S, chunk)) * size_t(p.a.rows) * size_t(p.a.Dv) * sizeof(float);
-  };
-  if (workspace == nullptr || workspace_bytes < bytes(kChunk)) return BDH_ERR_WORKSPACE;
-  while (bytes(p.a.chunk) > workspace_bytes) p.a.chunk *= 2;
-  p.nred = n_chunks(p.a.S, p.a.chunk);
-  p.part_bytes = bytes(p.a.chunk);
+  BDH_TRY(decode_fit(p, workspace, workspace_bytes));
   return decode_run(p, q, k, v, out, static_cast<float*>(workspace), static_cast<hipStream_t>(stream));
 }
 

@@ -1,21 +1,25 @@
 // One generate step of the whole model as one call: the layers' kernels are
 // launched back to back from here, so a step costs the host its launches and
-// one call instead of six calls a layer through the binding.  No kernel of its
-// own: every layer runs the library's entry points in the order of the
-// model's cached forward,
+// one call instead of six calls a layer through the binding.  Every layer runs the
+// library's entry points in the order of the model's cached forward,
 //   lat  = relu(x encoder)            (x: the bf16 row in this layer's V slot)
 //   KR slot = RoPE(lat), y = decode(KR slot, past)
 //   xy   = lat * relu(LN(y) encoder_v), y_mlp = xy decoder
-//   x    = LN(x + LN(y_mlp)), rounded to bf16 into the next layer's V slot.
+//   x    = LN(x + LN(y_mlp)), rounded to bf16 into the next layer's V slot,
+// with what is a launch of a few microseconds behind a product fused into it:
+// RoPE in the few-row encoder product, the LayerNorms in the sums of the
+// decode's chunks and of the decoder's splits (8 sequences, 6 layers, D = 256, S
+// = 300: 417 -> 380 us a step).
 #include <algorithm>
 
 #include "common.h"
+#include "few.h"
 
 namespace bdh {
 namespace {
 
 struct StepWs {
-  size_t lat, xy, ykv, yln, ymlp, xa, dec, gemm, end;
+  size_t lat, xy, yln, ymlp, xa, dec, gemm, end;
 };
 
 StepWs step_ws(int64_t B, int64_t nh, int64_t N, int64_t D, int64_t S) {
@@ -28,7 +32,6 @@ StepWs step_ws(int64_t B, int64_t nh, int64_t N, int64_t D, int64_t S) {
   };
   w.lat = take(size_t(B * nh * N) * 2);
   w.xy = take(size_t(B * nh * N) * 2);
-  w.ykv = take(size_t(B * nh * D) * 2);
   w.yln = take(size_t(B * nh * D) * 2);
   w.ymlp = take(size_t(B * D) * 2);
   w.xa = take(size_t(B * D) * 4 * 2);  // the residual stream, two buffers in turn
@@ -88,11 +91,13 @@ extern "C" int bdh_decode_step(const bdh_tensor4* x, const bdh_tensor4* out, con
   const bdh_tensor4 lat_h = view4(w + o.lat, BDH_BF16, B, nh, 1, N, nh * N, N, N);
   const bdh_tensor4 xy = view4(w + o.xy, BDH_BF16, B, 1, nh, N, nh * N, nh * N, N);
   const bdh_tensor4 xy_rows = view4(w + o.xy, BDH_BF16, 1, 1, B, nh * N, B * nh * N, B * nh * N, nh * N);
-  const bdh_tensor4 ykv = view4(w + o.ykv, BDH_BF16, B, nh, 1, D, nh * D, D, D);
   const bdh_tensor4 yln = view4(w + o.yln, BDH_BF16, B, nh, 1, D, nh * D, D, D);
   const bdh_tensor4 ymlp = view4(w + o.ymlp, BDH_BF16, 1, 1, B, D, B * D, B * D, D);
   const bdh_tensor4 cos_h = view4(cos->data, cos->dtype, B, nh, 1, N, 0, 0, 0);
   const bdh_tensor4 sin_h = view4(sin->data, sin->dtype, B, nh, 1, N, 0, 0, 0);
+  const bool few_dec = dec->dtype == BDH_BF16 && dec->size[0] == 1 && dec->size[1] == 1 && few_dec_takes(&xy_rows, dec) &&
+                       size_t(nh * N / 128) * size_t(B * D) * 4 <= o.end - o.gemm;
+  const hipStream_t s = static_cast<hipStream_t>(stream);
   bdh_tensor4 cur = *x;
   for (int32_t l = 0; l < n_layer; ++l) {
     const char* krl = static_cast<const char*>(kr->data) + int64_t(l) * kr_layer * 2;
@@ -103,17 +108,32 @@ extern "C" int bdh_decode_step(const bdh_tensor4* x, const bdh_tensor4* out, con
                                      kr->stride[1], kr->stride[2]);
     // this token's bf16 row for the heads to share
     const bdh_tensor4 row = view4(vl + seq_len * v->stride[2] * 2, BDH_BF16, B, nh, 1, D, v->stride[0], 0, v->stride[2]);
-    BDH_TRY(bdh_relu_gemm(&row, enc_t, &lat, stream));
-    BDH_TRY(bdh_rope_rotate(&lat_h, &cos_h, &sin_h, &slot_k, 0, stream));
-    BDH_TRY(bdh_tril_decode(&slot_k, &past_k, &past_v, &ykv, w + o.dec, o.gemm - o.dec, stream));
-    BDH_TRY(bdh_layer_norm_rows(nullptr, &ykv, &yln, stream));
+    const FewRope rope{static_cast<const float*>(cos->data), static_cast<const float*>(sin->data),
+                       static_cast<bf16_t*>(slot_k.data), slot_k.stride[0], slot_k.stride[1]};
+    const bool can_rope = cos->dtype == BDH_F32 && sin->dtype == BDH_F32 && vec16_ok(cos) && vec16_ok(sin) &&
+                          vec16_ok(&slot_k) && !views_overlap(&slot_k, &lat) && !views_overlap(&slot_k, &row) &&
+                          !views_overlap(&slot_k, enc_t) && !views_overlap(&slot_k, cos) && !views_overlap(&slot_k, sin);
+    bool roped = false;
+    BDH_TRY(relu_gemm_rope(&row, enc_t, &lat, can_rope ? &rope : nullptr, &roped, stream));
+    if (!roped) BDH_TRY(bdh_rope_rotate(&lat_h, &cos_h, &sin_h, &slot_k, 0, stream));
+    BDH_TRY(decode_ln(&slot_k, &past_k, &past_v, &yln, w + o.dec, o.gemm - o.dec, s));
     BDH_TRY(bdh_gated_gemm(&yln, encv_t, &lat, &xy, stream));
-    BDH_TRY(bdh_small_gemm(&xy_rows, dec, &ymlp, w + o.gemm, o.end - o.gemm, stream));
-    if (l + 1 == n_layer) return bdh_layer_norm_rows(&cur, &ymlp, out, stream);
-    const bdh_tensor4 nxt = view4(w + o.xa + size_t(l & 1) * size_t(B * D) * 4, BDH_F32, 1, 1, B, D, B * D, B * D, D);
+    const bool last = l + 1 == n_layer;
+    const bdh_tensor4 nxt = last ? *out
+                                 : view4(w + o.xa + size_t(l & 1) * size_t(B * D) * 4, BDH_F32, 1, 1, B, D, B * D,
+                                         B * D, D);
     const bdh_tensor4 slot_v = view4(vl + (v_layer + seq_len * v->stride[2]) * 2, BDH_BF16, 1, 1, B, D, 0, 0,
                                      v->stride[0]);
-    BDH_TRY(bdh_layer_norm_rows2(&cur, &ymlp, &nxt, &slot_v, stream));
+    const bdh_tensor4* out2 = last ? nullptr : &slot_v;
+    if (views_overlap(&nxt, &cur) || (out2 != nullptr && (views_overlap(out2, &nxt) || views_overlap(out2, &cur))))
+      return BDH_ERR_ALIAS;
+    if (few_dec) {
+      BDH_TRY(few_dec_ln_launch(&xy_rows, dec, &cur, &nxt, out2, reinterpret_cast<float*>(w + o.gemm), s));
+    } else {
+      BDH_TRY(bdh_small_gemm(&xy_rows, dec, &ymlp, w + o.gemm, o.end - o.gemm, stream));
+      BDH_TRY(last ? bdh_layer_norm_rows(&cur, &ymlp, &nxt, stream)
+                   : bdh_layer_norm_rows2(&cur, &ymlp, &nxt, &slot_v, stream));
+    }
     cur = nxt;
   }
   return BDH_OK;

@@ -8,6 +8,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "few.h"
 #include "lds_dma.h"
 
 namespace bdh {
@@ -29,9 +30,16 @@ struct FewArgs {
   bf16_t* o;
   int64_t o0, o1, o2;
   int T, M, N, nnb;
+  const float *c, *sn;  // (N) tables of k_few_gemm's RoPE
+  bf16_t* r;
+  int64_t r0, r1;  // (B, nh, 1, N)
 };
 
-template <int K, bool MUL>
+enum : int { kFewRelu = 0, kFewMul = 1, kFewRope = 2 };
+
+// kFewRope (one token a sequence): RoPE of the rounded result goes to a second
+// output, as k_rope8 rounds it; a lane holds whole pairs.
+template <int K, int MODE>
 __global__ __launch_bounds__(256) void k_few_gemm(const FewArgs a) {
   constexpr int S = K / 16;
   const int h = int(blockIdx.x) / a.nnb, nb = int(blockIdx.x) - h * a.nnb;
@@ -48,7 +56,16 @@ __global__ __launch_bounds__(256) void k_few_gemm(const FewArgs a) {
 #pragma unroll
   for (int s = 0; s < S; ++s) yf[s] = *reinterpret_cast<const bf16x8*>(yr + s * 16);
   u32x2 xv[4];
-  if constexpr (MUL) {
+  f32x4 cv[4], sv[4];
+  if constexpr (MODE == kFewRope) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int n = min(n0 + 8 * q + 4 * hl, a.N - 4);
+      cv[q] = *reinterpret_cast<const f32x4*>(a.c + n);
+      sv[q] = *reinterpret_cast<const f32x4*>(a.sn + n);
+    }
+  }
+  if constexpr (MODE == kFewMul) {
 #pragma unroll
     for (int q = 0; q < 4; ++q)
       xv[q] = *reinterpret_cast<const u32x2*>(a.x + b * a.x0 + t * a.x1 + h * a.x2 + min(n0 + 8 * q + 4 * hl, a.N - 4));
@@ -67,7 +84,7 @@ __global__ __launch_bounds__(256) void k_few_gemm(const FewArgs a) {
       v[e] = u != u ? u : fmaxf(u, 0.f);
     }
     uint32_t lo = pack_bf2(v[0], v[1]), hi = pack_bf2(v[2], v[3]);  // relu(s) as bf16, as the tile kernel rounds it
-    if constexpr (MUL) {
+    if constexpr (MODE == kFewMul) {
       const uint32_t x0 = xv[q].x, x1 = xv[q].y;
       lo = pack_bf2(__uint_as_float(x0 << 16) * __uint_as_float(lo << 16),
                     __uint_as_float(x0 & 0xffff0000u) * __uint_as_float(lo & 0xffff0000u));
@@ -75,17 +92,30 @@ __global__ __launch_bounds__(256) void k_few_gemm(const FewArgs a) {
                     __uint_as_float(x1 & 0xffff0000u) * __uint_as_float(hi & 0xffff0000u));
     }
     const int n = n0 + 8 * q + 4 * hl;
-    if (l32 < a.M && n < a.N)
+    if (l32 < a.M && n < a.N) {
       *reinterpret_cast<u32x2*>(a.o + b * a.o0 + t * a.o1 + h * a.o2 + n) = u32x2{lo, hi};
+      if constexpr (MODE == kFewRope) {
+        uint32_t w[2] = {lo, hi};
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          const float x0 = __uint_as_float(w[p] << 16), x1 = __uint_as_float(w[p] & 0xffff0000u);
+          w[p] = pack_bf2(bf_round(x0 * cv[q][2 * p]) + bf_round((-x1) * sv[q][2 * p]),
+                          bf_round(x1 * cv[q][2 * p + 1]) + bf_round(x0 * sv[q][2 * p + 1]));
+        }
+        *reinterpret_cast<u32x2*>(a.r + b * a.r0 + h * a.r1 + n) = u32x2{w[0], w[1]};
+      }
+    }
   }
 }
 
 template <int K> int launch_few(const FewArgs& a, int64_t H, hipStream_t s) {
   const dim3 grid(unsigned(a.nnb * H));
   if (a.x != nullptr)
-    BDH_LAUNCH("k_few_gemm", (k_few_gemm<K, true>), grid, dim3(256), 0, s, a);
+    BDH_LAUNCH("k_few_gemm", (k_few_gemm<K, kFewMul>), grid, dim3(256), 0, s, a);
+  else if (a.r != nullptr)
+    BDH_LAUNCH("k_few_gemm", (k_few_gemm<K, kFewRope>), grid, dim3(256), 0, s, a);
   else
-    BDH_LAUNCH("k_few_gemm", (k_few_gemm<K, false>), grid, dim3(256), 0, s, a);
+    BDH_LAUNCH("k_few_gemm", (k_few_gemm<K, kFewRelu>), grid, dim3(256), 0, s, a);
   return BDH_OK;
 }
 
@@ -198,6 +228,53 @@ __global__ __launch_bounds__(256) void k_few_reduce(const float* __restrict__ pa
   for (int c = 0; c < 4; ++c) o[c] = from_f<TO>(s[c]);
 }
 
+// The same with the layer's end behind it: o = LN(x + LN(sum rounded to bf16))
+// and o2 the same rounded, a workgroup of 16 waves a row (a wave takes every
+// 16th split, eight in flight).  Short, so what it saves is a launch: 8 rows,
+// 256 splits 4.0 us and 3.4 for the row LayerNorm before, 6.0 now.
+struct FewLnArgs {
+  const float* part;
+  int nsplit, M;
+  const float* x;
+  int64_t xs;
+  float* o;
+  int64_t os;
+  bf16_t* o2;  // may be null
+  int64_t o2s;
+};
+__global__ __launch_bounds__(1024) void k_few_ln(const FewLnArgs a) {
+  __shared__ f32x4 sums[16][64];
+  const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
+  const int64_t n = int64_t(a.M) * kFdD, e = int64_t(blockIdx.x) * kFdD + 4 * lane;
+  f32x4 s{0.f, 0.f, 0.f, 0.f};
+  for (int p = g; p < a.nsplit; p += 128) {
+    f32x4 v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const f32x4*>(a.part + int64_t(min(p + 16 * u, a.nsplit - 1)) * n + e);
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (p + 16 * u < a.nsplit) s += v[u];
+  }
+  sums[g][lane] = s;
+  __syncthreads();
+  if (g != 0) return;
+#pragma unroll
+  for (int u = 1; u < 16; ++u) s += sums[u][lane];
+  const float* x = a.x + blockIdx.x * a.xs + 4 * lane;
+  float v[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) v[c] = bf_round(s[c]);
+  ln_row<4>(v, kFdD);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) v[c] += x[c];
+  ln_row<4>(v, kFdD);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    a.o[blockIdx.x * a.os + 4 * lane + c] = v[c];
+    if (a.o2 != nullptr) a.o2[blockIdx.x * a.o2s + 4 * lane + c] = f2bf(v[c]);
+  }
+}
+
 }  // namespace
 
 // Whether the few-row kernel takes a [gated] ReLU product: up to 32 tokens, one
@@ -206,7 +283,7 @@ __global__ __launch_bounds__(256) void k_few_reduce(const float* __restrict__ pa
 bool few_gemm_takes(int64_t M, int64_t K) { return M <= 32 && (K == 64 || K == 128 || K == 256 || K == 512); }
 
 int few_gemm_launch(const bdh_tensor4* y, const bdh_tensor4* wt, const bdh_tensor4* x, const bdh_tensor4* out,
-                    hipStream_t s) {
+                    const FewRope* rope, hipStream_t s) {
   FewArgs a;
   a.y = static_cast<const bf16_t*>(y->data);
   a.y0 = y->stride[0];
@@ -227,6 +304,11 @@ int few_gemm_launch(const bdh_tensor4* y, const bdh_tensor4* wt, const bdh_tenso
   a.M = int(out->size[0] * out->size[1]);
   a.N = int(out->size[3]);
   a.nnb = (a.N + 127) / 128;
+  a.c = rope != nullptr ? rope->cos : nullptr;
+  a.sn = rope != nullptr ? rope->sin : nullptr;
+  a.r = rope != nullptr ? rope->out : nullptr;
+  a.r0 = rope != nullptr ? rope->s0 : 0;
+  a.r1 = rope != nullptr ? rope->s1 : 0;
   const int64_t H = out->size[2];
   if (int64_t(a.nnb) * H >= (int64_t(1) << 31)) return BDH_ERR_SHAPE;
   switch (y->size[3]) {
@@ -250,8 +332,7 @@ bool few_dec_takes(const bdh_tensor4* a, const bdh_tensor4* b) {
 }
 
 // part: 16-byte aligned, K / 128 x M x 256 floats.
-int few_dec_launch(const bdh_tensor4* a, const bdh_tensor4* b, const bdh_tensor4* out, float* part, hipStream_t s) {
-  FewDecArgs g;
+static int few_dec_parts(const bdh_tensor4* a, const bdh_tensor4* b, float* part, FewDecArgs& g, hipStream_t s) {
   g.a = static_cast<const bf16_t*>(a->data);
   g.as = a->stride[2];
   g.b = static_cast<const bf16_t*>(b->data);
@@ -260,6 +341,12 @@ int few_dec_launch(const bdh_tensor4* a, const bdh_tensor4* b, const bdh_tensor4
   g.M = int(a->size[2]);
   g.K = int(a->size[3]);
   BDH_LAUNCH("k_few_dec", k_few_dec, dim3(unsigned(g.K / kFdRows)), dim3(256), 0, s, g);
+  return BDH_OK;
+}
+
+int few_dec_launch(const bdh_tensor4* a, const bdh_tensor4* b, const bdh_tensor4* out, float* part, hipStream_t s) {
+  FewDecArgs g;
+  BDH_TRY(few_dec_parts(a, b, part, g, s));
   const dim3 grid(unsigned(g.M * (kFdD / 64)));
   if (out->dtype == BDH_BF16)
     BDH_LAUNCH("k_few_reduce", k_few_reduce<bf16_t>, grid, dim3(256), 0, s, part, g.K / kFdRows, g.M,
@@ -267,6 +354,25 @@ int few_dec_launch(const bdh_tensor4* a, const bdh_tensor4* b, const bdh_tensor4
   else
     BDH_LAUNCH("k_few_reduce", k_few_reduce<float>, grid, dim3(256), 0, s, part, g.K / kFdRows, g.M,
                static_cast<float*>(out->data), out->stride[2]);
+  return BDH_OK;
+}
+
+// out = LN(x + LN(a b)), x and out fp32 rows, out2 (may be null) bf16 rows.
+int few_dec_ln_launch(const bdh_tensor4* a, const bdh_tensor4* b, const bdh_tensor4* x, const bdh_tensor4* out,
+                      const bdh_tensor4* out2, float* part, hipStream_t s) {
+  FewDecArgs g;
+  BDH_TRY(few_dec_parts(a, b, part, g, s));
+  FewLnArgs l;
+  l.part = part;
+  l.nsplit = g.K / kFdRows;
+  l.M = g.M;
+  l.x = static_cast<const float*>(x->data);
+  l.xs = x->stride[2];
+  l.o = static_cast<float*>(out->data);
+  l.os = out->stride[2];
+  l.o2 = out2 != nullptr ? static_cast<bf16_t*>(out2->data) : nullptr;
+  l.o2s = out2 != nullptr ? out2->stride[2] : 0;
+  BDH_LAUNCH("k_few_ln", k_few_ln, dim3(unsigned(g.M)), dim3(1024), 0, s, l);
   return BDH_OK;
 }
 

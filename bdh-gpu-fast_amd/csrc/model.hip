@@ -11,6 +11,7 @@
 // product is formed in fp32 and rounded once to the output dtype, the same
 // value torch's bf16 / fp32 elementwise product gives.
 #include "common.h"
+#include "few.h"
 #include "lds_dma.h"
 #include "tile_gemm.h"
 
@@ -419,27 +420,6 @@ struct LnArgs {
   int D;
 };
 
-template <int E>
-__device__ __forceinline__ void ln_row(float (&v)[E], int D) {
-  float s = 0.f;
-#pragma unroll
-  for (int e = 0; e < E; ++e) s += v[e];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  const float mean = s / float(D);
-  float q = 0.f;
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    v[e] -= mean;
-    q += v[e] * v[e];
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) q += __shfl_xor(q, off, 64);
-  const float r = rsqrtf(q / float(D) + 1e-5f);
-#pragma unroll
-  for (int e = 0; e < E; ++e) v[e] *= r;
-}
-
 template <typename TX, typename TY, typename TO, int E>
 __global__ __launch_bounds__(256) void k_ln_rows(const LnArgs a) {
   const int64_t row = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
@@ -629,17 +609,13 @@ namespace bdh {
 bool relu_enc_takes(int64_t K, int64_t N);
 int relu_enc_launch(const bdh_tensor4* y, const bdh_tensor4* wt, const bdh_tensor4* x, const bdh_tensor4* out,
                     hipStream_t s);
-bool few_gemm_takes(int64_t M, int64_t K);
-int few_gemm_launch(const bdh_tensor4* y, const bdh_tensor4* wt, const bdh_tensor4* x, const bdh_tensor4* out,
-                    hipStream_t s);
-bool few_dec_takes(const bdh_tensor4* a, const bdh_tensor4* b);
-int few_dec_launch(const bdh_tensor4* a, const bdh_tensor4* b, const bdh_tensor4* out, float* part, hipStream_t s);
 }  // namespace bdh
 
 // out = [x *] relu(y @ wt^T) per head (x null: the ReLU GEMM alone, k_relu_enc
 // where it takes the shape); see k_gated_gemm.
 static int gated_gemm_launch(const bdh_tensor4* y, const bdh_tensor4* wt, const bdh_tensor4* x,
-                             const bdh_tensor4* out, bdh_stream stream) {
+                             const bdh_tensor4* out, bdh_stream stream, const FewRope* rope = nullptr,
+                             bool* roped = nullptr) {
   BDH_TRY(check_view(y));
   BDH_TRY(check_view(wt));
   if (x != nullptr) BDH_TRY(check_view(x));
@@ -702,7 +678,10 @@ static int gated_gemm_launch(const bdh_tensor4* y, const bdh_tensor4* wt, const 
   if (relu_enc_takes(K, N) && (M + 255) / 256 * H >= 128 && ((N - 1) * wt->stride[2] + K) * 2 < (int64_t(1) << 32))
     return relu_enc_launch(y, wt, x, out, static_cast<hipStream_t>(stream));
   // a generate step's few tokens
-  if (few_gemm_takes(M, K)) return few_gemm_launch(y, wt, x, out, static_cast<hipStream_t>(stream));
+  if (few_gemm_takes(M, K)) {
+    if (roped != nullptr) *roped = rope != nullptr;
+    return few_gemm_launch(y, wt, x, out, rope, static_cast<hipStream_t>(stream));
+  }
   if (x != nullptr)
     BDH_LAUNCH("k_gated_gemm", k_gated_gemm<true>, dim3(unsigned(grid)), dim3(512), 0,
                static_cast<hipStream_t>(stream), a);
@@ -723,6 +702,14 @@ extern "C" int bdh_relu_gemm(const bdh_tensor4* y, const bdh_tensor4* wt, const 
                              bdh_stream stream) {
   return gated_gemm_launch(y, wt, nullptr, out, stream);
 }
+
+namespace bdh {
+int relu_gemm_rope(const bdh_tensor4* y, const bdh_tensor4* wt, const bdh_tensor4* out, const FewRope* rope,
+                   bool* roped, bdh_stream stream) {
+  *roped = false;
+  return gated_gemm_launch(y, wt, nullptr, out, stream, rope, roped);
+}
+}  // namespace bdh
 
 extern "C" size_t bdh_small_gemm_workspace(int64_t M, int64_t K, int64_t D) {
   if (M <= 0 || K <= 0 || D <= 0) return 0;

@@ -21,7 +21,8 @@ BF = torch.bfloat16
 
 
 @pytest.mark.parametrize("L,D,nh,mult,B,S", [(1, 64, 2, 4, 1, 1), (2, 128, 4, 5, 3, 7), (3, 256, 4, 32, 65, 70),
-                                             (2, 512, 8, 16, 2, 300), (2, 64, 2, 24, 256, 33)])
+                                             (2, 512, 8, 16, 2, 300), (2, 64, 2, 24, 256, 33),
+                                             (3, 256, 4, 32, 9, 40), (2, 256, 4, 32, 40, 5), (2, 1024, 4, 5, 2, 9)])
 def test_native_step_equals_layer_by_layer(L, D, nh, mult, B, S, monkeypatch):
     torch.manual_seed(0)
     m = H.BDH(H.BDHConfig(n_layer=L, n_embd=D, n_head=nh, mlp_internal_dim_multiplier=mult)).cuda()
