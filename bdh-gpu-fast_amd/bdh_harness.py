@@ -19,8 +19,10 @@ Per layer (x: (B, T, D), LayerNorm without affine, eps 1e-5):
     y_bthn  = relu(einsum("bhtd,hdn->bthn", LN(yKV), encoder_v))
     x       = LN(x + LN((x_bthn * y_bthn).view(B, T, nh*N) @ decoder))
 
-then ``logits = x @ lm_head``.  The dense products run on torch (hipBLASLt);
-RoPE and attention go through the ``kernels`` surface, ``impl="hip"`` for the
+then ``logits = x @ lm_head``.  On the HIP path the dense products of a layer, and
+under bf16 autocast their backward, run on this library's kernels where the
+shapes allow (else on torch's GEMMs), and a one-token step of the packed cache
+is one native call; RoPE and attention go through the ``kernels`` surface, ``impl="hip"`` for the
 gfx950 kernels or ``"eager"`` for the reference's torch semantics.  Under
 ``torch.autocast(dtype=bfloat16)`` the GEMMs run in bf16 and LayerNorm in
 fp32, as in the reference's AMP runs.

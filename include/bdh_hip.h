@@ -133,7 +133,8 @@ int bdh_tril_decode(const bdh_tensor4* q, const bdh_tensor4* k_past,
  * keys: 64-key chunks on both streaming kernels (q and key rows 16-byte
  * aligned, and Dk a multiple of 2048 for bf16 q over bf16 keys, or of 256 /
  * 512 for fp32 / bf16 keys under the fp32-arithmetic kernel), 32-key chunks on
- * the generic kernel (any other operands).  C3's B*H = 256, Dv = 256 fits
+ * the generic kernel (any other operands); smaller chunks, down to 4 keys,
+ * where a call has few workgroups and their partials fit.  C3's B*H = 256, Dv = 256 fits
  * S <= 4096 on the streaming kernels.  The current device must be
  * the tensors' device.  Every call on one GPU shares that GPU's array: calls
  * that overlap in time on one GPU (other streams, other threads) race and must
