@@ -225,6 +225,19 @@ def _padded_rows(B: int, T: int, nh: int, N: int, dtype: torch.dtype, device) ->
     return torch.empty(B, T, nh * N + _XS_PAD, dtype=dtype, device=device).narrow(2, 0, nh * N).unflatten(2, (nh, N))
 
 
+def _token_splits(H: int, M: int, D: int, N: int, a_row: int, b_row: int) -> int:
+    """Parts of the M tokens for ``kernels.tn_gemm`` (a grid of about 192 workgroups of
+    256 x 256 or more), 0 where it does not take the operands.  More parts where the
+    library refuses a part's span; at least 1024 tokens each."""
+    tiles = H * (D // 256) * (N // 256)
+    splits = 1 if tiles >= 192 else 2 if tiles >= 96 else 4 if tiles >= 48 else 8
+    while D % 256 == 0 and M // splits >= 1024:
+        if kernels.tn_gemm_takes(H, M, D, N, a_row, b_row, splits):
+            return splits
+        splits *= 2
+    return 0
+
+
 def _weight_grad(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """a^T b per head, (H, M, D)^T (H, M, N) -> (H, D, N): over enough tokens on the
     library's row-contracting kernel (tiles of 256 x 256, the tokens in splits
@@ -233,9 +246,8 @@ def _weight_grad(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     in torch (128 workgroups each), and 225 for the encoder against 270."""
     H, M, D = a.shape
     N = b.size(2)
-    tiles = H * (D // 256) * (N // 256)
-    splits = 1 if tiles >= 192 else 2 if tiles >= 96 else 4 if tiles >= 48 else 8
-    if D % 256 == 0 and N % 256 == 0 and M % (32 * splits) == 0 and M // splits >= 1024 and M // splits * b.stride(1) < 2**30:
+    splits = _token_splits(H, M, D, N, a.stride(1), b.stride(1))
+    if splits:
         return kernels.tn_gemm(a, b, splits)
     out = torch.empty(H, D, N, dtype=a.dtype, device=a.device)
     for h in range(H):

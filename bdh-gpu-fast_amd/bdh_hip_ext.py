@@ -56,6 +56,7 @@ __all__ = [
     "gated_bwd",
     "relu_bwd_add",
     "tn_gemm",
+    "tn_gemm_takes",
     "small_gemm",
     "decode_step",
     "layer_norm_rows",
@@ -99,6 +100,7 @@ EXPORTED_SYMBOLS = (
     "bdh_gated_bwd",
     "bdh_relu_bwd_add",
     "bdh_tn_gemm",
+    "bdh_tn_gemm_takes",
     "bdh_small_gemm_workspace",
     "bdh_small_gemm",
     "bdh_decode_step_workspace",
@@ -175,6 +177,7 @@ def _load():
         "bdh_gated_bwd": (ctypes.c_int, [P, P, P, P, P, P, P, vp]),
         "bdh_relu_bwd_add": (ctypes.c_int, [P, P, P, P, vp]),
         "bdh_tn_gemm": (ctypes.c_int, [P, P, P, vp]),
+        "bdh_tn_gemm_takes": (ctypes.c_int, [i64] * 7),
         "bdh_small_gemm_workspace": (sz, [i64, i64, i64]),
         "bdh_small_gemm": (ctypes.c_int, [P, P, P, vp, sz, vp]),
         "bdh_decode_step_workspace": (sz, [i64, i64, i64, i64, i64]),
@@ -790,6 +793,11 @@ def relu_bwd_add(a: torch.Tensor, b: torch.Tensor, x: torch.Tensor, out: Optiona
                                    _t4(out), _stream(dev))
     _check(rc, "relu_bwd_add")
     return out
+
+
+def tn_gemm_takes(H: int, K: int, M: int, N: int, a_row: int, b_row: int, splits: int) -> bool:
+    """Whether :func:`tn_gemm` takes a (H, K, M) and b (H, K, N) with these row strides in ``splits`` parts."""
+    return bool(_lib.bdh_tn_gemm_takes(H, K, M, N, a_row, b_row, splits))
 
 
 def tn_gemm(a: torch.Tensor, b: torch.Tensor, splits: int = 1) -> torch.Tensor:

@@ -418,6 +418,18 @@ extern "C" int bdh_relu_bwd_add(const bdh_tensor4* a, const bdh_tensor4* b, cons
   return BDH_OK;
 }
 
+// 32-bit DMA offsets inside one split of one head.
+extern "C" int bdh_tn_gemm_takes(int64_t H, int64_t K, int64_t M, int64_t N, int64_t a_row, int64_t b_row,
+                                 int64_t splits) {
+  const int64_t S = splits, lim = int64_t(1) << 31, sizes[7] = {H, K, M, N, a_row, b_row, S};
+  for (int64_t n : sizes)
+    if (n < 1 || n >= lim) return 0;
+  if (K % (32 * S) != 0 || M % 8 != 0 || N % 256 != 0 || a_row % 8 != 0 || b_row % 8 != 0) return 0;
+  const int64_t ks = K / S;
+  if ((ks * a_row + M) * 2 >= lim || (ks * b_row + N) * 2 >= lim || S * H > (int64_t(1) << 24)) return 0;
+  return S * H * ((M + 255) / 256) <= (lim * 256 - 1) / N ? 1 : 0;  // workgroups of 256 x 256 outputs
+}
+
 extern "C" int bdh_tn_gemm(const bdh_tensor4* a, const bdh_tensor4* b, const bdh_tensor4* out, bdh_stream stream) {
   for (const bdh_tensor4* t : {a, b, out}) BDH_TRY(check_view(t));
   if (a->dtype != BDH_BF16 || b->dtype != BDH_BF16 || out->dtype != BDH_F32) return BDH_ERR_DTYPE;
@@ -426,12 +438,8 @@ extern "C" int bdh_tn_gemm(const bdh_tensor4* a, const bdh_tensor4* b, const bdh
   if (out->size[1] != H || out->size[2] != M || out->size[3] != N) return BDH_ERR_SHAPE;
   if (views_overlap(out, a) || views_overlap(out, b)) return BDH_ERR_ALIAS;
   if (numel4(out) == 0) return BDH_OK;
-  if (K <= 0 || K % (32 * S) != 0 || M % 8 != 0 || N % 256 != 0) return BDH_ERR_SHAPE;
   if (!rows_16(a) || !rows_16(b)) return BDH_ERR_STRIDE;
-  // 32-bit DMA offsets inside one split of one head; 4 rows of out below 2^31 bytes
-  const int64_t ks = K / S, lim = int64_t(1) << 31;
-  if ((ks * a->stride[2] + M) * 2 >= lim || (ks * b->stride[2] + N) * 2 >= lim || out->stride[2] >= (int64_t(1) << 26) ||
-      K >= lim || S * H > (int64_t(1) << 24))
+  if (!bdh_tn_gemm_takes(H, K, M, N, a->stride[2], b->stride[2], S) || out->stride[2] >= (int64_t(1) << 26))
     return BDH_ERR_SHAPE;
   return sy_tn(a, b, out, static_cast<hipStream_t>(stream));
 }

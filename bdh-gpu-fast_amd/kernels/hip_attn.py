@@ -177,6 +177,11 @@ def tn_gemm(a: torch.Tensor, b: torch.Tensor, splits: int = 1) -> torch.Tensor:
     return ext.tn_gemm(a, b, splits)
 
 
+def tn_gemm_takes(H: int, K: int, M: int, N: int, a_row: int, b_row: int, splits: int) -> bool:
+    """Whether :func:`tn_gemm` takes operands of these sizes and row strides (the library's own rule)."""
+    return _require().tn_gemm_takes(H, K, M, N, a_row, b_row, splits)
+
+
 def layer_norm_rows(y: torch.Tensor, x: Optional[torch.Tensor] = None,
                     out_dtype: Optional[torch.dtype] = None, out_bf16: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``LN(y)`` or ``LN(x + LN(y))`` over the last dim on the GPU (bdh.py:565-574, 731-750);
@@ -318,6 +323,7 @@ __all__ = [
     "gated_bwd",
     "relu_bwd_add",
     "tn_gemm",
+    "tn_gemm_takes",
     "relu_gemm",
     "small_gemm",
     "decode_step",

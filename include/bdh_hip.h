@@ -334,7 +334,10 @@ int bdh_gated_bwd(const bdh_tensor4* y, const bdh_tensor4* wt, const bdh_tensor4
  * K, M), b (1, H, K, N) bf16, out (S, H, M, N) fp32, split s the rows
  * [s K/S, (s+1) K/S).  K a multiple of 32 S, M of 8, N of 256, 16-byte rows;
  * one split of one head within 2 GiB.  (Weight gradients: K the tokens.)
+ * bdh_tn_gemm_takes: 1 when it takes these sizes, a_row and b_row the row
+ * strides of a and b in elements (the rule that bdh_tn_gemm itself applies).
  */
+int bdh_tn_gemm_takes(int64_t H, int64_t K, int64_t M, int64_t N, int64_t a_row, int64_t b_row, int64_t splits);
 int bdh_tn_gemm(const bdh_tensor4* a, const bdh_tensor4* b, const bdh_tensor4* out, bdh_stream stream);
 
 /*

@@ -159,3 +159,30 @@ def test_relu_margin_detects_inputs_near_zero():
     q = dict(p, encoder=p["encoder"].copy())
     q["encoder"][0, :, 3] = 0.0  # one latent column of head 0 is identically zero
     assert M.relu_margin(q, idx) == 0.0
+
+
+@pytest.mark.parametrize("D,width", [(256, 32768), (512, 32768), (512, 65536), (256, 65536)])
+def test_weight_gradient_takes_only_what_the_library_takes(D, width):
+    """The split rule of the training layer's weight gradients against the entry point's own
+    host checks, over the row counts at the library's span limit: (rows + 1 row's end) * 2
+    bytes below 2^31 for one split.  Refused calls return before any launch."""
+    import bdh_hip_ext as ext
+
+    row = width + H._XS_PAD
+
+    def entry(M, splits):  # bdh_tn_gemm's answer to a call that it refuses
+        t = [ext._pack4(p, *n, *s, 1, dt, 0) for p, n, s, dt in (
+            (0x100000, (1, 1, M, D), (0, 0, D), ext.BDH_BF16), (0x200000000000, (1, 1, M, width), (0, 0, row), ext.BDH_BF16),
+            (0x300000000000, (splits, 1, D, width), (D * width, D * width, width), ext.BDH_F32))]
+        return ext._lib.bdh_tn_gemm(*t, None)
+
+    most = max(M for M in range(32, 2**30 // row + 64, 32) if (M * row + width) * 2 < 2**31)
+    assert ext.tn_gemm_takes(1, most, D, width, D, row, 1)
+    # the spans between this limit and one without the row's end: B * T one 32-row step or more over
+    for M in (most + 32, most + 64):
+        assert not ext.tn_gemm_takes(1, M, D, width, D, row, 1) and entry(M, 1) == 1  # BDH_ERR_SHAPE
+    for M in [*range(1024, 4 * most, 1504), *range(most - 64, most + 96, 16), *range(2 * most - 128, 2 * most + 128, 32)]:
+        s = H._token_splits(1, M, D, width, D, row)
+        assert s == 0 or ext.tn_gemm_takes(1, M, D, width, D, row, s)
+        assert s == 0 or (M % (32 * s) == 0 and (M // s * row + width) * 2 < 2**31 and M // s >= 1024)
+    assert H._token_splits(1, most + 32 - (most + 32) % 64 + 64, D, width, D, row) == 2  # two parts fit
