@@ -365,7 +365,7 @@ def _steps_native(x: torch.Tensor, cache, prep: dict) -> bool:
     over one layer's V rows), few enough rows for the split-K decoder."""
     B, T, D = x.shape
     N = prep["enc_t"].size(1)
-    return (isinstance(cache, KVCache) and T == 1 and cache.seq_len > 0 and cache.dtype == torch.bfloat16
+    return (type(cache) is KVCache and T == 1 and cache.seq_len > 0 and cache.dtype == torch.bfloat16
             and x.dtype == torch.float32 and prep["enc_t"].dtype == torch.bfloat16 and _ln_rows_ok(x)
             and N % 8 == 0 and N <= 16320 and 0 < B <= 256 and B * cache.capacity * D * 2 <= 2**32)
 
@@ -420,6 +420,13 @@ class BDH(nn.Module):
         return prep
 
     # ----------------------------------------------------------- attention
+    def _own_attention(self) -> bool:
+        """Whether a layer's attention is this class's, over the ``kernels`` operators as they
+        were imported: what the fused training layer and the native step stand in for.  A
+        subclass's ``_attention`` or a replaced operator is run, not passed by."""
+        return (getattr(self._attention, "__func__", None) is _ATTENTION
+                and all(getattr(kernels, n) is f for n, f in _ATTN_OPS.items()))
+
     def _attention_managed(self, level, x_sparse, v_tok, cache: CacheManager, impl, cos_sin):
         """One layer against a ``CacheManager`` in bdh.py's order: reserve
         before get_past and RoPE into the slot when the storage dtype is the
@@ -513,6 +520,7 @@ class BDH(nn.Module):
         fast = impl == "hip" and not torch.is_grad_enabled()
         x = _ln(self.embed(idx))  # (B, T, D)
         fused = impl == "hip" and torch.is_grad_enabled() and cache is None and _trains_fused(x, self.encoder)
+        fused = fused and self._own_attention()
         if fused:  # (laid out anew for every forward: a training step changes them)
             with torch.no_grad():
                 enc_t, encv_t = (w.transpose(1, 2).to(torch.bfloat16, memory_format=torch.contiguous_format)
@@ -525,7 +533,7 @@ class BDH(nn.Module):
         # cache's V slot when the cache stores bf16, so a decode step makes neither a
         # cast nor a slot copy.  The bits are those of x.to(bf16).
         xb = None
-        native = fast and _steps_native(x, cache, prep)
+        native = fast and _steps_native(x, cache, prep) and self._own_attention()
         if native:
             cache.slot(0, 1)[1].copy_(x.unsqueeze(1))
             x = kernels.decode_step(x.view(B, -1), prep["enc_t"], prep["encv_t"], prep["dec"], *cos_sin, cache.kr,
@@ -646,5 +654,8 @@ class BDH(nn.Module):
                 logits, _ = self(nxt, cache=cache, impl=impl, last_only=True)
         return out
 
+
+_ATTENTION = BDH._attention
+_ATTN_OPS = {n: getattr(kernels, n) for n in ("bdh_attn_rope", "bdh_attn_decode", "bdh_rope_rotate")}
 
 __all__ = ["BDHConfig", "BDH", "KVCache"]

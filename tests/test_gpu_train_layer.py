@@ -129,3 +129,58 @@ def test_row_contraction_matches_float64(nh, K, M, N, splits):
     assert got.dtype == torch.float32 and _rel(got, want) <= 1e-5
     with pytest.raises(RuntimeError):
         ext.tn_gemm(a, b, splits + 4)  # K is not a multiple of 32 (splits + 4)
+
+
+def _tiny():
+    torch.manual_seed(0)
+    return H.BDHConfig(n_layer=2, n_embd=64, n_head=2, mlp_internal_dim_multiplier=8)
+
+
+def _train(m, idx):
+    with torch.autocast("cuda", dtype=BF):
+        loss = m(idx, idx.roll(-1, 1), impl="hip")[1]
+    loss.backward()
+    return {n: p.grad.clone() for n, p in m.named_parameters()}
+
+
+def test_a_replaced_operator_or_attention_is_run(monkeypatch):
+    """The fused training layer and the native generate step stand in for the class's own
+    attention over the surface's own operators, and for nothing else."""
+    calls = []
+
+    class Own(H.BDH):
+        def _attention(self, *a):
+            calls.append("attention")
+            return 0.5 * super()._attention(*a)
+
+    cfg = _tiny()
+    m = H.BDH(cfg).cuda()
+    own = Own(cfg).cuda()
+    own.load_state_dict(m.state_dict())
+    idx = torch.randint(0, 256, (2, 33), device="cuda")
+    plain = _train(m, idx)
+    _train(own, idx)
+    assert calls == ["attention"] * cfg.n_layer
+    # a generate step after the prompt
+    del calls[:]
+    own.generate(idx, 1, cache_dtype=BF, amp_dtype=BF, impl="hip")
+    assert calls == ["attention"] * (2 * cfg.n_layer)
+
+    rope = kernels.bdh_attn_rope
+
+    def fp32(x, v, freqs, rope_start=0, out_kr=None, impl=None):
+        calls.append("rope")
+        return rope(x.float(), v.float(), freqs, rope_start, impl=impl).to(x.dtype)
+
+    del calls[:]
+    monkeypatch.setattr(kernels, "bdh_attn_rope", fp32)
+    m.zero_grad(set_to_none=True)
+    assert any(not torch.equal(g, plain[n]) for n, g in _train(m, idx).items())
+    assert calls == ["rope"] * cfg.n_layer
+
+    monkeypatch.undo()
+    decode = kernels.bdh_attn_decode
+    monkeypatch.setattr(kernels, "bdh_attn_decode", lambda *a, **k: calls.append("decode") or decode(*a, **k))
+    del calls[:]
+    m.generate(idx, 1, cache_dtype=BF, amp_dtype=BF, impl="hip")
+    assert calls == ["decode"] * cfg.n_layer
