@@ -143,7 +143,7 @@ __device__ __forceinline__ void diag_item(char* lds, int* flag, L& la, L& lb, in
 #pragma unroll
   for (int n = 0; n < 9; ++n)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) bad |= !(acc[n][r] == acc[n][r]);
+    for (int r = 0; r < 16; ++r) bad |= f32_spoiled(acc[n][r]);
   if (f32_any(bad, flag)) run(std::true_type{});
   if constexpr (ONE) {  // the second half's sums through LDS, three blocks at a time
     f32x4* x = reinterpret_cast<f32x4*>(lds) + ((wave & 3) * 3 * 4 * 64 + lane);
@@ -260,7 +260,7 @@ __global__ __launch_bounds__(512, 2) void k_f32_scores(F32ScoresArgs a) {
     f32x16 acc[4][2];
     f32_zero<F32Big>(acc);
     f32_loop<false, F32Big>(f32_lds, la, lb, kb, ke, wm, wn, lane, acc, off);
-    if (f32_any(f32_has_nan(acc), &flag)) {
+    if (f32_any(f32_spoiled(acc), &flag)) {
       f32_zero<F32Big>(acc);
       f32_loop<true, F32Big>(f32_lds, la, lb, kb, ke, wm, wn, lane, acc, off);
     }
@@ -353,7 +353,7 @@ __global__ __launch_bounds__(256, 2) void k_f32_scores_mid(F32ScoresArgs a) {
     }
   };
   run(std::false_type{});
-  if (f32_any(f32_has_nan(acc), &flag)) run(std::true_type{});
+  if (f32_any(f32_spoiled(acc), &flag)) run(std::true_type{});
   float* tile = a.m + split * a.split_stride + int64_t(slab) * kTileElems;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -426,7 +426,7 @@ __global__ __launch_bounds__(256, 2) void k_f32_sv(F32SvArgs a) {
   f32x16 acc[1][2];
   f32_zero<F32Flat>(acc);
   f32_loop<false, F32Flat>(f32_lds, la, lb, 0, ke, wm, wn, lane, acc);
-  if (f32_any(f32_has_nan(acc), &flag)) {
+  if (f32_any(f32_spoiled(acc), &flag)) {
     f32_zero<F32Flat>(acc);
     f32_loop<true, F32Flat>(f32_lds, la, lb, 0, ke, wm, wn, lane, acc);
   }
@@ -491,7 +491,7 @@ __global__ __launch_bounds__(256, 2) void k_f32_dv(F32DvArgs a) {
     }
   };
   run(std::false_type{});
-  if (f32_any(f32_has_nan(acc), &flag)) run(std::true_type{});
+  if (f32_any(f32_spoiled(acc), &flag)) run(std::true_type{});
   TO* o = static_cast<TO*>(const_cast<void*>(a.o.p)) + b * a.o.s0 + hv * a.o.s1;
   float* pp = a.part + (int64_t(piece) * gridDim.z + bv) * a.T * a.Dv;
 #pragma unroll
@@ -567,7 +567,7 @@ __global__ __launch_bounds__(256, 2) void k_f32_g(F32GArgs a) {
   f32x16 acc[2][2];
   f32_zero<F32Mid>(acc);
   f32_loop<false, F32Mid>(f32_lds, la, lb, 0, a.Dv, wm, wn, lane, acc);
-  if (f32_any(f32_has_nan(acc), &flag)) {
+  if (f32_any(f32_spoiled(acc), &flag)) {
     f32_zero<F32Mid>(acc);
     f32_loop<true, F32Mid>(f32_lds, la, lb, 0, a.Dv, wm, wn, lane, acc);
   }
@@ -632,7 +632,7 @@ __global__ __launch_bounds__(C::NT, 2) void k_f32_dq(F32DqArgs a) {
   f32x16 acc[C::MI][C::NJ];
   f32_zero<C>(acc);
   f32_loop<false, C>(f32_lds, la, lb, kb, ke, wm, wn, lane, acc);
-  if (f32_any(f32_has_nan(acc), &flag)) {
+  if (f32_any(f32_spoiled(acc), &flag)) {
     f32_zero<C>(acc);
     f32_loop<true, C>(f32_lds, la, lb, kb, ke, wm, wn, lane, acc);
   }

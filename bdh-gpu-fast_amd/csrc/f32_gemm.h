@@ -15,9 +15,11 @@
 // leave 2.7 times the fp32 rate.
 //
 // Infinities, NaN and values that bf16 rounding would push to infinity make
-// the lower planes NaN, so every affected sum is NaN: a workgroup that finds
-// a NaN among its sums computes its tile once more with the fp32 matrix
-// instruction (EXACT), which gives what plain fp32 arithmetic gives.
+// the lower planes NaN, so every affected sum is NaN; a product near fp32's
+// largest value may overflow in its leading planes alone and leave an
+// infinity.  A workgroup that finds a sum that is not finite computes its tile
+// once more with the fp32 matrix instruction (EXACT), which gives what plain
+// fp32 arithmetic gives.
 //
 // LDS: per stage of 16 k and operand, three planes of [row][16] bf16 (32-byte
 // rows, so a 32-row MFMA fragment is one contiguous 1 KB read without bank
@@ -150,14 +152,17 @@ template <class C> __device__ __forceinline__ void f32_zero(f32x16 (&acc)[C::MI]
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 }
 
-template <int M, int N> __device__ __forceinline__ bool f32_has_nan(const f32x16 (&acc)[M][N]) {
+// A sum that the bf16 planes may have spoiled: NaN, or an infinity that fp32
+// products need not reach.
+__device__ __forceinline__ bool f32_spoiled(float v) { return !(__builtin_fabsf(v) <= 3.40282347e+38f); }
+template <int M, int N> __device__ __forceinline__ bool f32_spoiled(const f32x16 (&acc)[M][N]) {
   bool bad = false;
 #pragma unroll
   for (int i = 0; i < M; ++i)
 #pragma unroll
     for (int j = 0; j < N; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) bad |= !(acc[i][j][r] == acc[i][j][r]);
+      for (int r = 0; r < 16; ++r) bad |= f32_spoiled(acc[i][j][r]);
   return bad;
 }
 

@@ -129,3 +129,23 @@ def test_values_bf16_cannot_hold_take_fp32_products(T, bad):
     assert torch.equal(torch.isfinite(dx.cpu()), torch.isfinite(wdx))
     okx = torch.isfinite(wdx)
     assert _rel(dx.cpu()[okx], wdx[okx]) <= 1e-5
+
+
+@pytest.mark.parametrize("T", [100, 300, 520])
+def test_products_that_only_their_leading_planes_overflow(T):
+    """1.8425e19^2 = 3.39e38 is finite in fp32; its leading bf16 planes are 2^64 each."""
+    N, D, big = 64, 32, 1.8425e19
+    x = _latent(1, 2, T, N, seed=10) * 1e-3
+    x[..., 3] = 0
+    x[0, :, [0, T - 1], 3] = big
+    v = _randn(1, 1, T, D, seed=11) * 1e-3
+    got = ext.tril_score_v(x.cuda(), x.cuda(), v.cuda()).cpu()
+    assert torch.isfinite(got).all() and _rel(got, _attn64(x.double(), x.double(), v.double())) <= TOL
+    # G = dO V^T of the backward, and M^T dO and G x with both factors large
+    do, w = torch.zeros(1, 2, T, D), torch.zeros(1, 1, T, D)
+    do[0, :, T - 1, 0] = w[0, 0, 0, 0] = big
+    y = _latent(1, 2, T, N, seed=12) * 1e-3
+    dx, _, dv = ext.tril_score_v_bwd(y.cuda(), None, w.cuda(), do.cuda())
+    y64, w64 = y.double().requires_grad_(True), w.double().requires_grad_(True)
+    wdx, wdv = torch.autograd.grad(_attn64(y64, y64, w64), (y64, w64), do.double())
+    assert torch.isfinite(dx).all() and _rel(dx, wdx) <= TOL and _rel(dv, wdv) <= TOL
