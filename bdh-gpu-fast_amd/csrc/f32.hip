@@ -23,6 +23,7 @@ namespace bdh {
 namespace {
 
 // ------------------------------------------------------------------ scores
+constexpr int kF32ScoresValu = 5;  // (f32_loop's V)
 enum : int { kF32Full = 0, kF32Diag2 = 1, kF32Diag1 = 2 };
 
 struct F32ScoresArgs {
@@ -118,7 +119,7 @@ __device__ __forceinline__ void diag_loop(char* lds, L& la, L& lb, int kb, int k
     diag_mma<EXACT, P>(lds + cur * F32Big::kBuf + mine, lane, acc);
     la.template store<EXACT>(nx, kb + s1 * STEP);
     lb.template store<EXACT>(nx + F32Big::kBufA, kb + s1 * STEP + OFF);
-    if constexpr (!EXACT) f32_interleave<54, kF32Valu>();
+    if constexpr (!EXACT) f32_interleave<54, kF32ScoresValu>();
     la.load(kb + s2 * STEP);
     lb.load(kb + s2 * STEP + OFF);
     f32_barrier();
@@ -139,12 +140,11 @@ __device__ __forceinline__ void diag_item(char* lds, int* flag, L& la, L& lb, in
     diag_loop<decltype(exact)::value, ONE, P>(lds, la, lb, kb, ke, off, half * F32Big::kBufA, lane, acc);
   };
   run(std::false_type{});
-  bool bad = false;
-#pragma unroll
-  for (int n = 0; n < 9; ++n)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) bad |= f32_spoiled(acc[n][r]);
-  if (f32_any(bad, flag)) run(std::true_type{});
+  float us = kF32Unscale;
+  if (f32_any(f32_spoiled(acc), flag)) {
+    run(std::true_type{});
+    us = 1.f;
+  }
   if constexpr (ONE) {  // the second half's sums through LDS, three blocks at a time
     f32x4* x = reinterpret_cast<f32x4*>(lds) + ((wave & 3) * 3 * 4 * 64 + lane);
 #pragma unroll
@@ -177,7 +177,7 @@ __device__ __forceinline__ void diag_item(char* lds, int* flag, L& la, L& lb, in
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int row = f32_row(rb, lane, r), col = f32_col(cb, lane);
-      tile[row * 256 + col] = (row > col && r0 + row < T) ? acc[n][r] : 0.f;
+      tile[row * 256 + col] = (row > col && r0 + row < T) ? acc[n][r] * us : 0.f;
     }
   }
 }
@@ -195,7 +195,7 @@ __device__ __forceinline__ void diag_waves(char* lds, int* flag, L& la, L& lb, i
 
 // 256 x 256 tiles.  Bound by the matrix cores beside the staging's VALU work
 // (split, and RoPE's sine and cosine): per 16 k a wave issues 48 MFMAs of 32
-// clocks (54 on a diagonal pair) and about 165 VALU instructions, so the tile
+// clocks (54 on a diagonal pair) and about 180 VALU instructions, so the tile
 // is as large as two waves per SIMD allow, and the two diagonal tiles of a
 // pair share a workgroup (with Q = K each needs its rows once).  B = 8, nh =
 // 4, T = 512, N = 8192 with RoPE: 350-390 us by box (the fp32 matrix
@@ -259,10 +259,12 @@ __global__ __launch_bounds__(512, 2) void k_f32_scores(F32ScoresArgs a) {
     const int wm = wave >> 2, wn = wave & 3;
     f32x16 acc[4][2];
     f32_zero<F32Big>(acc);
-    f32_loop<false, F32Big>(f32_lds, la, lb, kb, ke, wm, wn, lane, acc, off);
+    f32_loop<false, F32Big, false, true, kF32ScoresValu>(f32_lds, la, lb, kb, ke, wm, wn, lane, acc, off);
+    float us = kF32Unscale;
     if (f32_any(f32_spoiled(acc), &flag)) {
       f32_zero<F32Big>(acc);
       f32_loop<true, F32Big>(f32_lds, la, lb, kb, ke, wm, wn, lane, acc, off);
+      us = 1.f;
     }
     float* tile = out + int64_t(f32_tile_index(ta, tb) - a.t0) * 65536;
 #pragma unroll
@@ -273,7 +275,7 @@ __global__ __launch_bounds__(512, 2) void k_f32_scores(F32ScoresArgs a) {
         for (int r = 0; r < 16; ++r) {
           const int row = f32_row(wm * 4 + i, lane, r), col = f32_col(wn * 2 + j, lane);
           const int gi = ta * 256 + row;
-          tile[row * 256 + col] = (tb * 256 + col < gi && gi < a.T) ? acc[i][j][r] : 0.f;
+          tile[row * 256 + col] = (tb * 256 + col < gi && gi < a.T) ? acc[i][j][r] * us : 0.f;
         }
     return;
   }
@@ -353,7 +355,11 @@ __global__ __launch_bounds__(256, 2) void k_f32_scores_mid(F32ScoresArgs a) {
     }
   };
   run(std::false_type{});
-  if (f32_any(f32_spoiled(acc), &flag)) run(std::true_type{});
+  float us = kF32Unscale;
+  if (f32_any(f32_spoiled(acc), &flag)) {
+    run(std::true_type{});
+    us = 1.f;
+  }
   float* tile = a.m + split * a.split_stride + int64_t(slab) * kTileElems;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -362,7 +368,7 @@ __global__ __launch_bounds__(256, 2) void k_f32_scores_mid(F32ScoresArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int row = f32_row(wm * 2 + i, lane, r), col = f32_col(wn * 2 + j, lane);
-        tile[row * 128 + col] = (row > col && row < a.T) ? acc[i][j][r] : 0.f;
+        tile[row * 128 + col] = (row > col && row < a.T) ? acc[i][j][r] * us : 0.f;
       }
 }
 
@@ -426,9 +432,11 @@ __global__ __launch_bounds__(256, 2) void k_f32_sv(F32SvArgs a) {
   f32x16 acc[1][2];
   f32_zero<F32Flat>(acc);
   f32_loop<false, F32Flat>(f32_lds, la, lb, 0, ke, wm, wn, lane, acc);
+  float us = kF32Unscale;
   if (f32_any(f32_spoiled(acc), &flag)) {
     f32_zero<F32Flat>(acc);
     f32_loop<true, F32Flat>(f32_lds, la, lb, 0, ke, wm, wn, lane, acc);
+    us = 1.f;
   }
   TO* o = static_cast<TO*>(const_cast<void*>(a.o.p)) + b * a.o.s0 + h * a.o.s1;
 #pragma unroll
@@ -436,7 +444,7 @@ __global__ __launch_bounds__(256, 2) void k_f32_sv(F32SvArgs a) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int gi = R * 64 + f32_row(wm, lane, r), gd = Dt * 128 + f32_col(wn * 2 + j, lane);
-      if (gi >= a.past && gi < a.T && gd < a.Dv) o[int64_t(gi - a.past) * a.o.s2 + gd] = from_f<TO>(acc[0][j][r]);
+      if (gi >= a.past && gi < a.T && gd < a.Dv) o[int64_t(gi - a.past) * a.o.s2 + gd] = from_f<TO>(acc[0][j][r] * us);
     }
 }
 
@@ -491,7 +499,11 @@ __global__ __launch_bounds__(256, 2) void k_f32_dv(F32DvArgs a) {
     }
   };
   run(std::false_type{});
-  if (f32_any(f32_spoiled(acc), &flag)) run(std::true_type{});
+  float us = kF32Unscale;
+  if (f32_any(f32_spoiled(acc), &flag)) {
+    run(std::true_type{});
+    us = 1.f;
+  }
   TO* o = static_cast<TO*>(const_cast<void*>(a.o.p)) + b * a.o.s0 + hv * a.o.s1;
   float* pp = a.part + (int64_t(piece) * gridDim.z + bv) * a.T * a.Dv;
 #pragma unroll
@@ -501,9 +513,9 @@ __global__ __launch_bounds__(256, 2) void k_f32_dv(F32DvArgs a) {
       const int gj = R * 64 + f32_row(wm, lane, r), gd = Dt * 128 + f32_col(wn * 2 + j, lane);
       if (gj < a.T && gd < a.Dv) {
         if (a.parts > 1)
-          pp[int64_t(gj) * a.Dv + gd] = acc[0][j][r];
+          pp[int64_t(gj) * a.Dv + gd] = acc[0][j][r] * us;
         else
-          o[int64_t(gj) * a.o.s2 + gd] = from_f<TO>(acc[0][j][r]);
+          o[int64_t(gj) * a.o.s2 + gd] = from_f<TO>(acc[0][j][r] * us);
       }
     }
 }
@@ -566,10 +578,12 @@ __global__ __launch_bounds__(256, 2) void k_f32_g(F32GArgs a) {
   const int wm = wave >> 1, wn = wave & 1;
   f32x16 acc[2][2];
   f32_zero<F32Mid>(acc);
-  f32_loop<false, F32Mid>(f32_lds, la, lb, 0, a.Dv, wm, wn, lane, acc);
+  f32_loop<false, F32Mid, false, true, 4>(f32_lds, la, lb, 0, a.Dv, wm, wn, lane, acc);
+  float us = kF32Unscale;
   if (f32_any(f32_spoiled(acc), &flag)) {
     f32_zero<F32Mid>(acc);
     f32_loop<true, F32Mid>(f32_lds, la, lb, 0, a.Dv, wm, wn, lane, acc);
+    us = 1.f;
   }
   float* g = a.g + int64_t(slab) * a.tpad * a.tpad;
 #pragma unroll
@@ -580,7 +594,7 @@ __global__ __launch_bounds__(256, 2) void k_f32_g(F32GArgs a) {
       for (int r = 0; r < 16; ++r) {
         const int gi = ti * 128 + f32_row(wm * 2 + i, lane, r), gj = tj * 128 + f32_col(wn * 2 + j, lane);
         if (gj > gi) continue;
-        const float val = gj == gi ? 0.f : acc[i][j][r];
+        const float val = gj == gi ? 0.f : acc[i][j][r] * us;
         g[int64_t(gi) * a.tpad + gj] = val;
         g[int64_t(gj) * a.tpad + gi] = val;
       }
@@ -631,10 +645,12 @@ __global__ __launch_bounds__(C::NT, 2) void k_f32_dq(F32DqArgs a) {
   const int wm = wave / C::WN, wn = wave % C::WN;
   f32x16 acc[C::MI][C::NJ];
   f32_zero<C>(acc);
-  f32_loop<false, C>(f32_lds, la, lb, kb, ke, wm, wn, lane, acc);
+  f32_loop<false, C, false, true, 4>(f32_lds, la, lb, kb, ke, wm, wn, lane, acc);
+  float us = kF32Unscale;
   if (f32_any(f32_spoiled(acc), &flag)) {
     f32_zero<C>(acc);
     f32_loop<true, C>(f32_lds, la, lb, kb, ke, wm, wn, lane, acc);
+    us = 1.f;
   }
   TO* o = static_cast<TO*>(const_cast<void*>(a.o.p)) + b * a.o.s0 + h * a.o.s1;
   const bool even = (lane & 1) == 0;
@@ -648,7 +664,7 @@ __global__ __launch_bounds__(C::NT, 2) void k_f32_dq(F32DqArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int gi = ti * C::TM + f32_row(wm * C::MI + i, lane, r);
-        float val = acc[i][j][r];
+        float val = acc[i][j][r] * us;
         if constexpr (ROPE) {
           // column pairs (2m, 2m+1) sit in lanes (2l, 2l+1): swap partners, rotate back
           const float other = __shfl_xor(val, 1, 64);

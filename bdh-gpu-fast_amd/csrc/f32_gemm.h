@@ -1,23 +1,26 @@
 // fp32 tile products on the bf16 matrix cores of gfx950.
 //
-// An fp32 value is the exact sum of three bf16 values (8 significant bits
-// each, every step rounded to nearest even):
-//   p1 = bf16(a), p2 = bf16(a - p1), p3 = bf16(a - p1 - p2).
+// An fp32 value times 2^16 is the exact sum of three bf16 values (8 significant
+// bits each, every step rounded to nearest even):
+//   a' = 2^16 a, p1 = bf16(a'), p2 = bf16(a' - p1), p3 = bf16(a' - p1 - p2).
+// The factor lifts fp32's last bit (2^-149) to bf16's (2^-133): without it the
+// lower planes of values below 2^-110 fall short (2.5e-6 of the result at
+// 2^-116, 6e-4 at 2^-124).  The sums are 2^32 times theirs.
 // A product keeps six of the nine plane products,
-//   a b = p1 q1 + (p1 q2 + p2 q1) + (p1 q3 + p2 q2 + p3 q1) + O(2^-26 |a b|),
+//   a' b' = p1 q1 + (p1 q2 + p2 q1) + (p1 q3 + p2 q2 + p3 q1) + d,
 // all exact in fp32, accumulated in fp32 by v_mfma_f32_32x32x16_bf16.  What is
-// dropped is below half an fp32 ulp of each product; the sum has six
-// accumulator updates per 16 k against eight of v_mfma_f32_32x32x2_f32, so
-// its error against 64 bits is no larger (measured at the call sites).
+// dropped, d = p2 q3 + p3 q2 + p3 q3, is at most about 2^-24 of the product
+// (|p2| <= 2^-8 |a'|, |p3| <= 2^-17 |a'|); the sum has six accumulator updates
+// per 16 k against eight of v_mfma_f32_32x32x2_f32.  Error against 64 bits, the
+// fp32 instruction before and this: 4.66e-7 -> 4.06e-7 at B = 8, nh = 4, T = 512,
+// N = 8192 (forward), no larger in any shape measured.
 //
 // Why: the fp32 matrix rate of this chip is 1/16 of its bf16 rate (157
 // TFLOP/s against 2.5 PFLOP/s); six bf16 products for one fp32 product still
 // leave 2.7 times the fp32 rate.
 //
-// Infinities, NaN and values that bf16 rounding would push to infinity make
-// the lower planes NaN, so every affected sum is NaN; a product near fp32's
-// largest value may overflow in its leading planes alone and leave an
-// infinity.  A workgroup that finds a sum that is not finite computes its tile
+// Infinities, NaN and values from about 2^112 on make the lower planes NaN, so
+// every affected sum is NaN; a sum from 2^96 on is an infinity.  A workgroup that finds a sum that is not finite computes its tile
 // once more with the fp32 matrix instruction (EXACT), which gives what plain
 // fp32 arithmetic gives.
 //
@@ -35,6 +38,7 @@
 namespace bdh {
 
 constexpr int kFK = 16;     // k per stage
+constexpr float kF32Scale = 65536.f, kF32Unscale = 1.f / (65536.f * 65536.f);  // of an operand; of a sum
 constexpr int kF32Valu = 3;  // VALU instructions per MFMA of a stage (f32_interleave)
 
 // Waves WM x WN, each owning MI x NJ blocks of 32 x 32.
@@ -51,11 +55,11 @@ typedef F32Cfg<2, 4, 4, 2> F32Big;   // 256 x 256, 8 waves, 96 KB
 typedef F32Cfg<2, 2, 2, 2> F32Mid;   // 128 x 128, 4 waves, 48 KB
 typedef F32Cfg<2, 2, 1, 2> F32Flat;  // 64 x 128, 4 waves, 36 KB
 
-// The three planes of four consecutive k (8 bytes each).
+// The three planes of four consecutive k (8 bytes each), times kF32Scale.
 __device__ __forceinline__ void f32_split4(const float (&f)[4], u32x2 (&p)[3]) {
   float r[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) r[e] = f[e];
+  for (int e = 0; e < 4; ++e) r[e] = f[e] * kF32Scale;
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
     const uint32_t lo = pack_bf2(r[0], r[1]), hi = pack_bf2(r[2], r[3]);
@@ -152,18 +156,26 @@ template <class C> __device__ __forceinline__ void f32_zero(f32x16 (&acc)[C::MI]
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 }
 
-// A sum that the bf16 planes may have spoiled: NaN, or an infinity that fp32
+// Sums that the bf16 planes may have spoiled: NaN, or an infinity that fp32
 // products need not reach.
-__device__ __forceinline__ bool f32_spoiled(float v) { return !(__builtin_fabsf(v) <= 3.40282347e+38f); }
+template <int N> __device__ __forceinline__ float f32_largest(const f32x16 (&acc)[N]) {
+  float m = 0.f;  // the largest magnitude; NaN if there is one (v_maximum3_f32, two sums each)
+#pragma unroll
+  for (int n = 0; n < N; ++n)
+#pragma unroll
+    for (int r = 0; r < 16; r += 2)
+      m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, __builtin_fabsf(acc[n][r])),
+                                        __builtin_fabsf(acc[n][r + 1]));
+  return m;
+}
+template <int N> __device__ __forceinline__ bool f32_spoiled(const f32x16 (&acc)[N]) {
+  return !(f32_largest(acc) <= 3.40282347e+38f);
+}
 template <int M, int N> __device__ __forceinline__ bool f32_spoiled(const f32x16 (&acc)[M][N]) {
-  bool bad = false;
+  float m = 0.f;
 #pragma unroll
-  for (int i = 0; i < M; ++i)
-#pragma unroll
-    for (int j = 0; j < N; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) bad |= f32_spoiled(acc[i][j][r]);
-  return bad;
+  for (int i = 0; i < M; ++i) m = __builtin_elementwise_maximum(m, f32_largest(acc[i]));
+  return !(m <= 3.40282347e+38f);
 }
 
 // Among the MFMAs of a stage, the VALU work of staging the next one: without
@@ -181,8 +193,11 @@ template <int N, int V> __device__ __forceinline__ void f32_interleave() {
 // stage wrap round (into a buffer that nobody reads), so every stage runs the
 // same code.  off: the stage to begin with (the k order of the sum).  Safe to call again after itself (its first barrier waits for
 // the readers of the buffers).  BISA: the A rows are the B operand too.  ACT:
-// whether this wave multiplies (it stages either way).
-template <bool EXACT, class C, bool BISA = false, bool ACT = true, class LA, class LB>
+// whether this wave multiplies (it stages either way).  V: VALU instructions
+// per MFMA, by kernel (2, 3, 4, 5 at B = 2, nh = 4, T = 387, N = 8192, in us:
+// scores 108, 106, 107, 103; score x V 26.0, 25.7, 28.1, 28.4; G 28.0, 28.3,
+// 26.4, 27.7; dQ 185, 187, 173, 187).
+template <bool EXACT, class C, bool BISA = false, bool ACT = true, int V = kF32Valu, class LA, class LB>
 __device__ __forceinline__ void f32_loop(char* lds, LA& la, LB& lb, int kb, int ke, int wm, int wn, int lane,
                                          f32x16 (&acc)[C::MI][C::NJ], int off = 0) {
   if (kb >= ke) return;
@@ -206,7 +221,7 @@ __device__ __forceinline__ void f32_loop(char* lds, LA& la, LB& lb, int kb, int 
     if constexpr (ACT) f32_mma<EXACT, C>(a, BISA ? a : a + C::kBufA, wm, wn, lane, acc);
     la.template store<EXACT>(nx, kb + s1 * kFK);
     if constexpr (!BISA) lb.template store<EXACT>(nx + C::kBufA, kb + s1 * kFK);
-    if constexpr (ACT && !EXACT) f32_interleave<6 * C::MI * C::NJ, kF32Valu>();
+    if constexpr (ACT && !EXACT) f32_interleave<6 * C::MI * C::NJ, V>();
     la.load(kb + s2 * kFK);
     if constexpr (!BISA) lb.load(kb + s2 * kFK);
     f32_barrier();

@@ -2,9 +2,10 @@
 tiles, against the same formula in float64.
 
 The tolerance: operands are represented exactly by three bf16 planes and the
-dropped plane products are below 2^-26 of a product, so what remains is fp32
-accumulation, at most about sqrt(K) 2^-24 of a sum for K updates (3e-6 at the
-widths here); 5e-6 leaves the rest of a forward or backward its own rounding.
+dropped plane products are at most 2^-24 of a product, a rounding, so what
+remains is fp32 accumulation, at most about sqrt(K) 2^-24 of a sum for K updates
+(3e-6 at the widths here); 5e-6 leaves the rest of a forward or backward its own
+rounding.
 """
 
 from __future__ import annotations
@@ -149,3 +150,24 @@ def test_products_that_only_their_leading_planes_overflow(T):
     y64, w64 = y.double().requires_grad_(True), w.double().requires_grad_(True)
     wdx, wdv = torch.autograd.grad(_attn64(y64, y64, w64), (y64, w64), do.double())
     assert torch.isfinite(dx).all() and _rel(dx, wdx) <= TOL and _rel(dv, wdv) <= TOL
+
+
+@pytest.mark.parametrize("T", [100, 300, 520])
+@pytest.mark.parametrize("e", [112, 120, 126])
+def test_small_values_keep_their_bits(T, e):
+    """Operands down to fp32's smallest normal: three bf16 planes of the plain value would miss
+    its last bits (6e-4 of the result at 2^-124)."""
+    N, D, small = 64, 32, 2.0**-e
+    x = _latent(1, 2, T, N, seed=13)
+    v, do = _randn(1, 1, T, D, seed=14), _randn(1, 2, T, D, seed=15)
+    x64, v64 = x.double().requires_grad_(True), v.double().requires_grad_(True)
+    want = _attn64(x64, x64, v64)
+    wdx, wdv = torch.autograd.grad(want, (x64, v64), do.double())
+    got = ext.tril_score_v(x.cuda(), x.cuda(), (v * small).cuda())
+    dx, _, dv = ext.tril_score_v_bwd(x.cuda(), None, v.cuda(), (do * small).cuda())
+    # (scaled back in 64 bits; a value of v below 2^-126 is its fp32 rounding, 2^-23 of the largest)
+    assert _rel(got.double() / small, want.detach()) <= TOL
+    assert _rel(dx.double() / small, wdx) <= TOL and _rel(dv.double() / small, wdv) <= TOL
+    # score tiles that are that small: both factors, taken back up by V
+    got = ext.tril_score_v(x.cuda() * 2.0**(-e // 2), x.cuda() * 2.0**(-e // 2), (v * 2.0**40).cuda())
+    assert _rel(got.double() * 2.0**(-40 - 2 * (-e // 2)), want.detach()) <= TOL
