@@ -809,9 +809,12 @@ def tn_gemm(a: torch.Tensor, b: torch.Tensor, splits: int = 1) -> torch.Tensor:
     with _on(dev):
         rc = _lib.bdh_tn_gemm(_t4(a.unsqueeze(0)), _t4(b.unsqueeze(0)), _t4(out), _stream(dev))
     _check(rc, "tn_gemm")
-    for s in range(1, splits):
-        out[0].add_(out[s])
-    return out[0]
+    if splits == 1:
+        return out[0]
+    total = out[0] + out[1]  # (a tensor of its own: a parameter's .grad may keep it)
+    for s in range(2, splits):
+        total.add_(out[s])
+    return total
 
 
 def small_gemm(a: torch.Tensor, b: torch.Tensor, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:

@@ -184,3 +184,11 @@ def test_a_replaced_operator_or_attention_is_run(monkeypatch):
     del calls[:]
     m.generate(idx, 1, cache_dtype=BF, amp_dtype=BF, impl="hip")
     assert calls == ["decode"] * cfg.n_layer
+
+
+@pytest.mark.parametrize("splits", [1, 2, 4])
+def test_row_contraction_holds_only_its_own_storage(splits):
+    """A weight gradient becomes a parameter's .grad: no split's partial sums may live on in it."""
+    a, b = _randn(2, 512, 64, seed=0), _randn(2, 512, 256, seed=1)
+    got = ext.tn_gemm(a, b, splits)
+    assert got.is_contiguous() and got.untyped_storage().nbytes() == got.numel() * 4
