@@ -192,3 +192,35 @@ def test_row_contraction_holds_only_its_own_storage(splits):
     a, b = _randn(2, 512, 64, seed=0), _randn(2, 512, 256, seed=1)
     got = ext.tn_gemm(a, b, splits)
     assert got.is_contiguous() and got.untyped_storage().nbytes() == got.numel() * 4
+
+
+# weight gradients on the row-contracting kernel (at least 1024 tokens a split), from kept tiles;
+# no kept tiles: n_embd over 256, N not a multiple of 256, or switched off
+@pytest.mark.parametrize("D,nh,mult,B,T,keep,kernel", [
+    (256, 2, 2, 16, 512, "1", "k_dq_sy_tn"), (256, 1, 3, 8, 1056, "1", "k_dq_sy_tn"),
+    (512, 2, 2, 2, 150, "1", "k_relu_bwd_add"), (96, 2, 4, 3, 130, "1", "k_relu_bwd_add"),
+    (64, 2, 8, 2, 33, "0", "k_relu_bwd_add"), (512, 1, 1, 4, 2048, "1", "k_dq_sy_tn")])
+def test_training_step_takes_each_route(D, nh, mult, B, T, keep, kernel, monkeypatch):
+    """Gradients of the routes that a small kept-tiles step does not reach, against the plain
+    autograd graph, from which single bf16 roundings (2^-9) of the latent's gradients set them
+    apart: 3e-3 to 5e-3 measured, 1.2e-2 allowed."""
+    torch.manual_seed(0)
+    monkeypatch.setenv("BDH_ATTN_SAVE_SCORES", keep)
+    m = H.BDH(H.BDHConfig(n_layer=2, n_embd=D, n_head=nh, mlp_internal_dim_multiplier=mult)).cuda()
+    idx = torch.randint(0, 256, (B, T), device="cuda")
+    ext.profile_enable(True)
+    try:
+        got = _train(m, idx)
+        torch.cuda.synchronize()
+        names = {n for n, _ in ext.profile_collect()}
+    finally:
+        ext.profile_enable(False)
+    assert kernel in names and "k_gated_bwd" in names, names
+    m.zero_grad(set_to_none=True)
+    monkeypatch.setattr(H, "_trains_fused", lambda *a: False)
+    want = _train(m, idx)
+    assert set(got) == set(want)
+    for n, g in want.items():
+        e = _rel(got[n], g.double())
+        print(f"  {n}: {e:.3e}", flush=True)
+        assert got[n].dtype == g.dtype and e <= 1.2e-2, n
