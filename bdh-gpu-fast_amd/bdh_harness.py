@@ -226,24 +226,28 @@ def _padded_rows(B: int, T: int, nh: int, N: int, dtype: torch.dtype, device) ->
 
 
 def _token_splits(H: int, M: int, D: int, N: int, a_row: int, b_row: int) -> int:
-    """Parts of the M tokens for ``kernels.tn_gemm`` (a grid of about 192 workgroups of
-    256 x 256 or more), 0 where it does not take the operands.  More parts where the
-    library refuses a part's span; at least 1024 tokens each."""
+    """Parts of the M tokens for ``kernels.tn_gemm``, 0 for torch's per-head products.
+
+    Parts fill the chip and cost the sum of their outputs.  Measured in us with that sum
+    (1, 2, 4, 8 parts; torch): 512 tiles (D = 512, N = 65536) at 4096 tokens 261, 339, 507,
+    872; 301.  128 tiles (D = 256, N = 32768) at 16384 tokens 356, 287, 327, 415; 324, and 793
+    as four heads of 8192.  32 tiles at 8192 tokens 163, 93, 65, 73; 102, at 16384 322, 172,
+    112, 111; 200.  8 tiles at 16384 tokens 317, 166, 94, 66; 97.  Fewer than 1024 tokens a
+    part gain nothing: 32 tiles at 4096 tokens 60 in eight, 57 in torch.  Twice the parts where
+    the library refuses a part's span (D = 512, N = 65536, 16384 tokens: 1046 in two, 1042 in
+    torch); more than that would cost more than torch does."""
     tiles = H * (D // 256) * (N // 256)
     splits = 1 if tiles >= 192 else 2 if tiles >= 96 else 4 if tiles >= 48 else 8
-    while D % 256 == 0 and M // splits >= 1024:
-        if kernels.tn_gemm_takes(H, M, D, N, a_row, b_row, splits):
-            return splits
-        splits *= 2
+    for s in (splits, 2 * splits):
+        if D % 256 == 0 and M // s >= 1024 and kernels.tn_gemm_takes(H, M, D, N, a_row, b_row, s):
+            return s
     return 0
 
 
 def _weight_grad(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """a^T b per head, (H, M, D)^T (H, M, N) -> (H, D, N): over enough tokens on the
-    library's row-contracting kernel (tiles of 256 x 256, the tokens in splits
-    that fill the chip; fp32), else per-head products of torch.  16384 tokens,
-    D = 256, nh N = 32768: 225 us for the four heads of encoder_v against 4 x 186
-    in torch (128 workgroups each), and 225 for the encoder against 270."""
+    library's row-contracting kernel (tiles of 256 x 256, the tokens in parts that fill
+    the chip; fp32), else per-head products of torch."""
     H, M, D = a.shape
     N = b.size(2)
     splits = _token_splits(H, M, D, N, a.stride(1), b.stride(1))
