@@ -358,7 +358,8 @@ int64_t gd_splits(int64_t nh, int64_t M, int64_t N, int64_t most) {
 }
 constexpr int64_t kGdMostSplits = 32;
 
-// Partials of the splits that N = 8192 takes; the launch stays within them.
+// Partials of the splits that N = 8192 takes, for any N (the size does not know
+// it): the launch stays within them, a wider latent too.
 size_t gated_dec_bytes(int64_t nh, int64_t M) { return size_t(nh) * size_t(M) * kGdD * sizeof(float); }
 size_t gated_dec_workspace(int64_t nh, int64_t M) {
   return size_t(gd_splits(nh, M, 8192, kGdMostSplits)) * gated_dec_bytes(nh, M);

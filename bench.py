@@ -644,7 +644,7 @@ def run_extra(torch, ext, kernels, dev, steps, warmup, x, v) -> dict:
     out["c1_torch_eager_gpu_on_qr"] = {"us": ms_e * 1e3, "tflops": F / ms_e / 1e9}
     log(f"[bench] unfused {ms * 1e3:.1f} us, rope {ms_r * 1e3:.1f} us, torch eager {ms_e * 1e3:.1f} us")
 
-    # C1 as BASELINE.json states it: fp32 in and out (the fp32 HIP path),
+    # the same op with fp32 operands in and out (the fp32 HIP path),
     # against the fp32 MFMA peak.
     x32, v32 = x.float(), v.float()
     ms_32 = time_steps(lambda: kernels.bdh_attn_rope(x32, v32, freqs, 0, impl="hip"), max(3, steps // 2), 2)
@@ -875,8 +875,7 @@ def run_pmc_targets(torch, ext, kernels, dev, reps: int = 3) -> None:
     for _ in range(reps):
         kernels.bdh_attn_rope(x, v, f, 0, impl="hip")
     section_end()
-    # C1 as BASELINE.json states it, fp32 operands (the generic MFMA kernels
-    # k_scores, k_score_v)
+    # the same op with fp32 operands (k_f32_scores, k_f32_msum, k_f32_sv)
     x32, v32 = x.float(), v.float()
     del x, v
     for _ in range(reps):
